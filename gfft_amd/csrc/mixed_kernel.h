@@ -1,0 +1,490 @@
+// mixed_kernel.h -- batched Stockham FFT of any length with the factors 2, 3, 5 and 7 that
+// fits the LDS, its radices and shape given at run time (gfx950).
+//
+// The tiles of tile_kernel.h are compiled per length.  A length without one used to be split
+// into passes of small compiled tiles (1000 = 25*8*5: three passes over HBM); this kernel runs
+// it in one.  The stages are the ones of tile_kernel.h, with
+//   - radices up to 16, composite ones included (6, 9, 10, 12, 14, 15), so that a length has few
+//     stages and a thread holds at most MIX_POINTS points;
+//   - a stage's radix chosen by a branch that is uniform over the launch: every radix is a
+//     register butterfly of its own, nothing is indexed at run time inside it;
+//   - division by a stage's Ns as one multiplication by a precomputed reciprocal, and an LDS
+//     layout (pad elements after every R_0) in which the elements of a butterfly lie at a
+//     constant distance, so that an element costs one address addition.
+// Access modes as in tile_kernel.h: E->E (single pass), T->E (first pass), T->T (later passes).
+#pragma once
+#include "tile_kernel.h"
+
+namespace gfftx {
+
+constexpr int MIX_POINTS = 16;    // most points of a sequence one thread holds
+constexpr int MIX_STAGES = 14;    // 2^14 = 16384 in radix-2 stages at the very most
+#define GFFTX_MIX_RADICES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(14) X(15) X(16)
+
+struct MixStage {
+    unsigned R;     // radix
+    unsigned lr;    // L / R: butterflies per sequence
+    unsigned ns;    // product of the earlier radices
+    unsigned mns;   // ceil(2^32 / ns): j / ns = umulhi(j, mns) for j < 2^14 (ns > 1)
+    unsigned rst;   // LDS distance of the elements j, j + L/R, .. a butterfly reads
+    unsigned wst;   // LDS distance of the elements it writes (ns apart)
+    unsigned tw;    // first entry of the stage's twiddles (FP32: ns FP64 roots; FP64: rows r = 1..R-1 of ns entries)
+};
+
+struct MixShape {
+    unsigned L, nb, tpt, wg;  // nb sequences of tpt threads each; wg >= nb * tpt threads
+    unsigned mtpt;            // ceil(2^32 / tpt) (tpt > 1)
+    unsigned ts;              // LDS distance between sequences
+    unsigned pad;             // LDS pad elements after every R_0 elements
+    unsigned mr0;             // ceil(2^32 / R_0)
+    unsigned ml;              // ceil(2^32 / L)
+    unsigned nst;
+    int nt_in;                // 1: rows are whole 128-byte lines, the input is loaded non-temporally
+    MixStage st[MIX_STAGES];
+};
+
+struct MixArgs {
+    TileArgs a;
+    MixShape m;
+};
+
+enum { MIX_EE = 0, MIX_TE = 1, MIX_TT = 2 };
+
+// Good-Thomas butterfly of A*B points, A and B coprime: an A x B two-dimensional DFT between
+// two index maps, without twiddles.  Input n = (B n1 + A n2) mod AB, output
+// k = (B (B^-1 mod A) k1 + A (A^-1 mod B) k2) mod AB (I. J. Good, 1958).
+template <int A, int B> struct PfaDft {
+    static constexpr int N = A * B;
+    static constexpr int inv(int x, int m)
+    {
+        for (int i = 1; i < m; ++i)
+            if (x * i % m == 1) return i;
+        return 1;
+    }
+    template <typename V> __device__ __forceinline__ static void run(V* v)
+    {
+        V w[A][B];
+#pragma unroll
+        for (int i = 0; i < A; ++i) {
+#pragma unroll
+            for (int k = 0; k < B; ++k) w[i][k] = v[(B * i + A * k) % N];
+            Dft<B>::run(w[i]);
+        }
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            V c[A];
+#pragma unroll
+            for (int i = 0; i < A; ++i) c[i] = w[i][k];
+            Dft<A>::run(c);
+#pragma unroll
+            for (int i = 0; i < A; ++i) v[(B * inv(B % A, A) * i + A * inv(A % B, B) * k) % N] = c[i];
+        }
+    }
+};
+template <> struct Dft<6> : PfaDft<2, 3> {};
+template <> struct Dft<10> : PfaDft<2, 5> {};
+template <> struct Dft<12> : PfaDft<4, 3> {};
+template <> struct Dft<14> : PfaDft<2, 7> {};
+template <> struct Dft<15> : PfaDft<3, 5> {};
+
+// 9 = 3 * 3: n = i + 3 m, k = q + 3 p, twiddles W_9^{iq}
+template <> struct Dft<9> {
+    template <typename V> __device__ __forceinline__ static void run(V* v)
+    {
+        using S = decltype(v[0].x);
+        const V w1{(S)0.76604444311897803520239265055541667394, (S)-0.64278760968653932632264340990726343291};
+        const V w2{(S)0.17364817766693034885171662676931479600, (S)-0.98480775301220805936674302458952301367};
+        const V w4{(S)-0.93969262078590838405410927732473146994, (S)-0.34202014332566873304409961468225958076};
+        V a[3][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            a[i][0] = v[i];
+            a[i][1] = v[i + 3];
+            a[i][2] = v[i + 6];
+            Dft<3>::run(a[i]);
+        }
+        a[1][1] = cmul(a[1][1], w1);
+        a[1][2] = cmul(a[1][2], w2);
+        a[2][1] = cmul(a[2][1], w2);
+        a[2][2] = cmul(a[2][2], w4);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            V b[3] = {a[0][q], a[1][q], a[2][q]};
+            Dft<3>::run(b);
+            v[q] = b[0];
+            v[q + 3] = b[1];
+            v[q + 6] = b[2];
+        }
+    }
+};
+
+// Thread context of one tile.
+template <typename T> struct MixCtx {
+    using V = V2<T>;
+    V* lds;        // this sequence's LDS region
+    const V* in;   // element e of the sequence at in[e * ies]
+    V* out;        // output q of the sequence at out[q * ns]
+    unsigned jt;   // thread within the sequence; beyond every butterfly for idle threads
+    unsigned ies, ons;
+    long long tg;  // sequence within the batch item
+    long long bo;  // element offset of the batch item
+};
+
+// Twiddles W^{k r}, r = 1..R-1, of one butterfly.  FP32: FP64 powers of the FP64 root, rounded
+// once (as in tile_kernel.h); FP64: the table's rows, row r contiguous in k.
+template <typename T, int R> __device__ __forceinline__ void mix_twiddle(V2<T>* v, const void* tw, const MixStage& st, unsigned k)
+{
+    using V = V2<T>;
+    if constexpr (sizeof(T) == 4) {
+        const double2 w1 = reinterpret_cast<const double2*>(tw)[st.tw + k];
+        v[1] = cmul(v[1], to_v<V>(w1));
+        if constexpr (R > 2) {
+            const double2 w2 = dmul(w1, w1);
+            v[2] = cmul(v[2], to_v<V>(w2));
+            if constexpr (R > 3) {
+                const double2 w3 = dmul(w2, w1);
+                v[3] = cmul(v[3], to_v<V>(w3));
+                if constexpr (R > 4) {
+                    // W^{4a + c} = (W^4)^a W^c: at most five products from the root
+                    const double2 w4 = dmul(w2, w2);
+                    double2 wa = w4;
+#pragma unroll
+                    for (int r = 4; r < R; ++r) {
+                        if (r % 4 == 0) {
+                            if (r > 4) wa = dmul(wa, w4);
+                            v[r] = cmul(v[r], to_v<V>(wa));
+                        } else {
+                            v[r] = cmul(v[r], to_v<V>(dmul(wa, r % 4 == 1 ? w1 : r % 4 == 2 ? w2 : w3)));
+                        }
+                    }
+                }
+            }
+        }
+    } else {
+        const V* row = reinterpret_cast<const V*>(tw) + st.tw + k;
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+            v[r] = cmul(v[r], row[(unsigned)(r - 1) * st.ns]);
+            if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four rows in flight: the registers hold no more
+        }
+    }
+}
+
+// Butterflies a thread runs per stage: as many as MIX_POINTS points hold (the host chooses tpt
+// so that they cover the sequence).
+template <int R> constexpr int mix_b() { return MIX_POINTS / R; }
+
+// First stage: global memory to registers (pass twiddle of a later pass, conjugation of an
+// inverse transform, C2R pre-pass of a real one), butterfly, LDS.
+template <typename T, int MODE, int REAL, int R, bool ONLY>
+__device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
+{
+    using V = V2<T>;
+    using S_ = T;
+    constexpr int B = mix_b<R>();
+    const TileArgs& a = x.a;
+    const unsigned lr = x.m.st[0].lr, tpt = x.m.tpt;
+    V v[B][R];
+    with_nt(x.m.nt_in != 0, [&](auto ntc) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const unsigned j = c.jt + b * tpt;
+            if (j >= lr) continue;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const V* p = &c.in[MODE == MIX_EE ? j + r * lr : (j + r * lr) * c.ies];
+                if constexpr (decltype(ntc)::value) v[b][r] = nt_load(p);
+                else v[b][r] = *p;
+            }
+        }
+    });
+    if constexpr (REAL == REAL_PRE) {
+        // Z[e] from X[e] and X[N - e] of the same sequence (see pre_split, tile_kernel.h); the
+        // exchange uses a plain layout, element e at e
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const unsigned j = c.jt + b * tpt;
+            if (j >= lr) continue;
+#pragma unroll
+            for (int r = 0; r < R; ++r) c.lds[j + r * lr] = v[b][r];
+        }
+        __syncthreads();
+        const S_ half = (S_)0.5;
+        const unsigned N = x.m.L;
+        const long long mask = (1LL << a.sp_shift) - 1;
+        const double2 step = dmul(a.sp_lo[lr & mask], a.sp_hi[lr >> a.sp_shift]);
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const unsigned j = c.jt + b * tpt;
+            if (j >= lr) continue;
+            double2 w = dmul(a.sp_lo[j & mask], a.sp_hi[j >> a.sp_shift]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const unsigned e = j + r * lr;
+                const V xe = v[b][r], xp = c.lds[e == 0 ? 0 : N - e];
+                V z;
+                if (e == 0) {
+                    const S_ x0 = xe.x, xn = a.split_bins ? c.in[N].x : xe.y;
+                    z = V{half * (x0 + xn), half * (x0 - xn)};
+                } else {
+                    const bool lo = e <= N - e;
+                    const V A = lo ? xe : xp, Bv = lo ? xp : xe;
+                    // conj(W^k) for k = min(e, N - e): conj(W^{N-e}) = -W^e
+                    const V cw = to_v<V>(lo ? double2{w.x, -w.y} : double2{-w.x, -w.y});
+                    const V h1 = V{half * (A.x + Bv.x), half * (A.y - Bv.y)};
+                    const V dd = V{half * (A.x - Bv.x), half * (A.y + Bv.y)};
+                    const V t = cmul(cw, dd);
+                    const V p = V{-t.y, t.x};  // i conj(W^k) d
+                    z = lo ? V{h1.x + p.x, h1.y + p.y} : V{h1.x - p.x, p.y - h1.y};
+                }
+                v[b][r] = z;
+                w = dmul(w, step);
+            }
+        }
+        __syncthreads();
+    }
+    const unsigned flip = a.conj_in ? 0x80000000u : 0u;
+    const long long kp = (MODE == MIX_TT && a.ptw_lo != nullptr) ? c.tg % a.ns_pass : 0;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const unsigned j = c.jt + b * tpt;
+        if (j >= lr) continue;
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[b][r] = flip_im(v[b][r], flip);
+        if constexpr (MODE == MIX_TT) {
+            if (kp != 0) {
+                // W_M^{kp e}, e = j + r lr: base W^{kp j} times step^r, step = W^{kp lr}
+                const long long pm = (1LL << a.ptw_shift) - 1, m0 = kp * j, ms = kp * lr;
+                const double2 step = dmul(a.ptw_lo[ms & pm], a.ptw_hi[ms >> a.ptw_shift]);
+                double2 w = dmul(a.ptw_lo[m0 & pm], a.ptw_hi[m0 >> a.ptw_shift]);
+                v[b][0] = cmul(v[b][0], to_v<V>(w));
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    w = dmul(w, step);
+                    v[b][r] = cmul(v[b][r], to_v<V>(w));
+                }
+            }
+        }
+        Dft<R>::run(v[b]);
+        if constexpr (!ONLY) {
+            V* w = c.lds + j * (R + x.m.pad);
+#pragma unroll
+            for (int r = 0; r < R; ++r) w[r] = v[b][r];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (ONLY) {
+        // a length that is one butterfly: straight to the output
+        const unsigned fo = a.conj_out ? 0x80000000u : 0u;
+        const T sc = (T)a.scale;
+        with_nt(a.nt_out != 0, [&](auto ntc) {
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                if (c.jt + b * tpt >= lr) continue;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    put<decltype(ntc)::value>(&c.out[r * c.ons], flip_im(a.scale == 1.0 ? v[b][r] : cscale(v[b][r], sc), fo));
+            }
+        });
+    } else {
+        __syncthreads();
+    }
+}
+
+// A later stage: LDS to registers, twiddles, butterfly, and back to the LDS or, after the last
+// stage of a mode whose stores match its lanes, to the output.
+template <typename T, int MODE, int REAL, int R, bool LAST>
+__device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const MixStage& st)
+{
+    using V = V2<T>;
+    constexpr int B = mix_b<R>();
+    constexpr bool DIRECT = LAST && MODE != MIX_TE && REAL != REAL_POST;
+    const TileArgs& a = x.a;
+    const unsigned lr = st.lr, tpt = x.m.tpt, rst = st.rst;
+    V v[B][R];
+    // LDS index of element j, and of the first element butterfly j writes
+    auto rpos = [&](unsigned j) { return j + x.m.pad * __umulhi(j, x.m.mr0); };
+    auto quot = [&](unsigned j) { return LAST ? 0u : __umulhi(j, st.mns); };  // after the last stage ns = lr > j
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const unsigned j = c.jt + b * tpt;
+        if (j >= lr) continue;
+        const V* rd = c.lds + rpos(j);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[b][r] = rd[r * rst];
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const unsigned j = c.jt + b * tpt;
+        if (j < lr) {
+            mix_twiddle<T, R>(v[b], a.tw, st, j - quot(j) * st.ns);
+            Dft<R>::run(v[b]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one butterfly's twiddles at a time (registers)
+    }
+    if constexpr (DIRECT) {
+        const unsigned fo = a.conj_out ? 0x80000000u : 0u;
+        const T sc = (T)a.scale;
+        const bool one = a.scale == 1.0;
+        with_nt(a.nt_out != 0, [&](auto ntc) {
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                const unsigned j = c.jt + b * tpt;
+                if (j >= lr) continue;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    put<decltype(ntc)::value>(&c.out[MODE == MIX_EE ? j + r * lr : (j + r * lr) * c.ons],
+                                              flip_im(one ? v[b][r] : cscale(v[b][r], sc), fo));
+            }
+        });
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const unsigned j = c.jt + b * tpt;
+            if (j >= lr) continue;
+            V* wr = c.lds + rpos(j) + quot(j) * (R - 1) * st.wst;
+#pragma unroll
+            for (int r = 0; r < R; ++r) wr[r * st.wst] = v[b][r];
+        }
+        __syncthreads();
+    }
+}
+
+// T->E store: the tile's nb * L outputs are one contiguous run (first pass, Ns = 1).
+template <typename T> __device__ __forceinline__ void mix_finish_te(const MixArgs& x, const V2<T>* lds, long long bo, unsigned tile)
+{
+    using V = V2<T>;
+    const TileArgs& a = x.a;
+    const unsigned L = x.m.L;
+    V* o = reinterpret_cast<V*>(a.out) + bo + (long long)tile * x.m.nb * L;
+    const long long left = a.ntrans - (long long)tile * x.m.nb;
+    const unsigned total = (left < (long long)x.m.nb ? (unsigned)left : x.m.nb) * L;
+    const unsigned fo = a.conj_out ? 0x80000000u : 0u;
+    const T sc = (T)a.scale;
+    const bool one = a.scale == 1.0;
+    with_nt(a.nt_out != 0, [&](auto ntc) {
+#pragma unroll 4
+        for (unsigned lin = threadIdx.x; lin < total; lin += x.m.wg) {
+            const unsigned t = __umulhi(lin, x.m.ml), q = lin - t * L;
+            const V u = lds[t * x.m.ts + q + x.m.pad * __umulhi(q, x.m.mr0)];
+            put<decltype(ntc)::value>(&o[lin], flip_im(one ? u : cscale(u, sc), fo));
+        }
+    });
+}
+
+// R2C post-pass of a single-pass real transform (see split_finish_e, tile_kernel.h).
+template <typename T> __device__ __forceinline__ void mix_split(const MixArgs& x, const MixCtx<T>& c)
+{
+    using V = V2<T>;
+    const TileArgs& a = x.a;
+    const unsigned L = x.m.L, tpt = x.m.tpt;
+    if (c.jt >= tpt) return;
+    const T half = (T)0.5;
+    const long long mask = (1LL << a.sp_shift) - 1;
+    double2 w = dmul(a.sp_lo[c.jt & mask], a.sp_hi[c.jt >> a.sp_shift]);
+    const double2 step = dmul(a.sp_lo[tpt & mask], a.sp_hi[tpt >> a.sp_shift]);
+    auto at = [&](unsigned e) { return c.lds[e + x.m.pad * __umulhi(e, x.m.mr0)]; };
+#pragma unroll 4
+    for (unsigned k = c.jt; k < L; k += tpt) {
+        const V zk = at(k), zp = at(k == 0 ? 0 : L - k);
+        if (k == 0) {
+            const T x0 = zk.x + zk.y, xn = zk.x - zk.y;
+            if (a.split_bins) {
+                c.out[0] = V{x0, 0};
+                c.out[L] = V{xn, 0};
+            } else {
+                c.out[0] = V{x0, xn};
+            }
+        } else {
+            const bool lo = k <= L - k;
+            const V A = lo ? zk : zp, B = lo ? zp : zk;
+            const V wv = to_v<V>(lo ? w : double2{-w.x, w.y});  // W^k, or W^{N-k} = -conj(W^k)
+            const V h1 = V{half * (A.x + B.x), half * (A.y - B.y)};
+            const V dd = V{half * (A.x - B.x), half * (A.y + B.y)};
+            const V p = cmul(wv, V{dd.y, -dd.x});
+            c.out[k] = lo ? V{h1.x + p.x, h1.y + p.y} : V{h1.x - p.x, p.y - h1.y};
+        }
+        w = dmul(w, step);
+    }
+}
+
+template <typename T, int MODE, int REAL>
+__global__ __launch_bounds__(1024, sizeof(T) == 4 ? 6 : 4) void mixed_kernel(MixArgs x)
+{
+    using V = V2<T>;
+    extern __shared__ __align__(16) unsigned char mix_lds[];
+    V* lds = reinterpret_cast<V*>(mix_lds);
+    const TileArgs& a = x.a;
+    const unsigned tile = tile_index(blockIdx.x, gridDim.x, a.xcd), tid = threadIdx.x;
+    unsigned t;
+    MixCtx<T> c;
+    if constexpr (MODE == MIX_EE) {
+        t = x.m.tpt == 1 ? tid : __umulhi(tid, x.m.mtpt);
+        c.jt = tid - t * x.m.tpt;
+    } else {
+        t = tid & (x.m.nb - 1);  // nb is a power of two in the T modes
+        c.jt = tid >> __builtin_ctz(x.m.nb);
+        if (c.jt >= x.m.tpt) c.jt = 1u << 20;
+    }
+    c.tg = (long long)tile * x.m.nb + t;
+    const bool valid = t < x.m.nb && c.tg < a.ntrans;
+    if (!valid) {  // beyond every loop bound: takes part in the barriers only
+        c.jt = 1u << 20;
+        c.tg = 0;
+        t = 0;
+    }
+    c.bo = batch_offset(a, blockIdx.y);
+    c.lds = lds + t * x.m.ts;
+    const long long so = a.seq_off ? a.seq_off[c.tg] : 0;
+    c.in = reinterpret_cast<const V*>(a.in) + c.bo + (a.seq_off ? so : c.tg * a.its);
+    c.ies = (unsigned)a.ies;
+    c.ons = (unsigned)a.ns_pass;
+    long long ob = so;
+    if (!a.seq_off) {
+        const unsigned ns = (unsigned)a.ns_pass, t32 = (unsigned)c.tg;
+        if (MODE == MIX_EE) ob = c.tg * a.its;
+        else ob = ns == 1 ? c.tg * x.m.L : (long long)(t32 / ns) * ns * x.m.L + (t32 % ns);
+    }
+    c.out = reinterpret_cast<V*>(a.out) + c.bo + ob;
+    const unsigned nst = x.m.nst;
+    if (MODE == MIX_EE && REAL == REAL_NONE && nst == 1) {
+        switch (x.m.st[0].R) {
+#define X(R_) \
+    case R_: mix_first<T, MODE, REAL, R_, true>(x, c); break;
+            GFFTX_MIX_RADICES(X)
+#undef X
+            default: break;
+        }
+        return;
+    }
+    switch (x.m.st[0].R) {
+#define X(R_) \
+    case R_: mix_first<T, MODE, REAL, R_, false>(x, c); break;
+        GFFTX_MIX_RADICES(X)
+#undef X
+        default: break;
+    }
+    for (unsigned s = 1; s + 1 < nst; ++s) {
+        const MixStage st = x.m.st[s];
+        switch (st.R) {
+#define X(R_) \
+    case R_: mix_stage<T, MODE, REAL, R_, false>(x, c, st); break;
+            GFFTX_MIX_RADICES(X)
+#undef X
+            default: break;
+        }
+    }
+    const MixStage sl = x.m.st[nst - 1];
+    switch (sl.R) {
+#define X(R_) \
+    case R_: mix_stage<T, MODE, REAL, R_, true>(x, c, sl); break;
+        GFFTX_MIX_RADICES(X)
+#undef X
+        default: break;
+    }
+    if constexpr (MODE == MIX_TE) mix_finish_te<T>(x, lds, c.bo, tile);
+    if constexpr (REAL == REAL_POST) mix_split<T>(x, c);
+}
+
+}  // namespace gfftx

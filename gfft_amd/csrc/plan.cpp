@@ -52,7 +52,7 @@ int dev_alloc(gfftx_plan_s* p, void** out, size_t bytes)
 
 int upload_stage_table(gfftx_plan_s* p, const TileEntry* k, void** out)
 {
-    return upload_stage_table_r(p->allocs, p->prec, k->nrad, k->radices, out);
+    return upload_tile_table(p->allocs, k, out);
 }
 
 int upload_pass_table(gfftx_plan_s* p, Pass& ps, long long M)
@@ -95,11 +95,11 @@ int build_c2c_passes(gfftx_plan_s* p)
     // single-pass tile; any other list is a pass split, which overrides the single-pass tile
     const bool forced_single = p->forced_lens.size() >= 2 && p->forced_lens[0] == (int)n && p->forced_lens[1] == 1;
     const TileEntry* single = nullptr;
-    if (n <= (1ull << 30) && (p->forced_lens.empty() || forced_single)) {
+    if (p->forced_lens.empty() || forced_single) {
         std::vector<int> fl;
         std::vector<std::pair<int, int>> ft;
         split_choice(p->forced_lens, fl, ft);
-        single = find_tile(p->prec, (int)n, false, false, ft.empty() ? 0 : ft[0].first, ft.empty() ? 0 : ft[0].second);
+        single = single_tile(p->prec, n, ft.empty() ? 0 : ft[0].first, ft.empty() ? 0 : ft[0].second);
     }
     if (single) {
         const TileEntry* k = single;
@@ -118,6 +118,8 @@ int build_c2c_passes(gfftx_plan_s* p)
         // the first stage inverse) when the tile has such a variant
         if (p->real && env_int("GFFTX_FUSED_SPLIT", 1)) {
             if (const TileEntry* kr = find_real_tile(k, p->inverse ? REAL_PRE : REAL_POST)) {
+                if (kr->mix) rc = upload_tile_table(p->allocs, kr, &ps.stage_tw);  // its own stages
+                if (rc) return rc;
                 ps.k = kr;
                 ps.real = kr->real;
                 rc = upload_root_tables(p->allocs, (long long)(2 * n), &ps.sp_lo, &ps.sp_hi, &ps.sp_shift);
@@ -139,7 +141,8 @@ int build_c2c_passes(gfftx_plan_s* p)
             const int L = lens[i];
             const int want_nb = i < tiles.size() && tiles[i].first ? tiles[i].first : env_int("GFFTX_TNB", 0);
             const int want_wg = i < tiles.size() && tiles[i].first ? tiles[i].second : env_int("GFFTX_TWG", 0);
-            const TileEntry* k = find_tile(p->prec, L, true, i > 0, want_nb, want_wg);
+            const TileEntry* k = want_nb || want_wg ? find_tile(p->prec, L, true, i > 0, want_nb, want_wg)
+                                                    : pass_tile(p->prec, L, i == 0, n, p->batch, device_cus(p->device));
             if (!k) return fail(GFFTX_ERR_UNSUPPORTED, "no pass kernel L=%d", L);
             Pass ps;
             ps.k = k;
@@ -340,7 +343,7 @@ int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range 
         dim3 grid(ntiles, ps.items_in_ntrans ? 1u : (unsigned)r.nb);
         std::pair<hipEvent_t, hipEvent_t> ev;
         const bool on = prof_begin(prof, slot0 + i, ps.k->name, s, &ev, true);
-        hipError_t e = ps.k->launch(a, grid, s, on ? ev.first : nullptr, on ? ev.second : nullptr);
+        hipError_t e = launch_entry(ps.k, a, grid, s, on ? ev.first : nullptr, on ? ev.second : nullptr);
         if (on) prof_end(prof, slot0 + i, s, ev, true);
         if (e != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "%s: %s", ps.k->name, hipGetErrorString(e));
         src = dst[i];

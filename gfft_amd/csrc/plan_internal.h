@@ -80,14 +80,23 @@ bool nt_output(size_t bytes);
 
 inline size_t elem_bytes(int prec) { return prec == PREC_F64 ? 16 : 8; }
 
+// --- mixed_plan.cpp: run-time mixed-radix tiles
+int mix_max(int prec, bool loadT);
+std::vector<const TileEntry*> mix_tiles(int prec, int L, bool loadT, bool storeT, int real = REAL_NONE);
+int upload_tile_table(std::vector<void*>& owned, const TileEntry* k, void** out);
+
+std::vector<const TileEntry*> tile_shapes(int prec, int L, bool loadT, bool storeT);
 const TileEntry* find_tile(int prec, int L, bool loadT, bool storeT, int want_nb = 0, int want_wg = 0);
+const TileEntry* single_tile(int prec, unsigned long long n, int want_nb = 0, int want_wg = 0);
 const TileEntry* find_real_tile(const TileEntry* k, int kind);
 int env_int(const char* name, int dflt);
 int device_cus(int device);
 double pass_bandwidth(int prec, int L);
-double pass_occupancy(int prec, int L, bool first, unsigned long long n, unsigned long long batch, int cus);
+double pass_cost(const TileEntry* k, unsigned long long n, unsigned long long batch, int cus);
+const TileEntry* pass_tile(int prec, int L, bool first, unsigned long long n, unsigned long long batch, int cus,
+                           double* cost = nullptr);
 std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch = 1,
-                                               int cus = 256);
+                                               int cus = 256, bool mixed = true);
 void split_choice(const std::vector<int>& c, std::vector<int>& lens, std::vector<std::pair<int, int>>& tiles);
 int xcd_remap(const TileEntry* k, int prec);
 bool native_length(int prec, unsigned long long n);

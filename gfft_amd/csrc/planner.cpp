@@ -10,25 +10,40 @@ namespace detail {
 
 void root_ld(long long m, long long N, long double* c, long double* s) { root_ld_eval(m, N, c, s); }
 
-// First registered tile for (prec, L, modes), or the first one with nb == want_nb and
-// wg == want_wg (each when nonzero) when there is one.
-const TileEntry* find_tile(int prec, int L, bool loadT, bool storeT, int want_nb, int want_wg)
+// Every tile of (prec, L, modes), the default first: the compiled ones in table order, or,
+// where there is none, the run-time mixed-radix tiles.
+std::vector<const TileEntry*> tile_shapes(int prec, int L, bool loadT, bool storeT)
 {
-    const TileEntry* first = nullptr;
+    std::vector<const TileEntry*> out;
     for (int i = 0; i < kNumTiles; ++i) {
         const TileEntry& e = kTiles[i];
-        if (e.prec == prec && e.L == L && e.loadT == loadT && e.storeT == storeT) {
-            if ((want_nb || want_wg) && (!want_nb || e.nb == want_nb) && (!want_wg || e.wg == want_wg)) return &e;
-            if (!first) first = &e;
-        }
+        if (e.prec == prec && e.L == L && e.loadT == loadT && e.storeT == storeT) out.push_back(&e);
     }
-    return first;
+    return out.empty() ? mix_tiles(prec, L, loadT, storeT) : out;
+}
+
+// First tile for (prec, L, modes), or the first one with nb == want_nb and wg == want_wg (each
+// when nonzero) when there is one.
+const TileEntry* find_tile(int prec, int L, bool loadT, bool storeT, int want_nb, int want_wg)
+{
+    const std::vector<const TileEntry*> v = tile_shapes(prec, L, loadT, storeT);
+    if (want_nb || want_wg)
+        for (const TileEntry* e : v)
+            if ((!want_nb || e->nb == want_nb) && (!want_wg || e->wg == want_wg)) return e;
+    return v.empty() ? nullptr : v[0];
 }
 
 // The variant of tile k (same length, shape, radices and access modes) with the real-transform
 // split `kind` (REAL_POST, REAL_PRE) fused in, or null.
 const TileEntry* find_real_tile(const TileEntry* k, int kind)
 {
+    if (k->mix) {
+        // same shape, or, beside a one-butterfly tile, a shape of its own (two stages or more)
+        const std::vector<const TileEntry*> v = mix_tiles(k->prec, k->L, k->loadT, k->storeT, kind);
+        for (const TileEntry* e : v)
+            if (e->nb == k->nb && e->wg == k->wg) return e;
+        return k->nrad == 1 && !v.empty() ? v[0] : nullptr;
+    }
     for (int i = 0; i < kNumRealTiles; ++i) {
         const TileEntry& e = kRealTiles[i];
         if (e.real != kind || e.prec != k->prec || e.L != k->L || e.nb != k->nb || e.wg != k->wg ||
@@ -73,53 +88,100 @@ double pass_bandwidth(int prec, int L)
     return f32 ? 2.6 : 2.5;
 }
 
-// Fraction of the device one pass of length L keeps busy: its tiles (n/L sequences per
-// batch item, NB per tile) over the workgroups all CUs hold at once (LDS and threads
-// limit a CU to 160 KB and 2048 threads).
-double pass_occupancy(int prec, int L, bool first, unsigned long long n, unsigned long long batch, int cus)
+// Modelled time (us) of one pass by tile `k` over `batch` items of n points: 2.5 us of launch,
+// and either the bytes at the bandwidth the tile reaches (less for a run-time tile and for rows
+// below a 128-byte line) or, when there is little to move, the time of one tile, 1.5 us and 0.12
+// us per KB, for each round of tiles the device holds at once (LDS and threads limit a CU to
+// 160 KB and 2048 threads).  The tile times are those of short passes issued back to back: 10 KB
+// tiles of 25 points 4.8 us in all, 49 KB ones of 1536 points 12.4 us, 64 KB ones of 1000 points
+// 13 us.
+double pass_cost(const TileEntry* k, unsigned long long n, unsigned long long batch, int cus)
 {
-    const TileEntry* k = find_tile(prec, L, true, !first);
-    if (!k) return 1.0;
     const int by_lds = k->lds_bytes > 0 ? (160 * 1024) / k->lds_bytes : 8;
     const int per_cu = std::max(1, std::min(by_lds, 2048 / k->wg));
-    const double tiles = std::ceil((double)(n / (unsigned long long)L) / k->nb) * (double)batch;
-    return std::min(1.0, tiles / ((double)cus * per_cu));
+    const double tiles = std::ceil((double)(n / (unsigned long long)k->L) / k->nb) * (double)batch;
+    const double rounds = std::ceil(tiles / ((double)cus * per_cu));
+    const double kb = (double)k->nb * k->L * elem_bytes(k->prec) / 1024.0;
+    const double row = (double)k->nb * elem_bytes(k->prec);
+    const double bw = pass_bandwidth(k->prec, k->L) * (k->mix ? 0.9 : 1.0) * (row >= 128 ? 1.0 : row >= 64 ? 0.9 : 0.7);
+    const double move = 2.0 * (double)n * (double)batch * elem_bytes(k->prec) / (bw * 1e6);
+    return 2.5 + std::max(move, rounds * (1.5 + 0.12 * kb));
 }
 
-// Pass splits of n into compiled T-mode tile lengths (2..4 passes), best `k` by the cost
-// model: each pass moves 2 n b_c bytes at the bandwidth its tile reaches
-// (pass_bandwidth()) times the fraction of the device its tiles occupy.  The first length
-// of every split has a T->E tile.
+// The tile a pass of length L takes unless one is named: the default one of a compiled length,
+// the one with the lowest modelled time of a run-time length; null when there is none.  *cost is
+// the lowest modelled time of the length's tiles (the autotuner times them all).
+const TileEntry* pass_tile(int prec, int L, bool first, unsigned long long n, unsigned long long batch, int cus, double* cost)
+{
+    const TileEntry* best = nullptr;
+    double bc = 0;
+    for (const TileEntry* k : tile_shapes(prec, L, true, !first)) {
+        const double c = pass_cost(k, n, batch, cus);
+        if (!best || (k->mix && c < bc)) best = k;
+        if (best == k || c < bc) bc = c;
+    }
+    if (cost) *cost = bc;
+    return best;
+}
+
+// Pass splits of n into T-mode tile lengths (2..4 passes), best `k` by the cost model
+// (pass_cost()).  The first length of every split has a T->E tile.  The lengths are the compiled
+// ones and, with `mixed`, every other divisor of n with the factors 2, 3, 5 and 7 from 17 up to
+// the run-time tiles' limit.
 std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch,
-                                               int cus)
+                                               int cus, bool mixed)
 {
     std::vector<int> lens;
     for (int i = 0; i < kNumTiles; ++i)
-        if (kTiles[i].prec == prec && kTiles[i].loadT && kTiles[i].storeT) lens.push_back(kTiles[i].L);
+        if (kTiles[i].prec == prec && kTiles[i].loadT && kTiles[i].storeT && n % (unsigned long long)kTiles[i].L == 0)
+            lens.push_back(kTiles[i].L);
     std::sort(lens.begin(), lens.end());
     lens.erase(std::unique(lens.begin(), lens.end()), lens.end());
+    if (mixed) {
+        std::vector<int> more;
+        const int most = mix_max(prec, true);
+        for (long long a = 1; a <= most; a *= 2)
+            for (long long b = a; b <= most; b *= 3)
+                for (long long c = b; c <= most; c *= 5)
+                    for (long long d = c; d <= most; d *= 7)
+                        if (d > 16 && n % (unsigned long long)d == 0 && !std::binary_search(lens.begin(), lens.end(), (int)d))
+                            more.push_back((int)d);
+        lens.insert(lens.end(), more.begin(), more.end());
+        std::sort(lens.begin(), lens.end());
+    }
+    // cost of each length as the first and as a later pass (negative: no such tile)
+    std::vector<double> cost0(lens.size()), cost1(lens.size());
+    for (size_t i = 0; i < lens.size(); ++i)
+        for (int later = 0; later < 2; ++later)
+            if (!pass_tile(prec, lens[i], !later, n, batch, cus, &(later ? cost1 : cost0)[i]))
+                (later ? cost1 : cost0)[i] = -1.0;
     std::vector<std::pair<double, std::vector<int>>> found;
-    std::vector<int> cur;
+    std::vector<int> cur;  // indices into lens, largest first
     std::function<void(unsigned long long, int)> rec = [&](unsigned long long rem, int maxi) {
         if (rem == 1) {
             if (cur.size() < 2) return;
             std::vector<int> order = cur;
             for (size_t i = 0; i < order.size(); ++i)
-                if (find_tile(prec, order[i], true, false)) {
+                if (cost0[order[i]] >= 0) {
                     std::swap(order[0], order[i]);
                     break;
                 }
-            if (!find_tile(prec, order[0], true, false)) return;
+            if (cost0[order[0]] < 0) return;
             double cost = 0;
-            for (size_t i = 0; i < order.size(); ++i)
-                cost += 1.0 / (pass_bandwidth(prec, order[i]) * pass_occupancy(prec, order[i], i == 0, n, batch, cus));
-            found.push_back({cost, order});
+            std::vector<int> l;
+            for (size_t i = 0; i < order.size(); ++i) {
+                const double c = i ? cost1[order[i]] : cost0[order[i]];
+                if (c < 0) return;
+                cost += c;
+                l.push_back(lens[order[i]]);
+            }
+            found.push_back({cost, l});
             return;
         }
         if (cur.size() == 4) return;
         for (int i = maxi; i >= 0; --i) {
             if (rem % (unsigned long long)lens[i]) continue;
-            cur.push_back(lens[i]);
+            cur.push_back(i);
             rec(rem / lens[i], i);
             cur.pop_back();
         }
@@ -169,31 +231,44 @@ bool native_length(int prec, unsigned long long n)
     return !candidate_passes(prec, n, 1).empty();
 }
 
-// Split n into pass lengths available as T-mode tiles (largest first).  An override list
-// (GFFTX_PASSES="a,b,c") is honoured when it multiplies to n.
+// The pass split GFFTX_PASSES="a,b,c" names, when it multiplies to n and every length has a tile.
+bool env_passes(int prec, unsigned long long n, std::vector<int>& out)
+{
+    const char* env = getenv("GFFTX_PASSES");
+    if (!env) return false;
+    std::vector<int> v;
+    unsigned long long prod = 1;
+    const char* p = env;
+    while (*p) {
+        const long x = strtol(p, const_cast<char**>(&p), 10);
+        if (x <= 1) break;
+        v.push_back((int)x);
+        prod *= (unsigned long long)x;
+        if (*p == ',') ++p;
+        else break;
+    }
+    bool ok = prod == n && v.size() >= 2;
+    for (size_t i = 0; ok && i < v.size(); ++i)
+        ok = find_tile(prec, v[i], true, i == 0 ? false : true) != nullptr;
+    if (ok) out = v;
+    return ok;
+}
+
+// The single-pass tile of n, or null where n runs in passes: no tile of that length, or a
+// run-time one and a split named by GFFTX_PASSES.
+const TileEntry* single_tile(int prec, unsigned long long n, int want_nb, int want_wg)
+{
+    if (n > (1ull << 30)) return nullptr;
+    const TileEntry* k = find_tile(prec, (int)n, false, false, want_nb, want_wg);
+    std::vector<int> v;
+    return k && k->mix && env_passes(prec, n, v) ? nullptr : k;
+}
+
+// Split n into pass lengths available as T-mode tiles (largest first), or the override list.
 bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch, int cus)
 {
     out.clear();
-    if (const char* env = getenv("GFFTX_PASSES")) {
-        std::vector<int> v;
-        unsigned long long prod = 1;
-        const char* p = env;
-        while (*p) {
-            const long x = strtol(p, const_cast<char**>(&p), 10);
-            if (x <= 1) break;
-            v.push_back((int)x);
-            prod *= (unsigned long long)x;
-            if (*p == ',') ++p;
-            else break;
-        }
-        bool ok = prod == n && v.size() >= 2;
-        for (size_t i = 0; ok && i < v.size(); ++i)
-            ok = find_tile(prec, v[i], true, i == 0 ? false : true) != nullptr;
-        if (ok) {
-            out = v;
-            return true;
-        }
-    }
+    if (env_passes(prec, n, out)) return true;
     std::vector<std::vector<int>> c = candidate_passes(prec, n, 1, batch, cus);
     if (c.empty()) return false;
     out = c[0];
@@ -220,10 +295,10 @@ unsigned long long bluestein_length(int prec, unsigned long long n, unsigned lon
     double best_cost = 0;
     for (unsigned long long m : cand) {
         double per = 0;
-        if (m <= (1ull << 30) && find_tile(prec, (int)m, false, false)) {
+        if (m <= 16384 && find_tile(prec, (int)m, false, false) && !find_tile(prec, (int)m, false, false)->mix) {
             per = 1.0 / 4.0;
         } else {
-            const std::vector<std::vector<int>> c = candidate_passes(prec, m, 1, batch);
+            const std::vector<std::vector<int>> c = candidate_passes(prec, m, 1, batch, 256, false);
             if (c.empty()) continue;
             for (int L : c[0]) per += 1.0 / pass_bandwidth(prec, L);
         }

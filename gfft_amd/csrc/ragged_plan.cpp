@@ -56,7 +56,7 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
     }
     std::vector<int> lens;
     bool multi = choose_passes(r->prec, (unsigned long long)L, lens, (unsigned long long)lc.count);
-    const TileEntry* k1 = (L <= (1 << 30)) ? find_tile(r->prec, (int)L, false, false) : nullptr;
+    const TileEntry* k1 = single_tile(r->prec, (unsigned long long)L);
     bool use_single = k1 && (!multi || lc.count >= min_single);
     // measured choice between the single-pass tile and the pass splits with their tile shapes
     // (unless the caller turned autotuning off or fixed the rule with GFFTX_RAGGED_MIN_SINGLE)
@@ -83,7 +83,7 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
         ps.items_in_ntrans = true;
         ps.ntrans = lc.count;
         ps.ies = 1;
-        e = upload_stage_table_r(r->allocs, r->prec, k->nrad, k->radices, &ps.stage_tw);
+        e = upload_tile_table(r->allocs, k, &ps.stage_tw);
         if (e) return e;
         lc.passes.push_back(ps);
     } else {
@@ -91,7 +91,9 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
         long long ns = 1;
         for (size_t i = 0; i < lens.size(); ++i) {
             const int tnb = i < t_tiles.size() ? t_tiles[i].first : 0, twg = i < t_tiles.size() ? t_tiles[i].second : 0;
-            const TileEntry* k = find_tile(r->prec, lens[i], true, i > 0, tnb, twg);
+            const TileEntry* k = tnb ? find_tile(r->prec, lens[i], true, i > 0, tnb, twg)
+                                     : pass_tile(r->prec, lens[i], i == 0, (unsigned long long)L,
+                                                 (unsigned long long)lc.count, device_cus(r->device));
             if (!k) return fail(GFFTX_ERR_UNSUPPORTED, "ragged batch: no pass kernel L=%d", lens[i]);
             Pass ps;
             ps.k = k;
@@ -101,7 +103,7 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
             ps.ies = L / lens[i];
             ps.ns_pass = ns;
             ps.batch = (unsigned)lc.count;
-            e = upload_stage_table_r(r->allocs, r->prec, k->nrad, k->radices, &ps.stage_tw);
+            e = upload_tile_table(r->allocs, k, &ps.stage_tw);
             if (e) return e;
             if (ns > 1) {
                 ps.ptw_m = ns * lens[i];
@@ -157,7 +159,7 @@ int ragged_run_long(gfftx_ragged_s* r, const gfftx_ragged_s::LongClass& lc, void
             a.xcd = ps.xcd;
             grid = dim3((unsigned)((ps.ntrans + ps.k->nb - 1) / ps.k->nb), (unsigned)lc.count);
         }
-        hipError_t le = ps.k->launch(a, grid, s, nullptr, nullptr);
+        hipError_t le = launch_entry(ps.k, a, grid, s);
         if (le != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "%s: %s", ps.k->name, hipGetErrorString(le));
     }
     return GFFTX_SUCCESS;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "mfma_kernel.h"
+#include "mixed_kernel.h"
 #include "tile_kernel.h"
 
 namespace gfftx {
@@ -27,7 +28,19 @@ struct TileEntry {
     TileLaunch launch;
     const char* name;
     int real;  // REAL_NONE, or the real-transform split fused in (REAL_POST, REAL_PRE: RealCfg)
+    const MixShape* mix = nullptr;  // run-time mixed-radix tile (mixed.hip; `launch` is null)
 };
+
+// Run-time mixed-radix tiles (mixed.hip).  mixed_prepare lifts the kernel's limit on dynamic
+// LDS; it is called once per shape, when a plan is made.
+hipError_t mixed_prepare(const TileEntry& k);
+hipError_t launch_mixed(const TileEntry& k, const TileArgs& a, dim3 grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1);
+
+inline hipError_t launch_entry(const TileEntry* k, const TileArgs& a, dim3 grid, hipStream_t s, hipEvent_t t0 = nullptr,
+                               hipEvent_t t1 = nullptr)
+{
+    return k->mix ? launch_mixed(*k, a, grid, s, t0, t1) : k->launch(a, grid, s, t0, t1);
+}
 
 // Complex tiles (kernels.hip) and tiles with a real-transform split fused in (real_tiles.hip).
 extern TileEntry kTiles[];

@@ -9,8 +9,8 @@ namespace detail {
 
 // ---------------------------------------------------------------------------------------
 // Autotuner: for a multi-pass plan, time the best few pass splits of the cost model on this
-// device and keep the fastest.  Results are cached per (device, precision, n, batch, kind,
-// place) in memory and in a versioned JSON file ($GFFTX_TUNE_CACHE, default
+// device and keep the fastest.  Results are cached per (device, kernel revision, precision, n,
+// batch, kind, place) in memory and in a versioned JSON file ($GFFTX_TUNE_CACHE, default
 // ~/.cache/gfftx/tune.json).
 std::mutex g_tune_mu;
 std::map<std::string, std::vector<int>> g_tune;
@@ -148,13 +148,17 @@ void tune_put(const std::string& key, const std::vector<int>& v)
     tune_store();
 }
 
+// Revision of the kernels the cached choices were measured with: part of every key, so that a
+// cache file written by a library with other tiles is measured afresh, not taken over.
+static constexpr int kTuneRevision = 2;
+
 std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 {
     hipDeviceProp_t prop;
     std::string dev = "dev";
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) dev = std::string(prop.gcnArchName) + ":" + std::to_string(prop.multiProcessorCount) + "cu";
     else (void)hipGetLastError();
-    return dev + "|" + (prec == PREC_F64 ? "f64" : "f32") + "|n=" + std::to_string(n) + "|b=" + std::to_string(batch);
+    return dev + ":r" + std::to_string(kTuneRevision) + "|" + (prec == PREC_F64 ? "f64" : "f32") + "|n=" + std::to_string(n) + "|b=" + std::to_string(batch);
 }
 
 // Time (ms) of one execution of a plan on scratch buffers, as a throughput: three groups of
@@ -196,10 +200,21 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
     return GFFTX_SUCCESS;
 }
 
+// The cost model's best `k` splits, and its best three of compiled tiles alone where they are
+// not among them.
+static std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus)
+{
+    std::vector<std::vector<int>> v = candidate_passes(prec, n, k, batch, cus);
+    for (const std::vector<int>& c : candidate_passes(prec, n, 3, batch, cus, false))
+        if (std::find(v.begin(), v.end(), c) == v.end()) v.push_back(c);
+    return v;
+}
+
 // Tuning candidates from pass splits: each split with its default tiles, then with every
 // other compiled tile shape of its first pass (T->E) and of each length it uses after the
 // first pass (T->T), one position at a time ([lens..., 0, nb, wg per pass], 0 = default).
-static std::vector<std::vector<int>> split_variants(int prec, const std::vector<std::vector<int>>& splits)
+static std::vector<std::vector<int>> split_variants(int prec, unsigned long long n, unsigned long long batch, int cus,
+                                                    const std::vector<std::vector<int>>& splits)
 {
     std::vector<std::vector<int>> cands;
     for (const std::vector<int>& sp : splits) {
@@ -210,10 +225,10 @@ static std::vector<std::vector<int>> split_variants(int prec, const std::vector<
             const bool later = i > 0;
             if (later && std::find(seen.begin(), seen.end(), L) != seen.end()) continue;
             if (later) seen.push_back(L);
-            const TileEntry* def = find_tile(prec, L, true, later);
-            for (int t = 0; t < kNumTiles; ++t) {
-                const TileEntry& e = kTiles[t];
-                if (e.prec != prec || e.L != L || !e.loadT || e.storeT != later || &e == def) continue;
+            const TileEntry* def = pass_tile(prec, L, !later, n, batch, cus);
+            for (const TileEntry* t : tile_shapes(prec, L, true, later)) {
+                if (t == def) continue;
+                const TileEntry& e = *t;
                 std::vector<int> c = sp;
                 c.push_back(0);
                 for (size_t j = 0; j < sp.size(); ++j) {
@@ -294,15 +309,16 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
     }
     if (chosen.empty()) {
         std::vector<std::vector<int>> splits;
-        if (!single_pass)
-            splits = candidate_passes(p->prec, n, (size_t)env_int("GFFTX_TUNE_CANDIDATES", 5), batch, device_cus(device));
-        std::vector<std::vector<int>> cands = split_variants(p->prec, splits);
+        // a single-pass plan is timed against pass splits where its workgroups leave most of
+        // the device idle: no more than the CUs for a run-time tile, 8 (one per XCD) for a
+        // compiled one of a complex transform, from 2048 points up
+        const uint64_t tiles = single_pass ? (batch + p->passes[0].k->nb - 1) / p->passes[0].k->nb : 0;
+        const uint64_t few = single_pass ? (p->passes[0].k->mix ? device_cus(device) : p->real ? 0 : 8) : 0;
+        if (!single_pass || (n >= 2048 && tiles <= few))
+            splits = tuned_splits(p->prec, n, (size_t)env_int("GFFTX_TUNE_CANDIDATES", 5), batch, device_cus(device));
+        std::vector<std::vector<int>> cands = split_variants(p->prec, n, batch, device_cus(device), splits);
         if (single_pass)
-            for (int t = 0; t < kNumTiles; ++t) {
-                const TileEntry& e = kTiles[t];
-                if (e.prec == p->prec && (uint64_t)e.L == n && !e.loadT && !e.storeT)
-                    cands.push_back({(int)n, 1, 0, e.nb, e.wg});
-            }
+            for (const TileEntry* e : tile_shapes(p->prec, (int)n, false, false)) cands.push_back({(int)n, 1, 0, e->nb, e->wg});
         if (cands.size() < 2) return GFFTX_SUCCESS;
         DeviceGuard g(device);
         // the candidates run on at most 1 GiB of data (a larger batch is timed on a prefix of
@@ -342,7 +358,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             std::vector<std::pair<int, int>> tl;
             split_choice(c, sl, tl);
             std::string lens;
-            if (single_pass) {
+            if (sl.size() == 2 && sl[1] == 1) {
                 lens = "single/" + std::to_string(tl[0].first) + "-" + std::to_string(tl[0].second);
             } else {
                 for (size_t j = 0; j < sl.size(); ++j) {
@@ -360,7 +376,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             return ms;
         };
         for (size_t i = 0; i < cands.size(); ++i) cms[i] = try_cand(cands[i]);
-        if (!single_pass && !chosen.empty()) {
+        if (!chosen.empty() && chosen[1] != 1) {
             const std::vector<int> combo = best_combination(chosen, cands, cms);
             if (!combo.empty()) try_cand(combo);
         }
@@ -395,8 +411,8 @@ bool tune_length_class(int device, int prec, long long L, long long count, bool 
 {
     if (env_int("GFFTX_AUTOTUNE", 1) == 0) return false;
     const bool has_single = L <= (1 << 30) && find_tile(prec, (int)L, false, false) != nullptr;
-    const std::vector<std::vector<int>> splits = candidate_passes(prec, (unsigned long long)L, 3,
-                                                                  (unsigned long long)count, device_cus(device));
+    const std::vector<std::vector<int>> splits = tuned_splits(prec, (unsigned long long)L, 3, (unsigned long long)count,
+                                                              device_cus(device));
     if ((has_single ? 1 : 0) + splits.size() < 2) return false;
     const std::string key = tune_key(device, prec, (uint64_t)L, (uint64_t)count) + "|class";
     std::vector<int> chosen;
@@ -408,11 +424,11 @@ bool tune_length_class(int device, int prec, long long L, long long count, bool 
     }
     if (chosen.empty()) {
         std::vector<std::vector<int>> cands;
-        for (int t = 0; has_single && t < kNumTiles; ++t) {
-            const TileEntry& e = kTiles[t];
-            if (e.prec == prec && e.L == L && !e.loadT && !e.storeT) cands.push_back({(int)L, 1, 0, e.nb, e.wg});
-        }
-        for (const std::vector<int>& sp : split_variants(prec, splits)) cands.push_back(sp);
+        if (has_single)
+            for (const TileEntry* e : tile_shapes(prec, (int)L, false, false)) cands.push_back({(int)L, 1, 0, e->nb, e->wg});
+        for (const std::vector<int>& sp : split_variants(prec, (unsigned long long)L, (unsigned long long)count,
+                                                         device_cus(device), splits))
+            cands.push_back(sp);
         DeviceGuard g(device);
         // at most 1 GiB of data, like plan tuning
         const uint64_t tcount = std::min<uint64_t>((uint64_t)count,
