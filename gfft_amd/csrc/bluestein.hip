@@ -1,15 +1,10 @@
-// bluestein.hip -- element-wise kernels of the chirp-z (Bluestein) path for lengths with a
-// prime factor above 5.
+// bluestein.hip -- tables of the chirp-z (Bluestein) path for lengths with a prime factor above 7:
+// the chirp c_j = W_{2n}^{j^2} = exp(-i pi j^2 / n), the filter
+//     b_j = conj(c_j) (0 <= j < n),  b_{m-j} = conj(c_j) (0 < j < n),  0 elsewhere,
+// and its spectrum in the working precision.  The transform itself runs in the passes of
+// mixed_kernel.h (CHIRP_*).
 //
-// With c_j = W_{2n}^{j^2} = exp(-i pi j^2 / n) and jk = (j^2 + k^2 - (k-j)^2) / 2,
-//     X_k = sum_j x_j W_n^{jk} = c_k * sum_j (x_j c_j) conj(c_{k-j}),
-// a linear convolution of length 2n-1, computed as a circular one of a 2/3/5-smooth length
-// m >= 2n-1 with two FFTs of length m and the precomputed spectrum of the chirp filter
-//     b_j = conj(c_j) (0 <= j < n),  b_{m-j} = conj(c_j) (0 < j < n),  0 elsewhere.
-// The inverse transform is conj(DFT(conj x)) / n, so one filter serves both directions.
-//
-// All kernels are streaming: one complex element per thread and iteration, batch items on
-// the y dimension of the grid (grid-stride in both dimensions).
+// All kernels are streaming: one complex element per thread and iteration.
 #include "registry.h"
 
 namespace gfftx {
@@ -31,113 +26,58 @@ template <class T> __global__ __launch_bounds__(256) void chirp_table_kernel(Chi
     }
 }
 
-// b over one length-m item: conj(c_j) at j < n and at m - j for 0 < j < n, zero elsewhere.
-template <class T> __global__ __launch_bounds__(256) void chirp_filter_kernel(BluesteinArgs a)
+// b over length m: conj(c_j) at j < n and at m - j for 0 < j < n, zero elsewhere.
+template <class T> __global__ __launch_bounds__(256) void chirp_filter_kernel(const V2<T>* c, V2<T>* b, unsigned long long n, unsigned long long m)
 {
-    const V2<T>* c = (const V2<T>*)a.chirp;
-    V2<T>* b = (V2<T>*)a.work;
-    for (unsigned long long j = blockIdx.x * 256ull + threadIdx.x; j < (unsigned long long)a.m;
-         j += (unsigned long long)gridDim.x * 256ull) {
+    for (unsigned long long j = blockIdx.x * 256ull + threadIdx.x; j < m; j += (unsigned long long)gridDim.x * 256ull) {
         V2<T> v{0, 0};
-        if (j < (unsigned long long)a.n) v = cconj(c[j]);
-        else if (j > (unsigned long long)(a.m - a.n)) v = cconj(c[a.m - j]);
+        if (j < n) v = cconj(c[j]);
+        else if (j > m - n) v = cconj(c[m - j]);
         b[j] = v;
     }
 }
 
-// work[b][j] = (conj? conj(x[b][j]) : x[b][j]) * c_j for j < n, zero up to m.
-template <class T> __global__ __launch_bounds__(256) void bluestein_pre_kernel(BluesteinArgs a)
+// The filter's spectrum over m, divided in FP64 and rounded once.
+template <class F, class T> __global__ __launch_bounds__(256) void chirp_spectrum_kernel(const V2<F>* s, V2<T>* f, unsigned long long m)
 {
-    const V2<T>* c = (const V2<T>*)a.chirp;
-    const unsigned flip = a.conj ? 0x80000000u : 0u;
-    for (unsigned long long b = blockIdx.y; b < (unsigned long long)a.batch; b += gridDim.y) {
-        const V2<T>* x = (const V2<T>*)a.in + (a.boff ? (unsigned long long)a.boff[b] : b * (unsigned long long)a.dist);
-        V2<T>* w = (V2<T>*)a.work + b * (unsigned long long)a.m;
-        for (unsigned long long j = blockIdx.x * 256ull + threadIdx.x; j < (unsigned long long)a.m;
-             j += (unsigned long long)gridDim.x * 256ull) {
-            V2<T> v{0, 0};
-            if (j < (unsigned long long)a.n) {
-                V2<T> u = x[j];
-                if (flip) u.y = -u.y;
-                v = cmul(u, c[j]);
-            }
-            w[j] = v;
-        }
-    }
+    for (unsigned long long j = blockIdx.x * 256ull + threadIdx.x; j < m; j += (unsigned long long)gridDim.x * 256ull)
+        f[j] = V2<T>{(T)((double)s[j].x / (double)m), (T)((double)s[j].y / (double)m)};
 }
 
-// work[b][k] *= filter[k] over the whole length m.
-template <class T> __global__ __launch_bounds__(256) void bluestein_mul_kernel(BluesteinArgs a)
+dim3 stream_grid(long long len)
 {
-    const V2<T>* f = (const V2<T>*)a.filter;
-    for (unsigned long long b = blockIdx.y; b < (unsigned long long)a.batch; b += gridDim.y) {
-        V2<T>* w = (V2<T>*)a.work + b * (unsigned long long)a.m;
-        for (unsigned long long j = blockIdx.x * 256ull + threadIdx.x; j < (unsigned long long)a.m;
-             j += (unsigned long long)gridDim.x * 256ull)
-            w[j] = cmul(w[j], f[j]);
-    }
-}
-
-// out[b][k] = scale * (conj? conj(c_k y_k) : c_k y_k) for k < n, y = work[b].
-template <class T> __global__ __launch_bounds__(256) void bluestein_post_kernel(BluesteinArgs a)
-{
-    const V2<T>* c = (const V2<T>*)a.chirp;
-    const T sc = (T)a.scale;
-    for (unsigned long long b = blockIdx.y; b < (unsigned long long)a.batch; b += gridDim.y) {
-        const V2<T>* y = (const V2<T>*)a.work + b * (unsigned long long)a.m;
-        V2<T>* o = (V2<T>*)a.out + (a.boff ? (unsigned long long)a.boff[b] : b * (unsigned long long)a.dist);
-        for (unsigned long long k = blockIdx.x * 256ull + threadIdx.x; k < (unsigned long long)a.n;
-             k += (unsigned long long)gridDim.x * 256ull) {
-            V2<T> v = cmul(c[k], y[k]);
-            if (a.conj) v.y = -v.y;
-            o[k] = V2<T>{v.x * sc, v.y * sc};
-        }
-    }
-}
-
-dim3 stream_grid(long long len, long long batch)
-{
-    // about 16K workgroups in all (every CU many times over); the kernels stride over the rest
-    const long long gy = batch < 65535 ? batch : 65535;
-    long long gx = (len + 255) / 256;
-    const long long cap = 16384 / gy > 1 ? 16384 / gy : 1;
-    if (gx > cap) gx = cap;
-    return dim3((unsigned)gx, (unsigned)gy);
-}
-
-template <class T> hipError_t launch_bluestein_t(int which, const BluesteinArgs& a, hipStream_t s)
-{
-    switch (which) {
-        case BLUESTEIN_PRE:
-            bluestein_pre_kernel<T><<<stream_grid(a.m, a.batch), 256, 0, s>>>(a);
-            break;
-        case BLUESTEIN_MUL:
-            bluestein_mul_kernel<T><<<stream_grid(a.m, a.batch), 256, 0, s>>>(a);
-            break;
-        case BLUESTEIN_POST:
-            bluestein_post_kernel<T><<<stream_grid(a.n, a.batch), 256, 0, s>>>(a);
-            break;
-        case BLUESTEIN_FILTER:
-            chirp_filter_kernel<T><<<stream_grid(a.m, 1), 256, 0, s>>>(a);
-            break;
-        default:
-            return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    // up to 16K workgroups (every CU many times over); the kernels stride over the rest
+    const long long g = (len + 255) / 256;
+    return dim3((unsigned)(g < 16384 ? g : 16384));
 }
 
 }  // namespace
 
-hipError_t launch_bluestein(int prec, int which, const BluesteinArgs& a, hipStream_t s)
-{
-    return prec == PREC_F64 ? launch_bluestein_t<double>(which, a, s) : launch_bluestein_t<float>(which, a, s);
-}
-
 hipError_t launch_chirp_table(int prec, const ChirpTableArgs& a, hipStream_t s)
 {
-    const dim3 g = stream_grid(a.n, 1);
+    const dim3 g = stream_grid(a.n);
     if (prec == PREC_F64) chirp_table_kernel<double><<<g, 256, 0, s>>>(a);
     else chirp_table_kernel<float><<<g, 256, 0, s>>>(a);
+    return hipGetLastError();
+}
+
+hipError_t launch_chirp_filter(int prec, const void* chirp, void* b, long long n, long long m, hipStream_t s)
+{
+    const dim3 g = stream_grid(m);
+    if (prec == PREC_F64) chirp_filter_kernel<double><<<g, 256, 0, s>>>((const double2*)chirp, (double2*)b, n, m);
+    else chirp_filter_kernel<float><<<g, 256, 0, s>>>((const float2*)chirp, (float2*)b, n, m);
+    return hipGetLastError();
+}
+
+hipError_t launch_chirp_spectrum(int from, int to, const void* spec, void* filter, long long m, hipStream_t s)
+{
+    const dim3 g = stream_grid(m);
+    if (from == PREC_F64 && to == PREC_F64)
+        chirp_spectrum_kernel<double, double><<<g, 256, 0, s>>>((const double2*)spec, (double2*)filter, m);
+    else if (from == PREC_F64)
+        chirp_spectrum_kernel<double, float><<<g, 256, 0, s>>>((const double2*)spec, (float2*)filter, m);
+    else
+        chirp_spectrum_kernel<float, float><<<g, 256, 0, s>>>((const float2*)spec, (float2*)filter, m);
     return hipGetLastError();
 }
 

@@ -8,44 +8,80 @@
 //     stages and a thread holds at most MIX_POINTS points;
 //   - a stage's radix chosen by a branch that is uniform over the launch: every radix is a
 //     register butterfly of its own, nothing is indexed at run time inside it;
-//   - division by a stage's Ns as one multiplication by a precomputed reciprocal, and an LDS
-//     layout (pad elements after every R_0) in which the elements of a butterfly lie at a
-//     constant distance, so that an element costs one address addition.
+//   - division by a stage's Ns as a 24-bit multiplication and a shift (Div; 32-bit products run at
+//     a quarter of the rate and took a fifth of a stage's issue slots), and an LDS layout (pad
+//     elements after every R_0) in which the elements of a butterfly lie at a constant distance,
+//     so that an element costs one address addition.
 // Access modes as in tile_kernel.h: E->E (single pass), T->E (first pass), T->T (later passes).
 #pragma once
+#include <cstddef>
+
 #include "tile_kernel.h"
 
 namespace gfftx {
 
 constexpr int MIX_POINTS = 16;    // most points of a sequence one thread holds
-constexpr int MIX_STAGES = 14;    // 2^14 = 16384 in radix-2 stages at the very most
+constexpr int MIX_STAGES = 10;    // more than any length takes (16384 = 16*16*8*8)
 #define GFFTX_MIX_RADICES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(14) X(15) X(16)
+
+// Product of a 16-bit and a 24-bit number, the ranges spelled out: one full-rate instruction.
+__host__ __device__ __forceinline__ unsigned mul24(unsigned a, unsigned b) { return (a & 0xffffu) * (b & 0xffffffu); }
+
+// x / d = (x * m) >> s for x < 2^15, m < 2^17: s = 15 + ceil(log2 d), m = floor(2^s / d) + 1
+// (x * (m d - 2^s) < 2^s, since 0 < m d - 2^s <= d <= 2^(s - 15)).
+struct Div {
+    unsigned m, s;
+    __host__ __device__ __forceinline__ unsigned operator()(unsigned x) const
+    {
+        return mul24(x, m) >> s;
+    }
+};
 
 struct MixStage {
     unsigned R;     // radix
     unsigned lr;    // L / R: butterflies per sequence
     unsigned ns;    // product of the earlier radices
-    unsigned mns;   // ceil(2^32 / ns): j / ns = umulhi(j, mns) for j < 2^14 (ns > 1)
+    Div dns;        // j / ns
     unsigned rst;   // LDS distance of the elements j, j + L/R, .. a butterfly reads
     unsigned wst;   // LDS distance of the elements it writes (ns apart)
+    unsigned wq;    // (R - 1) wst
     unsigned tw;    // first entry of the stage's twiddles (FP32: ns FP64 roots; FP64: rows r = 1..R-1 of ns entries)
 };
 
 struct MixShape {
     unsigned L, nb, tpt, wg;  // nb sequences of tpt threads each; wg >= nb * tpt threads
-    unsigned mtpt;            // ceil(2^32 / tpt) (tpt > 1)
+    Div dtpt, dr0, dl;        // x / tpt, x / R_0, x / L
     unsigned ts;              // LDS distance between sequences
-    unsigned pad;             // LDS pad elements after every R_0 elements
-    unsigned mr0;             // ceil(2^32 / R_0)
-    unsigned ml;              // ceil(2^32 / L)
+    unsigned pad;             // LDS pad elements after every R_0 elements: 0 or 1
     unsigned nst;
     int nt_in;                // 1: rows are whole 128-byte lines, the input is loaded non-temporally
     MixStage st[MIX_STAGES];
 };
 
+// Chirp-z kinds of a tile, beside the real-transform ones (REAL_NONE, REAL_POST, REAL_PRE).  The
+// convolution of length m runs in passes P_0 .. P_k forward and P_k .. P_0 backward:
+//   CHIRP_IN    first pass (T->E): x[e] c[e] for e < n, zero beyond, in the loads;
+//   CHIRP_TURN  last forward pass and first backward pass in one (T->E).  The forward one leaves
+//               element q of sequence t at t + q S (S = m / L), which is what the backward one
+//               takes as element q of its sequence t: the filter is multiplied in between, in
+//               registers, and the conjugate goes on (the inverse FFT is conj FFT conj);
+//   CHIRP_OUT   last backward pass (T->T): conj and c[k] in the stores of k < n;
+//   CHIRP_ALL   all of it in one tile (E->E) where m points fit: HBM holds nothing but x and X.
+// The turn needs the same radix first and last: a thread's outputs of the last stage are then
+// its inputs of the first one.
+enum { CHIRP_ALL = 3, CHIRP_IN = 4, CHIRP_TURN = 5, CHIRP_OUT = 6 };
+
+struct ChirpArgs {
+    const void* chirp;   // n entries c_j = W_{2n}^{j^2}
+    const void* filter;  // m entries: FFT_m of the chirp filter, over m
+    unsigned n;
+    long long mdist;     // distance between the work array's batch items
+};
+
 struct MixArgs {
     TileArgs a;
     MixShape m;
+    ChirpArgs c;
 };
 
 enum { MIX_EE = 0, MIX_TE = 1, MIX_TT = 2 };
@@ -127,8 +163,11 @@ template <typename T> struct MixCtx {
     unsigned jt;   // thread within the sequence; beyond every butterfly for idle threads
     unsigned ies, ons;
     long long tg;  // sequence within the batch item
-    long long bo;  // element offset of the batch item
+    long long bo;  // element offset of the batch item in the output
 };
+
+// LDS index of element e (pad is 0 or 1).
+__device__ __forceinline__ unsigned mix_pos(const MixShape& m, unsigned e) { return e + (m.dr0(e) & (0u - m.pad)); }
 
 // Twiddles W^{k r}, r = 1..R-1, of one butterfly.  FP32: FP64 powers of the FP64 root, rounded
 // once (as in tile_kernel.h); FP64: the table's rows, row r contiguous in k.
@@ -184,15 +223,23 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
     constexpr int B = mix_b<R>();
     const TileArgs& a = x.a;
     const unsigned lr = x.m.st[0].lr, tpt = x.m.tpt;
+    const unsigned cn = x.c.n, e0 = REAL == CHIRP_IN ? (unsigned)c.tg : 0u;  // chirp-z: element e0 + i
+    const unsigned istep = MODE == MIX_EE ? lr : lr * c.ies;  // between the elements of a butterfly
     V v[B][R];
     with_nt(x.m.nt_in != 0, [&](auto ntc) {
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const unsigned j = c.jt + b * tpt;
             if (j >= lr) continue;
+            const unsigned i0 = MODE == MIX_EE ? j : j * c.ies;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const V* p = &c.in[MODE == MIX_EE ? j + r * lr : (j + r * lr) * c.ies];
+                const unsigned i = i0 + r * istep;
+                const V* p = &c.in[i];
+                if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_IN) {
+                    v[b][r] = V{0, 0};
+                    if (e0 + i >= cn) continue;
+                }
                 if constexpr (decltype(ntc)::value) v[b][r] = nt_load(p);
                 else v[b][r] = *p;
             }
@@ -244,14 +291,24 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
         __syncthreads();
     }
     const unsigned flip = a.conj_in ? 0x80000000u : 0u;
-    const long long kp = (MODE == MIX_TT && a.ptw_lo != nullptr) ? c.tg % a.ns_pass : 0;
+    constexpr bool PTW = MODE == MIX_TT || REAL == CHIRP_TURN;
+    const long long kp = (PTW && a.ptw_lo != nullptr) ? c.tg % a.ns_pass : 0;
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const unsigned j = c.jt + b * tpt;
         if (j >= lr) continue;
 #pragma unroll
         for (int r = 0; r < R; ++r) v[b][r] = flip_im(v[b][r], flip);
-        if constexpr (MODE == MIX_TT) {
+        if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_IN) {
+            const V* ch = reinterpret_cast<const V*>(x.c.chirp) + e0;
+            const unsigned i0 = MODE == MIX_EE ? j : j * c.ies;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const unsigned i = i0 + r * istep;
+                if (e0 + i < cn) v[b][r] = cmul(v[b][r], ch[i]);
+            }
+        }
+        if constexpr (PTW) {
             if (kp != 0) {
                 // W_M^{kp e}, e = j + r lr: base W^{kp j} times step^r, step = W^{kp lr}
                 const long long pm = (1LL << a.ptw_shift) - 1, m0 = kp * j, ms = kp * lr;
@@ -267,7 +324,7 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
         }
         Dft<R>::run(v[b]);
         if constexpr (!ONLY) {
-            V* w = c.lds + j * (R + x.m.pad);
+            V* w = c.lds + mul24(j, R + x.m.pad);
 #pragma unroll
             for (int r = 0; r < R; ++r) w[r] = v[b][r];
         }
@@ -302,22 +359,21 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
     const TileArgs& a = x.a;
     const unsigned lr = st.lr, tpt = x.m.tpt, rst = st.rst;
     V v[B][R];
-    // LDS index of element j, and of the first element butterfly j writes
-    auto rpos = [&](unsigned j) { return j + x.m.pad * __umulhi(j, x.m.mr0); };
-    auto quot = [&](unsigned j) { return LAST ? 0u : __umulhi(j, st.mns); };  // after the last stage ns = lr > j
+    // j / ns (the last stage has ns = lr > j)
+    auto quot = [&](unsigned j) { return LAST ? 0u : st.dns(j); };
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const unsigned j = c.jt + b * tpt;
         if (j >= lr) continue;
-        const V* rd = c.lds + rpos(j);
+        const V* rd = c.lds + mix_pos(x.m, j);
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[b][r] = rd[r * rst];
+        for (int r = 0; r < R; ++r, rd += rst) v[b][r] = *rd;
     }
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const unsigned j = c.jt + b * tpt;
         if (j < lr) {
-            mix_twiddle<T, R>(v[b], a.tw, st, j - quot(j) * st.ns);
+            mix_twiddle<T, R>(v[b], a.tw, st, j - mul24(quot(j), st.ns));
             Dft<R>::run(v[b]);
         }
         __builtin_amdgcn_sched_barrier(0);  // one butterfly's twiddles at a time (registers)
@@ -326,15 +382,27 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
         const unsigned fo = a.conj_out ? 0x80000000u : 0u;
         const T sc = (T)a.scale;
         const bool one = a.scale == 1.0;
+        const V* chirp = reinterpret_cast<const V*>(x.c.chirp);  // (copies: the lambda would take x's address)
+        const unsigned cn = x.c.n, ostep = MODE == MIX_EE ? lr : lr * c.ons;
         with_nt(a.nt_out != 0, [&](auto ntc) {
 #pragma unroll
             for (int b = 0; b < B; ++b) {
                 const unsigned j = c.jt + b * tpt;
                 if (j >= lr) continue;
+                const unsigned i0 = MODE == MIX_EE ? j : j * c.ons;
 #pragma unroll
-                for (int r = 0; r < R; ++r)
-                    put<decltype(ntc)::value>(&c.out[MODE == MIX_EE ? j + r * lr : (j + r * lr) * c.ons],
-                                              flip_im(one ? v[b][r] : cscale(v[b][r], sc), fo));
+                for (int r = 0; r < R; ++r) {
+                    const unsigned i = i0 + r * ostep;
+                    if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_OUT) {
+                        const unsigned k = (REAL == CHIRP_OUT ? (unsigned)c.tg : 0u) + i;
+                        if (k < cn) {
+                            const V u = cmul(chirp[k], V{v[b][r].x, -v[b][r].y});
+                            put<decltype(ntc)::value>(&c.out[i], flip_im(one ? u : cscale(u, sc), fo));
+                        }
+                    } else {
+                        put<decltype(ntc)::value>(&c.out[i], flip_im(one ? v[b][r] : cscale(v[b][r], sc), fo));
+                    }
+                }
             }
         });
     } else {
@@ -343,12 +411,61 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
         for (int b = 0; b < B; ++b) {
             const unsigned j = c.jt + b * tpt;
             if (j >= lr) continue;
-            V* wr = c.lds + rpos(j) + quot(j) * (R - 1) * st.wst;
+            V* wr = c.lds + mix_pos(x.m, j) + mul24(quot(j), st.wq);
 #pragma unroll
-            for (int r = 0; r < R; ++r) wr[r * st.wst] = v[b][r];
+            for (int r = 0; r < R; ++r, wr += st.wst) *wr = v[b][r];
         }
         __syncthreads();
     }
+}
+
+// The turn of a chirp-z tile: last stage of the forward transform, filter, conjugate, first stage
+// of the backward one (the same radix), back to the LDS.
+template <typename T, int REAL, int R>
+__device__ __forceinline__ void mix_turn(const MixArgs& x, MixCtx<T>& c, const MixStage& st)
+{
+    using V = V2<T>;
+    constexpr int B = mix_b<R>();
+    const unsigned lr = st.lr, tpt = x.m.tpt, rst = st.rst;
+    V v[B][R];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const unsigned j = c.jt + b * tpt;
+        if (j >= lr) continue;
+        const V* rd = c.lds + mix_pos(x.m, j);
+#pragma unroll
+        for (int r = 0; r < R; ++r, rd += rst) v[b][r] = *rd;
+    }
+    const unsigned istep = REAL == CHIRP_TURN ? lr * c.ies : lr;
+    const V* filter = reinterpret_cast<const V*>(x.c.filter) + (REAL == CHIRP_TURN ? (unsigned)c.tg : 0u);
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const unsigned j = c.jt + b * tpt;
+        if (j < lr) {
+            mix_twiddle<T, R>(v[b], x.a.tw, st, j);
+            Dft<R>::run(v[b]);
+            const unsigned i0 = REAL == CHIRP_TURN ? j * c.ies : j;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const unsigned i = i0 + r * istep;
+                v[b][r] = cmul(v[b][r], filter[i]);
+                v[b][r].y = -v[b][r].y;
+                if (sizeof(T) == 8 && r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            Dft<R>::run(v[b]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const unsigned j = c.jt + b * tpt;
+        if (j >= lr) continue;
+        V* w = c.lds + mul24(j, R + x.m.pad);
+#pragma unroll
+        for (int r = 0; r < R; ++r) w[r] = v[b][r];
+    }
+    __syncthreads();
 }
 
 // T->E store: the tile's nb * L outputs are one contiguous run (first pass, Ns = 1).
@@ -366,8 +483,8 @@ template <typename T> __device__ __forceinline__ void mix_finish_te(const MixArg
     with_nt(a.nt_out != 0, [&](auto ntc) {
 #pragma unroll 4
         for (unsigned lin = threadIdx.x; lin < total; lin += x.m.wg) {
-            const unsigned t = __umulhi(lin, x.m.ml), q = lin - t * L;
-            const V u = lds[t * x.m.ts + q + x.m.pad * __umulhi(q, x.m.mr0)];
+            const unsigned t = x.m.dl(lin), q = lin - mul24(t, L);
+            const V u = lds[mul24(t, x.m.ts) + mix_pos(x.m, q)];
             put<decltype(ntc)::value>(&o[lin], flip_im(one ? u : cscale(u, sc), fo));
         }
     });
@@ -384,7 +501,7 @@ template <typename T> __device__ __forceinline__ void mix_split(const MixArgs& x
     const long long mask = (1LL << a.sp_shift) - 1;
     double2 w = dmul(a.sp_lo[c.jt & mask], a.sp_hi[c.jt >> a.sp_shift]);
     const double2 step = dmul(a.sp_lo[tpt & mask], a.sp_hi[tpt >> a.sp_shift]);
-    auto at = [&](unsigned e) { return c.lds[e + x.m.pad * __umulhi(e, x.m.mr0)]; };
+    auto at = [&](unsigned e) { return c.lds[mix_pos(x.m, e)]; };
 #pragma unroll 4
     for (unsigned k = c.jt; k < L; k += tpt) {
         const V zk = at(k), zp = at(k == 0 ? 0 : L - k);
@@ -409,8 +526,35 @@ template <typename T> __device__ __forceinline__ void mix_split(const MixArgs& x
     }
 }
 
+// Stage s of the launch's shape, read from the kernel arguments where they lie (MixArgs is the only
+// argument): indexing the by-value struct at run time makes the compiler copy all of it to scratch
+// memory (616 bytes a thread; the chirp-z tile then ran three times as long).
+__device__ __forceinline__ MixStage mix_stage_args(unsigned s)
+{
+    typedef const __attribute__((address_space(4))) unsigned char* Bytes;
+    typedef const __attribute__((address_space(4))) MixStage* Stages;
+    const Bytes k = (Bytes)__builtin_amdgcn_kernarg_segment_ptr();
+    const Stages st = (Stages)(k + offsetof(MixArgs, m) + offsetof(MixShape, st)) + s;
+    return MixStage{st->R, st->lr, st->ns, Div{st->dns.m, st->dns.s}, st->rst, st->wst, st->wq, st->tw};
+}
+
+// The stages between the first and the last one.
+template <typename T, int MODE, int REAL> __device__ __forceinline__ void mix_middle(const MixArgs& x, MixCtx<T>& c)
+{
+    for (unsigned s = 1; s + 1 < x.m.nst; ++s) {
+        const MixStage st = mix_stage_args(s);
+        switch (st.R) {
+#define X(R_) \
+    case R_: mix_stage<T, MODE, REAL, R_, false>(x, c, st); break;
+            GFFTX_MIX_RADICES(X)
+#undef X
+            default: break;
+        }
+    }
+}
+
 template <typename T, int MODE, int REAL>
-__global__ __launch_bounds__(1024, sizeof(T) == 4 ? 6 : 4) void mixed_kernel(MixArgs x)
+__global__ __launch_bounds__(1024, sizeof(T) == 8 ? 4 : MODE == MIX_EE && REAL != REAL_PRE ? 6 : 5) void mixed_kernel(MixArgs x)
 {
     using V = V2<T>;
     extern __shared__ __align__(16) unsigned char mix_lds[];
@@ -420,7 +564,7 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 6 : 4) void mixed_kernel(Mix
     unsigned t;
     MixCtx<T> c;
     if constexpr (MODE == MIX_EE) {
-        t = x.m.tpt == 1 ? tid : __umulhi(tid, x.m.mtpt);
+        t = x.m.dtpt(tid);
         c.jt = tid - t * x.m.tpt;
     } else {
         t = tid & (x.m.nb - 1);  // nb is a power of two in the T modes
@@ -434,10 +578,12 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 6 : 4) void mixed_kernel(Mix
         c.tg = 0;
         t = 0;
     }
-    c.bo = batch_offset(a, blockIdx.y);
+    const long long bo = batch_offset(a, blockIdx.y);
+    c.bo = REAL == CHIRP_IN ? (long long)blockIdx.y * x.c.mdist : bo;
     c.lds = lds + t * x.m.ts;
     const long long so = a.seq_off ? a.seq_off[c.tg] : 0;
-    c.in = reinterpret_cast<const V*>(a.in) + c.bo + (a.seq_off ? so : c.tg * a.its);
+    c.in = reinterpret_cast<const V*>(a.in) + (REAL == CHIRP_OUT ? (long long)blockIdx.y * x.c.mdist : bo) +
+           (a.seq_off ? so : c.tg * a.its);
     c.ies = (unsigned)a.ies;
     c.ons = (unsigned)a.ns_pass;
     long long ob = so;
@@ -465,17 +611,18 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 6 : 4) void mixed_kernel(Mix
 #undef X
         default: break;
     }
-    for (unsigned s = 1; s + 1 < nst; ++s) {
-        const MixStage st = x.m.st[s];
-        switch (st.R) {
+    mix_middle<T, MODE, REAL>(x, c);
+    const MixStage sl = mix_stage_args(nst - 1);
+    if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_TURN) {
+        switch (sl.R) {
 #define X(R_) \
-    case R_: mix_stage<T, MODE, REAL, R_, false>(x, c, st); break;
+    case R_: mix_turn<T, REAL, R_>(x, c, sl); break;
             GFFTX_MIX_RADICES(X)
 #undef X
             default: break;
         }
+        mix_middle<T, MODE, REAL>(x, c);
     }
-    const MixStage sl = x.m.st[nst - 1];
     switch (sl.R) {
 #define X(R_) \
     case R_: mix_stage<T, MODE, REAL, R_, true>(x, c, sl); break;

@@ -83,7 +83,32 @@ std::vector<int> mix_radices(int L, size_t least)
     return best;
 }
 
-unsigned recip(unsigned d) { return d <= 1 ? 0 : (unsigned)(((1ull << 32) + d - 1) / d); }
+// The same for a chirp-z turn: the first radix and the last one alike.
+std::vector<int> turn_radices(int L)
+{
+    std::vector<int> best;
+    double best_cost = 0;
+    for (int R : kMixRadix) {
+        if (L % (R * R)) continue;
+        std::vector<int> r = L == R * R ? std::vector<int>() : mix_radices(L / (R * R), 1);
+        if (L != R * R && r.empty()) continue;
+        r.insert(r.begin(), R);
+        r.push_back(R);
+        const double c = shape_cost(L, r);
+        if (best.empty() || c < best_cost) {
+            best = r;
+            best_cost = c;
+        }
+    }
+    return best;
+}
+
+Div divisor(unsigned d)
+{
+    unsigned s = 15;
+    while ((1u << (s - 15)) < d) ++s;
+    return Div{(unsigned)((1ull << s) / d) + 1, s};
+}
 
 struct MixTile {
     TileEntry e;
@@ -105,10 +130,10 @@ bool fill(MixTile& t, int prec, int L, bool loadT, bool storeT, int real, int nb
     const unsigned wg = (m.tpt * nb + 63) / 64 * 64;
     if (wg > 1024) return false;
     m.wg = wg;
-    m.mtpt = recip(m.tpt);
+    m.dtpt = divisor(m.tpt);
     m.pad = r[0] % 2 == 0 ? 1 : 0;  // an odd distance between the runs the first stage writes
-    m.mr0 = recip(r[0]);
-    m.ml = recip(L);
+    m.dr0 = divisor(r[0]);
+    m.dl = divisor(L);
     m.nst = (unsigned)r.size();
     m.ts = L + m.pad * (L / r[0]);
     if (m.ts % 2 == 0) ++m.ts;      // lanes that walk sequences hit distinct banks
@@ -118,9 +143,10 @@ bool fill(MixTile& t, int prec, int L, bool loadT, bool storeT, int real, int nb
         st.R = r[s];
         st.lr = L / r[s];
         st.ns = ns;
-        st.mns = recip(ns);
+        st.dns = divisor(ns);
         st.rst = st.lr + (s ? m.pad * st.lr / r[0] : 0);
         st.wst = s ? ns + m.pad * ns / r[0] : 1;
+        st.wq = (st.R - 1) * st.wst;
         st.tw = tw;
         if (s) tw += prec == PREC_F64 ? ns * (r[s] - 1) : ns;
         ns *= r[s];
@@ -191,7 +217,8 @@ const std::vector<MixTile*>& tiles_locked(int prec, int L, bool loadT, bool stor
     auto it = g_mix.find(key);
     if (it != g_mix.end()) return it->second;
     std::vector<MixTile*> v;
-    const std::vector<int> r = mix_radices(L, loadT || real != REAL_NONE ? 2 : 1);
+    const std::vector<int> r = real == CHIRP_ALL || real == CHIRP_TURN ? turn_radices(L)
+                                                                       : mix_radices(L, loadT || real != REAL_NONE ? 2 : 1);
     if (!r.empty())
         for (int nb : tile_widths(prec, L, loadT, r)) {
             MixTile* t = new MixTile();
@@ -201,8 +228,14 @@ const std::vector<MixTile*>& tiles_locked(int prec, int L, bool loadT, bool stor
             }
             char buf[96];
             snprintf(buf, sizeof(buf), "mixed_%s_L%d_nb%d_wg%d_%s", prec == PREC_F64 ? "double" : "float", L, nb, t->e.wg,
-                     loadT ? (storeT ? "truetrue" : "truefalse")
-                           : real == REAL_POST ? "e_split" : real == REAL_PRE ? "e_presplit" : "falsefalse");
+                     real == CHIRP_ALL    ? "chirp"
+                     : real == CHIRP_IN   ? "chirp_in"
+                     : real == CHIRP_TURN ? "chirp_turn"
+                     : real == CHIRP_OUT  ? "chirp_out"
+                     : loadT              ? (storeT ? "truetrue" : "truefalse")
+                     : real == REAL_POST  ? "e_split"
+                     : real == REAL_PRE   ? "e_presplit"
+                                          : "falsefalse");
             t->name = buf;
             t->e.name = t->name.c_str();
             t->e.radices = t->radices.data();
@@ -221,7 +254,8 @@ int mix_max(int prec, bool loadT) { return prec == PREC_F64 ? (loadT ? 2048 : 81
 std::vector<const TileEntry*> mix_tiles(int prec, int L, bool loadT, bool storeT, int real)
 {
     std::vector<const TileEntry*> out;
-    if (L < 2 || L > mix_max(prec, loadT) || (storeT && !loadT) || (real != REAL_NONE && loadT)) return out;
+    if (L < 2 || L > mix_max(prec, loadT) || (storeT && !loadT)) return out;
+    if (loadT && (real == REAL_POST || real == REAL_PRE)) return out;
     int rest = L;
     for (int f : {2, 3, 5, 7})
         while (rest % f == 0) rest /= f;
@@ -230,6 +264,9 @@ std::vector<const TileEntry*> mix_tiles(int prec, int L, bool loadT, bool storeT
     for (MixTile* t : tiles_locked(prec, L, loadT, storeT, real)) out.push_back(&t->e);
     return out;
 }
+
+// Modelled time of one of a tile's sequences (shape_cost).
+double mix_cost(const TileEntry& e) { return shape_cost(e.L, std::vector<int>(e.radices, e.radices + e.nrad)); }
 
 // Stage twiddles of a run-time tile: FP32 the FP64 roots W_{Ns R}^k (k < Ns) of every later
 // stage, FP64 the rows W_{Ns R}^{k r}, r = 1..R-1, each contiguous in k.

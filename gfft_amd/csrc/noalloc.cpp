@@ -55,7 +55,7 @@ int gfftx_exec_inplace_noalloc(gfftx_plan plan, void* data, void* stream)
     if (!plan) return fail(GFFTX_ERR_INVALID_ARG, "plan is NULL");
     if (!data) return fail(GFFTX_ERR_INVALID_ARG, "data is NULL");
     if (plan->place != GFFTX_IN_PLACE) return fail(GFFTX_ERR_INVALID_ARG, "plan is out-of-place");
-    if (plan->blue_fwd)
+    if (plan->blue_m)
         return fail(GFFTX_ERR_UNSUPPORTED, "no-allocation calls take lengths of the factors 2, 3, 5 and 7 only (n=%llu)",
                     plan->n);
     const size_t bytes = (size_t)plan->dist * plan->batch * elem_bytes(plan->prec);

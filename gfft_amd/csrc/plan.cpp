@@ -261,12 +261,9 @@ void prof_end(gfftx_plan_s* p, size_t slot, hipStream_t s, const std::pair<hipEv
 }
 
 // Runs the pass list of `p` on batch items `r` of the arrays `in`/`out` (base pointers of
-// the whole batch).  Profiling events go to the slots of `prof` (the plan itself, or the
-// plan that owns `p` as an inner plan) starting at `slot0`.
-int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r, gfftx_plan_s* prof,
-               size_t slot0)
+// the whole batch).
+int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r)
 {
-    if (!prof) prof = p;
     if (!r.nb) r.nb = p->batch;
     const size_t off = (size_t)r.b0 * p->dist * elem_bytes(p->prec);
     auto at = [off](const void* q) { return (void*)((char*)const_cast<void*>(q) + off); };
@@ -300,9 +297,9 @@ int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range 
             ma.nt_out = (r.nt && i == m - 1) ? 1 : 0;
             dim3 grid((unsigned)((ma.ntrans + ps.mfma->nb - 1) / ps.mfma->nb));
             std::pair<hipEvent_t, hipEvent_t> ev;
-            const bool on = prof_begin(prof, slot0 + i, ps.mfma->name, s, &ev, true);
+            const bool on = prof_begin(p, i, ps.mfma->name, s, &ev, true);
             hipError_t e = ps.mfma->launch(ma, grid, s, on ? ev.first : nullptr, on ? ev.second : nullptr);
-            if (on) prof_end(prof, slot0 + i, s, ev, true);
+            if (on) prof_end(p, i, s, ev, true);
             if (e != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "%s: %s", ps.mfma->name, hipGetErrorString(e));
             src = dst[i];
             continue;
@@ -342,9 +339,9 @@ int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range 
         }
         dim3 grid(ntiles, ps.items_in_ntrans ? 1u : (unsigned)r.nb);
         std::pair<hipEvent_t, hipEvent_t> ev;
-        const bool on = prof_begin(prof, slot0 + i, ps.k->name, s, &ev, true);
+        const bool on = prof_begin(p, i, ps.k->name, s, &ev, true);
         hipError_t e = launch_entry(ps.k, a, grid, s, on ? ev.first : nullptr, on ? ev.second : nullptr);
-        if (on) prof_end(prof, slot0 + i, s, ev, true);
+        if (on) prof_end(p, i, s, ev, true);
         if (e != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "%s: %s", ps.k->name, hipGetErrorString(e));
         src = dst[i];
     }
@@ -354,60 +351,12 @@ int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range 
 // Launch slots the complex transform of `p` uses (profiling); the split pass comes next.
 size_t c2c_slots(const gfftx_plan_s* p)
 {
-    if (!p->blue_fwd) return p->passes.size();
-    return 3 + p->blue_fwd->passes.size() + p->blue_inv->passes.size();
-}
-
-int blue_launch(gfftx_plan_s* p, int which, const BluesteinArgs& a, size_t slot, const char* name, hipStream_t s)
-{
-    std::pair<hipEvent_t, hipEvent_t> ev;
-    const bool on = prof_begin(p, slot, name, s, &ev, false);
-    hipError_t e = launch_bluestein(p->prec, which, a, s);
-    if (on) prof_end(p, slot, s, ev, false);
-    if (e != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "%s: %s", name, hipGetErrorString(e));
-    return GFFTX_SUCCESS;
-}
-
-// Chirp-z transform: pre-multiply into the zero-padded work buffer, forward FFT of length m,
-// multiply by the filter spectrum, inverse FFT, post-multiply into `out`.
-// `boff` (optional) gives the element offset of every batch item in `in` and `out`; the
-// range must then cover the whole batch.
-int run_bluestein(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r, const long long* boff)
-{
-    if (!r.nb) r.nb = p->batch;
-    r.nt = false;  // the inner transforms write the work array, which the next kernel reads
-    const size_t eb = elem_bytes(p->prec);
-    BluesteinArgs a;
-    memset(&a, 0, sizeof(a));
-    a.boff = boff;
-    a.in = (const char*)in + (boff ? 0 : (size_t)r.b0 * p->dist * eb);
-    a.out = (char*)out + (boff ? 0 : (size_t)r.b0 * p->dist * eb);
-    a.work = (char*)p->blue_work + (size_t)r.b0 * p->blue_m * eb;
-    a.chirp = p->blue_chirp;
-    a.filter = p->blue_filter;
-    a.n = (long long)p->n;
-    a.m = (long long)p->blue_m;
-    a.dist = (long long)p->dist;
-    a.batch = (long long)r.nb;
-    a.conj = p->inverse ? 1 : 0;
-    a.scale = p->inverse ? 1.0 / (double)p->n : 1.0;
-    size_t slot = 0;
-    int rc = blue_launch(p, BLUESTEIN_PRE, a, slot++, "bluestein_pre", s);
-    if (rc) return rc;
-    rc = run_passes(p->blue_fwd, p->blue_work, p->blue_work, s, r, p, slot);
-    if (rc) return rc;
-    slot += p->blue_fwd->passes.size();
-    rc = blue_launch(p, BLUESTEIN_MUL, a, slot++, "bluestein_mul", s);
-    if (rc) return rc;
-    rc = run_passes(p->blue_inv, p->blue_work, p->blue_work, s, r, p, slot);
-    if (rc) return rc;
-    slot += p->blue_inv->passes.size();
-    return blue_launch(p, BLUESTEIN_POST, a, slot, "bluestein_post", s);
+    return p->blue_m ? p->blue.size() : p->passes.size();
 }
 
 int run_c2c(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r)
 {
-    return p->blue_fwd ? run_bluestein(p, in, out, s, r) : run_passes(p, in, out, s, r);
+    return p->blue_m ? run_bluestein(p, in, out, s, r) : run_passes(p, in, out, s, r);
 }
 
 int run_split(gfftx_plan_s* p, void* data, hipStream_t s, Range r)
@@ -527,81 +476,6 @@ int exec_any(gfftx_plan_s* p, const void* in, void* out, hipStream_t s)
     return exec_dispatch(p, in, out, s);
 }
 
-// Moves the scratch buffers of `src` into `dst` where both have one (same length, batch and
-// precision): the two inner plans of a chirp-z plan run one after the other on one stream.
-void share_scratch(gfftx_plan_s* dst, gfftx_plan_s* src)
-{
-    for (int k = 0; k < 2; ++k) {
-        if (!dst->scratch[k] || !src->scratch[k]) continue;
-        auto it = std::find(dst->allocs.begin(), dst->allocs.end(), dst->scratch[k]);
-        if (it != dst->allocs.end()) dst->allocs.erase(it);
-        (void)hipFree(dst->scratch[k]);
-        dst->scratch[k] = src->scratch[k];
-    }
-}
-
-int build_bluestein(gfftx_plan_s* p)
-{
-    const unsigned long long n = p->n;
-    if (p->flags & GFFTX_FLAG_SPLIT_MFMA)
-        return fail(GFFTX_ERR_UNSUPPORTED, "split-precision MFMA path: FP32 C2C of length 256 or 4096 only (n=%llu)", n);
-    if (n < 2 || 2 * n - 1 > bluestein_max_m(p->prec))
-        return fail(GFFTX_ERR_UNSUPPORTED, "length %llu with a prime factor above 5: the chirp-z path takes 2 <= n <= %llu",
-                    n, (bluestein_max_m(p->prec) + 1) / 2);
-    const unsigned long long m = bluestein_length(p->prec, n, p->batch);
-    if (!m) return fail(GFFTX_ERR_UNSUPPORTED, "no convolution length for n=%llu", n);
-    p->blue_m = m;
-    const int cvt = p->prec == PREC_F64 ? GFFTX_COMPLEX_DOUBLE : GFFTX_COMPLEX_FLOAT;
-    const uint32_t iflags = p->flags & GFFTX_FLAG_NO_AUTOTUNE;
-    gfftx_plan f = nullptr, b = nullptr;
-    int rc = create_plan(&f, m, p->batch, cvt, GFFTX_DFT, GFFTX_IN_PLACE, p->device, iflags);
-    if (rc) return rc;
-    p->blue_fwd = f;
-    rc = create_plan(&b, m, p->batch, cvt, GFFTX_IDFT, GFFTX_IN_PLACE, p->device, iflags);
-    if (rc) return rc;
-    p->blue_inv = b;
-    share_scratch(b, f);
-    const size_t eb = elem_bytes(p->prec);
-    rc = dev_alloc(p, &p->blue_work, (size_t)m * p->batch * eb);
-    if (rc) return rc;
-    rc = dev_alloc(p, &p->blue_chirp, (size_t)n * eb);
-    if (rc) return rc;
-    rc = dev_alloc(p, &p->blue_filter, (size_t)m * eb);
-    if (rc) return rc;
-    // chirp from the two-level root table of order 2n
-    ChirpTableArgs ca;
-    memset(&ca, 0, sizeof(ca));
-    ca.chirp = p->blue_chirp;
-    ca.n = (long long)n;
-    rc = upload_root_tables(p->allocs, (long long)(2 * n), const_cast<double2**>(&ca.lo),
-                            const_cast<double2**>(&ca.hi), &ca.shift);
-    if (rc) return rc;
-    hipError_t e = launch_chirp_table(p->prec, ca, nullptr);
-    if (e != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "chirp table: %s", hipGetErrorString(e));
-    // filter spectrum: b in the work buffer, one forward transform of length m into the filter
-    BluesteinArgs ba;
-    memset(&ba, 0, sizeof(ba));
-    ba.work = p->blue_work;
-    ba.chirp = p->blue_chirp;
-    ba.n = (long long)n;
-    ba.m = (long long)m;
-    ba.batch = 1;
-    e = launch_bluestein(p->prec, BLUESTEIN_FILTER, ba, nullptr);
-    if (e != hipSuccess) return fail(GFFTX_ERR_LAUNCH, "chirp filter: %s", hipGetErrorString(e));
-    gfftx_plan fp = nullptr;
-    rc = create_plan_impl(&fp, m, 1, cvt, GFFTX_DFT, GFFTX_OUT_OF_PLACE, p->device, 0, {}, "");
-    if (rc) return rc;
-    rc = exec_device(fp, p->blue_work, p->blue_filter, nullptr);
-    const hipError_t se = hipStreamSynchronize(nullptr);
-    gfftx_plan_destroy(fp);
-    if (rc) return rc;
-    if (se != hipSuccess) return fail(GFFTX_ERR_DEVICE, "filter transform: %s", hipGetErrorString(se));
-    p->desc = "{\"n\":" + std::to_string(n) + ",\"batch\":" + std::to_string(p->batch) + ",\"precision\":\"" +
-              (p->prec == PREC_F64 ? "f64" : "f32") + "\",\"passes\":[],\"bluestein\":{\"m\":" + std::to_string(m) +
-              ",\"fwd\":" + f->desc + ",\"inv\":" + b->desc + "}}";
-    return GFFTX_SUCCESS;
-}
-
 int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
                      uint32_t flags, const std::vector<int>& forced, const std::string& note)
 {
@@ -663,7 +537,7 @@ int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int
         return rc;
     }
     // device arrays that every call writes: calls from different streams must not overlap
-    p->shared_state = p->scratch[0] || p->blue_fwd || p->real_work || (flags & GFFTX_FLAG_GRAPH);
+    p->shared_state = p->scratch[0] || p->blue_work[0] || p->real_work || (flags & GFFTX_FLAG_GRAPH);
     *out = p;
     return GFFTX_SUCCESS;
 }
@@ -771,8 +645,6 @@ int gfftx_plan_destroy(gfftx_plan plan)
     if (plan->done_ev) (void)hipEventDestroy(plan->done_ev);
     if (plan->h2d_stream) (void)hipStreamDestroy(plan->h2d_stream);
     if (plan->d2h_stream) (void)hipStreamDestroy(plan->d2h_stream);
-    if (plan->blue_inv) gfftx_plan_destroy(plan->blue_inv);  // shares scratch owned by blue_fwd
-    if (plan->blue_fwd) gfftx_plan_destroy(plan->blue_fwd);
     for (auto& sl : plan->slots) {
         for (auto& ev : sl.pending) { (void)hipEventDestroy(ev.first); (void)hipEventDestroy(ev.second); }
         for (auto& ev : sl.pool) { (void)hipEventDestroy(ev.first); (void)hipEventDestroy(ev.second); }

@@ -66,6 +66,7 @@ struct Pass {
     double2* sp_lo = nullptr;      // its W_{2N} table
     double2* sp_hi = nullptr;
     int sp_shift = 0;
+    const char* slot = nullptr;    // chirp-z passes: name of the profiling slot
 };
 
 // Batch items [b0, b0 + nb) of a plan; nb == 0 means every item.
@@ -83,6 +84,7 @@ inline size_t elem_bytes(int prec) { return prec == PREC_F64 ? 16 : 8; }
 // --- mixed_plan.cpp: run-time mixed-radix tiles
 int mix_max(int prec, bool loadT);
 std::vector<const TileEntry*> mix_tiles(int prec, int L, bool loadT, bool storeT, int real = REAL_NONE);
+double mix_cost(const TileEntry& e);
 int upload_tile_table(std::vector<void*>& owned, const TileEntry* k, void** out);
 
 std::vector<const TileEntry*> tile_shapes(int prec, int L, bool loadT, bool storeT);
@@ -101,8 +103,6 @@ void split_choice(const std::vector<int>& c, std::vector<int>& lens, std::vector
 int xcd_remap(const TileEntry* k, int prec);
 bool native_length(int prec, unsigned long long n);
 bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch = 1, int cus = 256);
-unsigned long long bluestein_max_m(int prec);
-unsigned long long bluestein_length(int prec, unsigned long long n, unsigned long long batch);
 int dev_alloc_list(std::vector<void*>& owned, void** out, size_t bytes);
 int upload_stage_table_r(std::vector<void*>& owned, int prec, int nrad, const int* radices, void** out,
                          double scale = 1.0);
@@ -267,13 +267,12 @@ struct gfftx_plan_s {
     bool no_events = false;
     // GFFTX_FLAG_GRAPH: launches captured once per (in, out) pair and replayed
     GraphCache graphs;
-    // chirp-z path (n has a prime factor above 5): convolution of length blue_m
+    // chirp-z path (n has a prime factor above 7): convolution of length blue_m
     unsigned long long blue_m = 0;
-    gfftx_plan_s* blue_fwd = nullptr;  // forward C2C of length blue_m, in place on blue_work
-    gfftx_plan_s* blue_inv = nullptr;  // inverse C2C (1/blue_m), in place on blue_work
+    std::vector<Pass> blue;            // one CHIRP_ALL tile, or the 2k - 1 passes of both transforms
     void* blue_chirp = nullptr;        // n entries W_{2n}^{j^2}
-    void* blue_filter = nullptr;       // blue_m entries: spectrum of the chirp filter
-    void* blue_work = nullptr;         // batch x blue_m
+    void* blue_filter = nullptr;       // blue_m entries: spectrum of the chirp filter, over blue_m
+    void* blue_work[2] = {nullptr, nullptr};  // batch x blue_m each (several passes)
     // calls from several threads run one at a time: the graph cache, the profiling slots and
     // the host staging are the plan's own
     std::mutex mu;
@@ -334,8 +333,16 @@ int dev_alloc(gfftx_plan_s* p, void** out, size_t bytes);
 int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
                      uint32_t flags, const std::vector<int>& forced, const std::string& note);
 int exec_device(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r = Range());
-int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r, gfftx_plan_s* prof = nullptr,
-               size_t slot0 = 0);
+int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r);
+bool prof_begin(gfftx_plan_s* p, size_t slot, const char* name, hipStream_t s, std::pair<hipEvent_t, hipEvent_t>* ev,
+                bool attached);
+void prof_end(gfftx_plan_s* p, size_t slot, hipStream_t s, const std::pair<hipEvent_t, hipEvent_t>& ev, bool attached);
+
+// --- chirp_plan.cpp: chirp-z transforms
+unsigned long long bluestein_max_m(int prec);
+std::vector<std::vector<int>> chirp_candidates(int prec, unsigned long long n, unsigned long long batch, int cus, size_t k);
+std::vector<std::vector<int>> chirp_variants(int prec, unsigned long long n, const std::vector<int>& v, size_t i);
+int build_bluestein(gfftx_plan_s* p);
 int run_bluestein(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r, const long long* boff = nullptr);
 
 // --- host_pipeline.cpp: host-pointer calls

@@ -1,5 +1,5 @@
-// planner.cpp -- twiddle roots, compiled-tile lookup, the pass cost model and pass splits,
-// the chirp-z convolution length, and the device tables plans upload.
+// planner.cpp -- twiddle roots, tile lookup, the pass cost model and pass splits, and the device
+// tables plans upload.
 #include "plan_internal.h"
 
 #include <cstring>
@@ -273,42 +273,6 @@ bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsign
     if (c.empty()) return false;
     out = c[0];
     return true;
-}
-
-// Largest complex length the chirp-z path takes: its convolution length m < 2n must stay
-// within the multi-pass limit of the precision.
-unsigned long long bluestein_max_m(int prec) { return prec == PREC_F64 ? (1ull << 26) : (1ull << 28); }
-
-// Convolution length for the chirp-z path: the 2/3/5-smooth m >= 2n-1 (up to twice that)
-// with the lowest modelled cost, m times the sum over its passes of 1/bandwidth (a
-// single-pass tile counts as one pass at 4 TB/s).  0 when none can be planned.
-unsigned long long bluestein_length(int prec, unsigned long long n, unsigned long long batch)
-{
-    const unsigned long long lo = 2 * n - 1, hi = 2 * lo, maxm = bluestein_max_m(prec);
-    std::vector<unsigned long long> cand;
-    for (unsigned long long a = 1; a <= hi; a *= 2)
-        for (unsigned long long b = a; b <= hi; b *= 3)
-            for (unsigned long long c = b; c <= hi; c *= 5)
-                if (c >= lo && c <= maxm) cand.push_back(c);
-    std::sort(cand.begin(), cand.end());
-    unsigned long long best = 0;
-    double best_cost = 0;
-    for (unsigned long long m : cand) {
-        double per = 0;
-        if (m <= 16384 && find_tile(prec, (int)m, false, false) && !find_tile(prec, (int)m, false, false)->mix) {
-            per = 1.0 / 4.0;
-        } else {
-            const std::vector<std::vector<int>> c = candidate_passes(prec, m, 1, batch, 256, false);
-            if (c.empty()) continue;
-            for (int L : c[0]) per += 1.0 / pass_bandwidth(prec, L);
-        }
-        const double cost = per * (double)m;
-        if (!best || cost < best_cost) {
-            best = m;
-            best_cost = cost;
-        }
-    }
-    return best;
 }
 
 template <typename T> void pack_stage_table(int nrad, const int* radices, std::vector<T>& out)

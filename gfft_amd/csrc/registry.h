@@ -34,7 +34,8 @@ struct TileEntry {
 // Run-time mixed-radix tiles (mixed.hip).  mixed_prepare lifts the kernel's limit on dynamic
 // LDS; it is called once per shape, when a plan is made.
 hipError_t mixed_prepare(const TileEntry& k);
-hipError_t launch_mixed(const TileEntry& k, const TileArgs& a, dim3 grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1);
+hipError_t launch_mixed(const TileEntry& k, const TileArgs& a, dim3 grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1,
+                        const ChirpArgs* c = nullptr);
 
 inline hipError_t launch_entry(const TileEntry* k, const TileArgs& a, dim3 grid, hipStream_t s, hipEvent_t t0 = nullptr,
                                hipEvent_t t1 = nullptr)
@@ -73,7 +74,7 @@ struct SplitArgs {
 };
 hipError_t launch_split(int prec, const SplitArgs& a, hipStream_t s);
 
-// Chirp-z (Bluestein) path for lengths with a prime factor above 5 (bluestein.hip).
+// Tables of the chirp-z (Bluestein) path for lengths with a prime factor above 7 (bluestein.hip).
 struct ChirpTableArgs {
     void* chirp;            // n entries c_j = W_{2n}^{j^2}, working precision
     long long n;
@@ -81,20 +82,11 @@ struct ChirpTableArgs {
     const double2* hi;
     int shift;
 };
-struct BluesteinArgs {
-    const void* in;         // caller's input (pre), batch items `dist` apart
-    void* out;              // caller's output (post)
-    void* work;             // batch x m convolution buffer
-    const void* chirp;      // n entries
-    const void* filter;     // m entries: FFT_m of the chirp filter
-    long long n, m, dist, batch;
-    int conj;               // inverse transform: conjugate on input and on output
-    double scale;           // post: 1 or 1/n
-    const long long* boff;  // optional: element offset of every batch item (else b * dist)
-};
-enum { BLUESTEIN_PRE = 0, BLUESTEIN_MUL = 1, BLUESTEIN_POST = 2, BLUESTEIN_FILTER = 3 };
-hipError_t launch_bluestein(int prec, int which, const BluesteinArgs& a, hipStream_t s);
 hipError_t launch_chirp_table(int prec, const ChirpTableArgs& a, hipStream_t s);
+// b over length m: conj(c_j) at j < n and at m - j for 0 < j < n, zero elsewhere
+hipError_t launch_chirp_filter(int prec, const void* chirp, void* b, long long n, long long m, hipStream_t s);
+// filter[i] = spec[i] / m, from precision `from` to `to`
+hipError_t launch_chirp_spectrum(int from, int to, const void* spec, void* filter, long long m, hipStream_t s);
 
 // Digit reversal dst[rev(k)] = src[k] over radix^digits elements.
 hipError_t launch_digit_reverse(int prec, const void* src, void* dst, long long radix, int digits,

@@ -280,45 +280,50 @@ static std::vector<int> best_combination(const std::vector<int>& chosen, const s
 int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
                 uint32_t flags)
 {
-    int rc = create_plan_impl(out, n, batch, vtype, ttype, place, device, flags, {}, "");
-    if (rc != GFFTX_SUCCESS) return rc;
-    gfftx_plan_s* p = *out;
-    // a batched single-pass plan is tuned over the compiled tiles of its length (shape and
-    // radices), a multi-pass plan over pass splits and tile shapes
-    const bool single_pass = p->passes.size() == 1 && p->passes[0].k && p->passes[0].items_in_ntrans;
-    if ((p->passes.size() < 2 && !single_pass) || (flags & GFFTX_FLAG_NO_AUTOTUNE) ||
-        env_int("GFFTX_AUTOTUNE", 1) == 0 || getenv("GFFTX_PASSES"))
-        return GFFTX_SUCCESS;
     // a real plan is timed with the split fused into its last (forward) or first (inverse)
     // pass, and every candidate runs with the plan's own placement (one buffer or two), so
     // the choice is kept per transform kind and place; forward and inverse complex transforms
     // share it
-    const std::string key = tune_key(device, p->prec, n, batch) +
-                            (ttype == GFFTX_RDFT ? "|rdft" : ttype == GFFTX_IRDFT ? "|irdft" : "") +
-                            (place == GFFTX_IN_PLACE ? "|ip" : "|oop");
+    const bool tune = !(flags & (GFFTX_FLAG_NO_AUTOTUNE | GFFTX_FLAG_SPLIT_MFMA)) && env_int("GFFTX_AUTOTUNE", 1) != 0 &&
+                      !getenv("GFFTX_PASSES");
+    std::string key;
     std::vector<int> chosen;
     std::string note;
-    {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        tune_load();
-        auto it = g_tune.find(key);
-        if (it != g_tune.end()) {
-            chosen = it->second;
-            note = ",\"tuned\":\"cache\"";
+    if (tune) {
+        const int prec = (vtype == GFFTX_DOUBLE || vtype == GFFTX_COMPLEX_DOUBLE) ? PREC_F64 : PREC_F32;
+        key = tune_key(device, prec, n, batch) +
+              (ttype == GFFTX_RDFT ? "|rdft" : ttype == GFFTX_IRDFT ? "|irdft" : "") +
+              (place == GFFTX_IN_PLACE ? "|ip" : "|oop");
+        // a measured choice: the plan is built with it at once (a plan that cannot be built this
+        // way, or at all, is built by the cost model below, which says why not)
+        if (tune_get(key, &chosen)) {
+            if (create_plan_impl(out, n, batch, vtype, ttype, place, device, flags, chosen, ",\"tuned\":\"cache\"") ==
+                GFFTX_SUCCESS)
+                return GFFTX_SUCCESS;
+            return create_plan_impl(out, n, batch, vtype, ttype, place, device, flags, {}, "");
         }
     }
-    if (chosen.empty()) {
+    int rc = create_plan_impl(out, n, batch, vtype, ttype, place, device, flags, {}, "");
+    if (rc != GFFTX_SUCCESS) return rc;
+    gfftx_plan_s* p = *out;
+    // a batched single-pass plan is tuned over the tiles of its length (shape and radices), a
+    // multi-pass plan over pass splits and tile shapes
+    const bool single_pass = p->passes.size() == 1 && p->passes[0].k && p->passes[0].items_in_ntrans;
+    const bool chirp = p->blue_m != 0;  // convolution lengths, their splits and the passes' shapes
+    if (!tune || (p->passes.size() < 2 && !single_pass && !chirp)) return GFFTX_SUCCESS;
+    {
         std::vector<std::vector<int>> splits;
         // a single-pass plan is timed against pass splits where its workgroups leave most of
         // the device idle: no more than the CUs for a run-time tile, 8 (one per XCD) for a
         // compiled one of a complex transform, from 2048 points up
         const uint64_t tiles = single_pass ? (batch + p->passes[0].k->nb - 1) / p->passes[0].k->nb : 0;
         const uint64_t few = single_pass ? (p->passes[0].k->mix ? device_cus(device) : p->real ? 0 : 8) : 0;
-        if (!single_pass || (n >= 2048 && tiles <= few))
+        if (!chirp && (!single_pass || (n >= 2048 && tiles <= few)))
             splits = tuned_splits(p->prec, n, (size_t)env_int("GFFTX_TUNE_CANDIDATES", 5), batch, device_cus(device));
         std::vector<std::vector<int>> cands = split_variants(p->prec, n, batch, device_cus(device), splits);
         if (single_pass)
             for (const TileEntry* e : tile_shapes(p->prec, (int)n, false, false)) cands.push_back({(int)n, 1, 0, e->nb, e->wg});
+        if (chirp) cands = chirp_candidates(p->prec, n, batch, device_cus(device), 6);
         if (cands.size() < 2) return GFFTX_SUCCESS;
         DeviceGuard g(device);
         // the candidates run on at most 1 GiB of data (a larger batch is timed on a prefix of
@@ -376,7 +381,10 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             return ms;
         };
         for (size_t i = 0; i < cands.size(); ++i) cms[i] = try_cand(cands[i]);
-        if (!chosen.empty() && chosen[1] != 1) {
+        if (chirp && !chosen.empty()) {
+            for (size_t i = 0; i < 5; ++i)
+                for (const std::vector<int>& c : chirp_variants(p->prec, n, chosen, i)) try_cand(c);
+        } else if (!chosen.empty() && chosen[1] != 1) {
             const std::vector<int> combo = best_combination(chosen, cands, cms);
             if (!combo.empty()) try_cand(combo);
         }

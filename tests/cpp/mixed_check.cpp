@@ -14,8 +14,6 @@
 
 typedef std::complex<double> cd;
 
-static unsigned umulhi(unsigned a, unsigned b) { return (unsigned)(((unsigned long long)a * b) >> 32); }
-
 static int fails = 0;
 #define CHECK(c)                                                                                          \
     do {                                                                                                  \
@@ -33,15 +31,18 @@ static void check(const TileEntry& e)
     const MixShape& m = *e.mix;
     const unsigned L = m.L, tpt = m.tpt;
     CHECK((int)L == e.L && m.nb == (unsigned)e.nb && m.wg == (unsigned)e.wg && m.wg <= 1024 && m.wg % 64 == 0);
-    CHECK(m.nb * tpt <= m.wg && e.lds_bytes <= 160 * 1024);
+    CHECK(m.nb * tpt <= m.wg && e.lds_bytes <= 160 * 1024 && m.nst <= MIX_STAGES && m.nb * L < (1u << 15));
+    for (const Div& d : {m.dtpt, m.dr0, m.dl}) CHECK(d.m < (1u << 17));
+    for (unsigned x = 0; x < (1u << 15); x += 7) CHECK(m.dl(x) == x / L && m.dr0(x) == x / m.st[0].R);
     CHECK(m.nst == 1 || (size_t)e.lds_bytes == (size_t)m.nb * m.ts * (e.prec == PREC_F64 ? 16 : 8));
     CHECK(!e.loadT || (m.nb & (m.nb - 1)) == 0);
     CHECK(!(e.loadT || e.real) || m.nst >= 2);
+    CHECK((e.real != CHIRP_ALL && e.real != CHIRP_TURN) || m.st[0].R == m.st[m.nst - 1].R);
     if (!e.loadT)
         for (unsigned tid = 0; tid < m.wg; ++tid)
-            CHECK((tpt == 1 ? tid : umulhi(tid, m.mtpt)) == tid / tpt);
+            CHECK(m.dtpt(tid) == tid / tpt);
     if (e.loadT && !e.storeT)
-        for (unsigned lin = 0; lin < m.nb * L; ++lin) CHECK(umulhi(lin, m.ml) == lin / L);
+        for (unsigned lin = 0; lin < m.nb * L; ++lin) CHECK(m.dl(lin) == lin / L);
     std::vector<cd> in(L, 0), lds(m.ts), out(L);
     const unsigned at[3] = {0, L / 3, L - 1};
     for (int i = 0; i < 3; ++i) in[at[i]] += cd(1.0 + i, 0.5 * i);
@@ -60,7 +61,8 @@ static void check(const TileEntry& e)
                 if (j >= lr) continue;
                 CHECK(!done[j]);
                 done[j] = 1;
-                const unsigned p = j + m.pad * umulhi(j, m.mr0), q = s == 0 ? j : last ? 0 : umulhi(j, st.mns);
+                CHECK(m.dr0(j) == j / m.st[0].R && st.dns(j) == j / ns && j < (1u << 15));
+                const unsigned p = j + (m.dr0(j) & (0u - m.pad)), q = s == 0 ? j : last ? 0 : st.dns(j);
                 CHECK(q == j / ns);
                 const unsigned k = j - q * ns;
                 std::vector<cd> v(R), y(R);
@@ -83,7 +85,7 @@ static void check(const TileEntry& e)
                         out[j + r * lr] = y[r];
                     }
                     if (m.nst == 1) continue;
-                    const unsigned w = s == 0 ? j * (R + m.pad) + r : p + q * (R - 1) * st.wst + r * st.wst;
+                    const unsigned w = s == 0 ? j * (R + m.pad) + r : p + q * st.wq + r * st.wst;
                     CHECK(w < m.ts && !hit[w]);
                     const unsigned el = q * ns * R + k + r * ns;  // the Stockham rule
                     CHECK(w == el + m.pad * (el / m.st[0].R));
@@ -112,12 +114,14 @@ int main()
     for (int prec = 0; prec < 2; ++prec)
         for (int L = 2; L <= 16384; ++L) {
             bool any = false;
-            for (int mode = 0; mode < 5; ++mode) {
-                const bool loadT = mode == 1 || mode == 2, storeT = mode == 2;
-                const int real = mode == 3 ? REAL_POST : mode == 4 ? REAL_PRE : REAL_NONE;
-                if (mode >= 3 && L % 2) continue;
+            for (int mode = 0; mode < 9; ++mode) {
+                static const int kinds[9] = {REAL_NONE, REAL_NONE, REAL_NONE, REAL_POST, REAL_PRE,
+                                             CHIRP_ALL, CHIRP_IN, CHIRP_TURN, CHIRP_OUT};
+                const bool storeT = mode == 2 || mode == 8, loadT = storeT || mode == 1 || mode == 6 || mode == 7;
+                const int real = kinds[mode];
+                if ((real == REAL_POST || real == REAL_PRE) && L % 2) continue;
                 for (const TileEntry* e : mix_tiles(prec, L, loadT, storeT, real)) {
-                    if (mode < 3) check(*e);
+                    check(*e);
                     ++tiles;
                     any = true;
                 }
