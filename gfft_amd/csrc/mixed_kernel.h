@@ -164,18 +164,44 @@ template <typename T> struct MixCtx {
     unsigned ies, ons;
     long long tg;  // sequence within the batch item
     long long bo;  // element offset of the batch item in the output
+    double2 rw;    // FP32: root of the next stage's first butterfly, in flight (see fetch_roots, tile_kernel.h)
 };
+
+// Whether the roots are fetched one stage ahead.  Not in plain single passes: they run at the rate
+// of memory with six waves per SIMD, whose 80 registers have no room for it (16384 x 1000: 51 us
+// without, 56 us with it and five waves, 67 us with it and six, spilling).
+template <int MODE, int REAL> constexpr bool mix_ahead() { return MODE != MIX_EE || REAL != REAL_NONE; }
+
+template <typename T> __device__ __forceinline__ void mix_fetch(MixCtx<T>& c, const void* tw, const MixStage& st)
+{
+    if constexpr (sizeof(T) == 4) {
+        if (c.jt < st.lr) c.rw = reinterpret_cast<const double2*>(tw)[st.tw + c.jt - mul24(st.dns(c.jt), st.ns)];
+    }
+}
+
+// Stage s of the launch's shape, read from the kernel arguments where they lie (MixArgs is the only
+// argument): indexing the by-value struct at run time makes the compiler copy all of it to scratch
+// memory (616 bytes a thread; the chirp-z tile then ran three times as long).
+__device__ __forceinline__ MixStage mix_stage_args(unsigned s)
+{
+    typedef const __attribute__((address_space(4))) unsigned char* Bytes;
+    typedef const __attribute__((address_space(4))) MixStage* Stages;
+    const Bytes k = (Bytes)__builtin_amdgcn_kernarg_segment_ptr();
+    const Stages st = (Stages)(k + offsetof(MixArgs, m) + offsetof(MixShape, st)) + s;
+    return MixStage{st->R, st->lr, st->ns, Div{st->dns.m, st->dns.s}, st->rst, st->wst, st->wq, st->tw};
+}
 
 // LDS index of element e (pad is 0 or 1).
 __device__ __forceinline__ unsigned mix_pos(const MixShape& m, unsigned e) { return e + (m.dr0(e) & (0u - m.pad)); }
 
 // Twiddles W^{k r}, r = 1..R-1, of one butterfly.  FP32: FP64 powers of the FP64 root, rounded
 // once (as in tile_kernel.h); FP64: the table's rows, row r contiguous in k.
-template <typename T, int R> __device__ __forceinline__ void mix_twiddle(V2<T>* v, const void* tw, const MixStage& st, unsigned k)
+template <typename T, int R>
+__device__ __forceinline__ void mix_twiddle(V2<T>* v, const void* tw, const MixStage& st, unsigned k, const double2* root = nullptr)
 {
     using V = V2<T>;
     if constexpr (sizeof(T) == 4) {
-        const double2 w1 = reinterpret_cast<const double2*>(tw)[st.tw + k];
+        const double2 w1 = root ? *root : reinterpret_cast<const double2*>(tw)[st.tw + k];
         v[1] = cmul(v[1], to_v<V>(w1));
         if constexpr (R > 2) {
             const double2 w2 = dmul(w1, w1);
@@ -225,7 +251,15 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
     const unsigned lr = x.m.st[0].lr, tpt = x.m.tpt;
     const unsigned cn = x.c.n, e0 = REAL == CHIRP_IN ? (unsigned)c.tg : 0u;  // chirp-z: element e0 + i
     const unsigned istep = MODE == MIX_EE ? lr : lr * c.ies;  // between the elements of a butterfly
+    // chirp-z: n <= (m + 1) / 2, so the elements r lr + j with 2 r >= R lie in the zero padding
+    constexpr int RN = REAL == CHIRP_ALL || REAL == CHIRP_IN ? (R + 1) / 2 : R;
     V v[B][R];
+    if constexpr (RN < R) {
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+#pragma unroll
+            for (int r = RN; r < R; ++r) v[b][r] = V{0, 0};
+    }
     with_nt(x.m.nt_in != 0, [&](auto ntc) {
 #pragma unroll
         for (int b = 0; b < B; ++b) {
@@ -233,7 +267,7 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
             if (j >= lr) continue;
             const unsigned i0 = MODE == MIX_EE ? j : j * c.ies;
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
+            for (int r = 0; r < RN; ++r) {
                 const unsigned i = i0 + r * istep;
                 const V* p = &c.in[i];
                 if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_IN) {
@@ -245,6 +279,7 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
             }
         }
     });
+    if constexpr (!ONLY && mix_ahead<MODE, REAL>()) mix_fetch(c, a.tw, mix_stage_args(1));
     if constexpr (REAL == REAL_PRE) {
         // Z[e] from X[e] and X[N - e] of the same sequence (see pre_split, tile_kernel.h); the
         // exchange uses a plain layout, element e at e
@@ -298,12 +333,13 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
         const unsigned j = c.jt + b * tpt;
         if (j >= lr) continue;
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[b][r] = flip_im(v[b][r], flip);
+        for (int r = 0; r < RN; ++r)
+            if (flip) v[b][r].y = -v[b][r].y;
         if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_IN) {
             const V* ch = reinterpret_cast<const V*>(x.c.chirp) + e0;
             const unsigned i0 = MODE == MIX_EE ? j : j * c.ies;
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
+            for (int r = 0; r < RN; ++r) {
                 const unsigned i = i0 + r * istep;
                 if (e0 + i < cn) v[b][r] = cmul(v[b][r], ch[i]);
             }
@@ -351,7 +387,7 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
 // A later stage: LDS to registers, twiddles, butterfly, and back to the LDS or, after the last
 // stage of a mode whose stores match its lanes, to the output.
 template <typename T, int MODE, int REAL, int R, bool LAST>
-__device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const MixStage& st)
+__device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const MixStage& st, const MixStage& next)
 {
     using V = V2<T>;
     constexpr int B = mix_b<R>();
@@ -369,11 +405,15 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
 #pragma unroll
         for (int r = 0; r < R; ++r, rd += rst) v[b][r] = *rd;
     }
+    const double2 w1 = c.rw;
+    if constexpr (!LAST && mix_ahead<MODE, REAL>()) mix_fetch(c, a.tw, next);  // (by every thread: it may take part in the next stage alone)
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const unsigned j = c.jt + b * tpt;
         if (j < lr) {
-            mix_twiddle<T, R>(v[b], a.tw, st, j - mul24(quot(j), st.ns));
+            const unsigned k = j - mul24(quot(j), st.ns);
+            if (mix_ahead<MODE, REAL>() && b == 0) mix_twiddle<T, R>(v[b], a.tw, st, k, &w1);
+            else mix_twiddle<T, R>(v[b], a.tw, st, k);
             Dft<R>::run(v[b]);
         }
         __builtin_amdgcn_sched_barrier(0);  // one butterfly's twiddles at a time (registers)
@@ -382,7 +422,16 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
         const unsigned fo = a.conj_out ? 0x80000000u : 0u;
         const T sc = (T)a.scale;
         const bool one = a.scale == 1.0;
+        constexpr int RN = REAL == CHIRP_ALL || REAL == CHIRP_OUT ? (R + 1) / 2 : R;  // the others are k >= n
         const V* chirp = reinterpret_cast<const V*>(x.c.chirp);  // (copies: the lambda would take x's address)
+        if constexpr (REAL != CHIRP_ALL && REAL != CHIRP_OUT) {
+            if (a.conj_out || !one) {  // inverse transforms
+#pragma unroll
+                for (int b = 0; b < B; ++b)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) v[b][r] = flip_im(cscale(v[b][r], sc), fo);
+            }
+        }
         const unsigned cn = x.c.n, ostep = MODE == MIX_EE ? lr : lr * c.ons;
         with_nt(a.nt_out != 0, [&](auto ntc) {
 #pragma unroll
@@ -391,7 +440,7 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
                 if (j >= lr) continue;
                 const unsigned i0 = MODE == MIX_EE ? j : j * c.ons;
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
+                for (int r = 0; r < RN; ++r) {
                     const unsigned i = i0 + r * ostep;
                     if constexpr (REAL == CHIRP_ALL || REAL == CHIRP_OUT) {
                         const unsigned k = (REAL == CHIRP_OUT ? (unsigned)c.tg : 0u) + i;
@@ -400,7 +449,7 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
                             put<decltype(ntc)::value>(&c.out[i], flip_im(one ? u : cscale(u, sc), fo));
                         }
                     } else {
-                        put<decltype(ntc)::value>(&c.out[i], flip_im(one ? v[b][r] : cscale(v[b][r], sc), fo));
+                        put<decltype(ntc)::value>(&c.out[i], v[b][r]);
                     }
                 }
             }
@@ -436,13 +485,16 @@ __device__ __forceinline__ void mix_turn(const MixArgs& x, MixCtx<T>& c, const M
 #pragma unroll
         for (int r = 0; r < R; ++r, rd += rst) v[b][r] = *rd;
     }
+    const double2 w1 = c.rw;
+    mix_fetch(c, x.a.tw, mix_stage_args(1));  // the backward transform's second stage
     const unsigned istep = REAL == CHIRP_TURN ? lr * c.ies : lr;
     const V* filter = reinterpret_cast<const V*>(x.c.filter) + (REAL == CHIRP_TURN ? (unsigned)c.tg : 0u);
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const unsigned j = c.jt + b * tpt;
         if (j < lr) {
-            mix_twiddle<T, R>(v[b], x.a.tw, st, j);
+            if (b == 0) mix_twiddle<T, R>(v[b], x.a.tw, st, j, &w1);
+            else mix_twiddle<T, R>(v[b], x.a.tw, st, j);
             Dft<R>::run(v[b]);
             const unsigned i0 = REAL == CHIRP_TURN ? j * c.ies : j;
 #pragma unroll
@@ -526,26 +578,16 @@ template <typename T> __device__ __forceinline__ void mix_split(const MixArgs& x
     }
 }
 
-// Stage s of the launch's shape, read from the kernel arguments where they lie (MixArgs is the only
-// argument): indexing the by-value struct at run time makes the compiler copy all of it to scratch
-// memory (616 bytes a thread; the chirp-z tile then ran three times as long).
-__device__ __forceinline__ MixStage mix_stage_args(unsigned s)
-{
-    typedef const __attribute__((address_space(4))) unsigned char* Bytes;
-    typedef const __attribute__((address_space(4))) MixStage* Stages;
-    const Bytes k = (Bytes)__builtin_amdgcn_kernarg_segment_ptr();
-    const Stages st = (Stages)(k + offsetof(MixArgs, m) + offsetof(MixShape, st)) + s;
-    return MixStage{st->R, st->lr, st->ns, Div{st->dns.m, st->dns.s}, st->rst, st->wst, st->wq, st->tw};
-}
-
 // The stages between the first and the last one.
 template <typename T, int MODE, int REAL> __device__ __forceinline__ void mix_middle(const MixArgs& x, MixCtx<T>& c)
 {
+    MixStage next = mix_stage_args(1);
     for (unsigned s = 1; s + 1 < x.m.nst; ++s) {
-        const MixStage st = mix_stage_args(s);
+        const MixStage st = next;
+        next = mix_stage_args(s + 1);
         switch (st.R) {
 #define X(R_) \
-    case R_: mix_stage<T, MODE, REAL, R_, false>(x, c, st); break;
+    case R_: mix_stage<T, MODE, REAL, R_, false>(x, c, st, next); break;
             GFFTX_MIX_RADICES(X)
 #undef X
             default: break;
@@ -553,8 +595,13 @@ template <typename T, int MODE, int REAL> __device__ __forceinline__ void mix_mi
     }
 }
 
+// Waves per SIMD the registers are allotted for (128, 96 or 80 of them).
+template <typename T, int MODE, int REAL> struct MixWaves {
+    static constexpr int value = sizeof(T) == 8 ? 4 : mix_ahead<MODE, REAL>() ? 5 : 6;
+};
+
 template <typename T, int MODE, int REAL>
-__global__ __launch_bounds__(1024, sizeof(T) == 8 ? 4 : MODE == MIX_EE && REAL != REAL_PRE ? 6 : 5) void mixed_kernel(MixArgs x)
+__global__ __launch_bounds__(1024, (MixWaves<T, MODE, REAL>::value)) void mixed_kernel(MixArgs x)
 {
     using V = V2<T>;
     extern __shared__ __align__(16) unsigned char mix_lds[];
@@ -625,7 +672,7 @@ __global__ __launch_bounds__(1024, sizeof(T) == 8 ? 4 : MODE == MIX_EE && REAL !
     }
     switch (sl.R) {
 #define X(R_) \
-    case R_: mix_stage<T, MODE, REAL, R_, true>(x, c, sl); break;
+    case R_: mix_stage<T, MODE, REAL, R_, true>(x, c, sl, sl); break;
         GFFTX_MIX_RADICES(X)
 #undef X
         default: break;

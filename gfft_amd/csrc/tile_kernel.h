@@ -107,6 +107,15 @@ struct TileCfg {
         for (int i = 1; i < s; ++i) o += ns(i);
         return o;
     }
+    static constexpr int most_roots()
+    {
+        int m = 1;
+        for (int i = 1; i < NS; ++i) m = ahead(i) && nbf(i) > m ? nbf(i) : m;
+        return m;
+    }
+    // stages whose roots are fetched one stage ahead: at most 16 registers of them
+    static constexpr bool ahead(int s) { return TW_POW && s > 0 && s < NS && nbf(s) <= 4; }
+    static constexpr int ROOTS = TW_POW ? most_roots() : 1;
     static constexpr int TW_ROOT_OFF = (twoff(NS) * (int)sizeof(V2<T_>) + 15) / 16 * 16;  // bytes
     // LDS: one padded element every 16, odd distance between sequences (bank spread).
     static constexpr int LP = L + L / 16;
@@ -184,8 +193,22 @@ template <class C> struct Ctx {
     bool valid;          // sequence exists (loads are clamped to a valid one regardless)
     bool active;         // thread takes part (threads beyond C::WG idle through the barriers)
     long long bo;        // element offset of the batch item
+    double2 rw[C::ROOTS];  // FP64 roots of the next stage's butterflies (TW_POW tiles), in flight
     TileArgs a;
 };
+
+// Issues the loads of stage S's roots.  They are asked for one stage ahead (with the inputs for
+// the second stage) and need nothing but the thread's index, so their trip to the L2 runs under
+// the butterflies and the barrier before the stage instead of after it: a pass of a transform of
+// a few MB is one wave of workgroups, and each trip was on its critical path.
+template <class C, int S> __device__ __forceinline__ void fetch_roots(Ctx<C>& x)
+{
+    if constexpr (C::ahead(S)) {
+        const double2* roots = reinterpret_cast<const double2*>(reinterpret_cast<const char*>(x.tw) + C::TW_ROOT_OFF) + C::twbase(S);
+#pragma unroll
+        for (int b = 0; b < C::nbf(S); ++b) x.rw[b] = roots[(x.jt + b * C::TPT) % C::ns(S)];
+    }
+}
 
 template <typename V> __device__ __forceinline__ V to_v(double2 w);
 template <> __device__ __forceinline__ float2 to_v<float2>(double2 w) { return float2{(float)w.x, (float)w.y}; }
@@ -249,6 +272,10 @@ template <class C> struct FirstIn {
     double2 blo[C::nbf(0)], bhi[C::nbf(0)];
     double2 slo, shi;
     bool rot;
+    // C2R pre-pass (REAL_PRE): the table halves of W_{2N}^e at each group's first element and of
+    // the step between a group's elements, fetched with the inputs: looked up behind the LDS
+    // exchange they added a trip to the L2 to the critical path of a pass of one wave of tiles
+    double2 pelo[C::REAL == REAL_PRE ? C::nbf(0) : 1], pehi[C::REAL == REAL_PRE ? C::nbf(0) : 1], pslo, pshi;
 };
 
 // The input of a pass is dead once read (a scratch array, or the caller's input that the
@@ -258,7 +285,7 @@ template <class C> struct FirstIn {
 // 128-byte lines (T mode: NB adjacent sequences per row; E mode: NB whole sequences), so
 // that no other tile needs a line this one evicts early; a row of, say, 21 sequences
 // (168 bytes) shares its end lines with the neighbouring tiles.
-template <class C, bool IDLE> __device__ __forceinline__ void load_first(const Ctx<C>& x, FirstIn<C>& f)
+template <class C, bool IDLE> __device__ __forceinline__ void load_first(Ctx<C>& x, FirstIn<C>& f)
 {
     using V = typename C::V;
     constexpr int R = C::R[0];
@@ -276,7 +303,22 @@ template <class C, bool IDLE> __device__ __forceinline__ void load_first(const C
             f.v[b][r] = NT ? nt_load(p) : *p;
         }
     }
+    fetch_roots<C, 1>(x);
     const TileArgs& a = x.a;
+    if constexpr (C::REAL == REAL_PRE) {
+        const long long e0 = C::PAIRED ? (x.valid ? x.tg : 0) : 0, es = C::PAIRED ? a.ntrans : 1;
+        const long long mask = (1LL << a.sp_shift) - 1, rst = (long long)LR * es;
+        f.pslo = a.sp_lo[rst & mask];
+        f.pshi = a.sp_hi[rst >> a.sp_shift];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int j = x.jt + b * C::TPT;
+            if ((IDLE && !x.active) || (GUARD && j >= LR)) continue;
+            const long long eb = e0 + (long long)j * es;
+            f.pelo[b] = a.sp_lo[eb & mask];
+            f.pehi[b] = a.sp_hi[eb >> a.sp_shift];
+        }
+    }
     f.rot = false;
     if (a.ptw_lo != nullptr) {
         const long long kp = x.tg % a.ns_pass;
@@ -306,6 +348,12 @@ template <class C, bool IDLE, int S> __device__ __forceinline__ void tile_stage(
     constexpr bool LAST = (S == C::NS - 1);
     constexpr bool GUARD = (B * C::TPT > LR);
     V v[B][R];
+    double2 w1s[B];
+    if constexpr (C::ahead(S)) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) w1s[b] = x.rw[b];
+    }
+    if constexpr (!FIRST) fetch_roots<C, S + 1>(x);
 
 #pragma unroll
     for (int b = 0; b < B; ++b) {
@@ -331,9 +379,12 @@ template <class C, bool IDLE, int S> __device__ __forceinline__ void tile_stage(
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b][r] = x.lds[C::lidx(x.t, j + r * LR)];
             const int k = j % NSS;
+            (void)k;
             if constexpr (C::TW_POW) {
-                const double2 w1 = reinterpret_cast<const double2*>(reinterpret_cast<const char*>(x.tw) +
-                                                                    C::TW_ROOT_OFF)[C::twbase(S) + k];
+                if constexpr (!C::ahead(S))
+                    w1s[b] = reinterpret_cast<const double2*>(reinterpret_cast<const char*>(x.tw) +
+                                                              C::TW_ROOT_OFF)[C::twbase(S) + k];
+                const double2 w1 = w1s[b];
                 if constexpr (R >= 8 && R % 4 == 0) {
                     // W^{k (4a + c)} = (W^{4k})^a W^{k c}: short dependency chains (the
                     // stage's latency); each twiddle is at most five FP64 products from the
@@ -726,15 +777,14 @@ template <class C, bool IDLE> __device__ __forceinline__ void pre_split(const Ct
             e0 = x.tg;
             es = a.ntrans;
         }
-        const long long mask = (1LL << a.sp_shift) - 1;
         const long long rst = (long long)LR * es;  // e steps by LR S between a thread's r
-        const double2 step = dmul(a.sp_lo[rst & mask], a.sp_hi[rst >> a.sp_shift]);
+        const double2 step = dmul(f.pslo, f.pshi);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const int j = x.jt + b * C::TPT;
             if (GUARD && j >= LR) continue;
             const long long eb = e0 + (long long)j * es;
-            double2 w = dmul(a.sp_lo[eb & mask], a.sp_hi[eb >> a.sp_shift]);
+            double2 w = dmul(f.pelo[b], f.pehi[b]);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int q = j + r * LR;

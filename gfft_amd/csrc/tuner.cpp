@@ -165,10 +165,18 @@ std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 // `reps` executions issued back to back between two events, the median of the group means.
 // Back-to-back calls are what a batch loop issues; a call timed alone after a synchronisation
 // also carries the start of an idle device.
-int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float* ms_out)
+// The calls walk over `sets` pairs of arrays, `stride` bytes apart, as a program's successive
+// inputs do: on one pair a transform of a few MB runs from the L2 caches, and the choice between
+// two splits can come out the other way.
+int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float* ms_out, int sets = 1, size_t stride = 0)
 {
+    int call = 0;
+    auto exec = [&]() {
+        const size_t off = (size_t)(call++ % sets) * stride;
+        return exec_device(p, (char*)a + off, (char*)b + off, s);
+    };
     for (int i = 0; i < 2; ++i) {
-        int rc = exec_device(p, a, b, s);
+        int rc = exec();
         if (rc) return rc;
     }
     std::vector<float> t;
@@ -181,7 +189,7 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
     for (int g = 0; g < 3; ++g) {
         (void)hipEventRecord(e0, s);
         int rc = GFFTX_SUCCESS;
-        for (int i = 0; i < reps && !rc; ++i) rc = exec_device(p, a, b, s);
+        for (int i = 0; i < reps && !rc; ++i) rc = exec();
         (void)hipEventRecord(e1, s);
         (void)hipEventSynchronize(e1);
         if (rc) {
@@ -320,6 +328,12 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         const uint64_t few = single_pass ? (p->passes[0].k->mix ? device_cus(device) : p->real ? 0 : 8) : 0;
         if (!chirp && (!single_pass || (n >= 2048 && tiles <= few)))
             splits = tuned_splits(p->prec, n, (size_t)env_int("GFFTX_TUNE_CANDIDATES", 5), batch, device_cus(device));
+        // an inverse real transform's first pass carries the C2R pre-split, which halves the runs of
+        // its rows: its two-pass splits are timed in the other order too
+        if (p->real && p->inverse)
+            for (size_t i = splits.size(); i-- > 0;)
+                if (splits[i].size() == 2 && splits[i][0] != splits[i][1] && find_tile(p->prec, splits[i][1], true, false))
+                    splits.push_back({splits[i][1], splits[i][0]});
         std::vector<std::vector<int>> cands = split_variants(p->prec, n, batch, device_cus(device), splits);
         if (single_pass)
             for (const TileEntry* e : tile_shapes(p->prec, (int)n, false, false)) cands.push_back({(int)n, 1, 0, e->nb, e->wg});
@@ -331,20 +345,22 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         // the 256 MB Infinity Cache, so the timings see HBM as the plan will
         const size_t item_bytes = (size_t)p->dist * elem_bytes(p->prec);
         const uint64_t tbatch = std::min<uint64_t>(batch, std::max<uint64_t>(1, (1ull << 30) / item_bytes));
-        const size_t bytes = item_bytes * tbatch;
+        const size_t bytes = (item_bytes * tbatch + 255) / 256 * 256;
+        const int sets = bytes <= (64u << 20) ? 3 : 1;
         void *a = nullptr, *b = nullptr;
-        if (hipMalloc(&a, bytes) != hipSuccess || hipMalloc(&b, bytes) != hipSuccess) {
+        if (hipMalloc(&a, bytes * sets) != hipSuccess || hipMalloc(&b, bytes * sets) != hipSuccess) {
             (void)hipGetLastError();
             if (a) (void)hipFree(a);
             return GFFTX_SUCCESS;  // no room to tune: keep the cost-model plan
         }
         hipStream_t s = nullptr;
         (void)hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-        (void)hipMemsetAsync(a, 0, bytes, s);
+        (void)hipMemsetAsync(a, 0, bytes * sets, s);
         float best = 1e30f;
         std::string timings = ",\"tuned\":[";
         size_t ntimed = 0;
         std::vector<float> cms(cands.size(), -1.f);  // time of each candidate (-1: failed)
+        std::vector<std::pair<float, std::vector<int>>> timed;
         // time one candidate, record it in `timings`, keep it if it is the fastest so far
         auto try_cand = [&](const std::vector<int>& c) -> float {
             gfftx_plan cp = nullptr;
@@ -356,7 +372,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
                 GFFTX_SUCCESS)
                 return -1.f;
             float ms = 0;
-            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms);
+            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms, sets, bytes);
             gfftx_plan_destroy(cp);
             if (trc) return -1.f;
             std::vector<int> sl;
@@ -378,6 +394,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
                 best = ms;
                 chosen = c;
             }
+            timed.push_back({ms, c});
             return ms;
         };
         for (size_t i = 0; i < cands.size(); ++i) cms[i] = try_cand(cands[i]);
@@ -387,6 +404,26 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         } else if (!chosen.empty() && chosen[1] != 1) {
             const std::vector<int> combo = best_combination(chosen, cands, cms);
             if (!combo.empty()) try_cand(combo);
+        }
+        // the fastest few once more, in turn, on plans that stay: a single timing of a short transform
+        // moves by more than the candidates differ
+        std::vector<std::pair<float, std::vector<int>>> top = timed;
+        std::stable_sort(top.begin(), top.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+        top.resize(std::min<size_t>(top.size(), bytes <= (64u << 20) ? 4 : 2));
+        if (top.size() > 1) {
+            std::vector<gfftx_plan> tp(top.size(), nullptr);
+            std::vector<float> tms(top.size(), 1e30f);
+            for (size_t i = 0; i < top.size(); ++i)
+                (void)create_plan_impl(&tp[i], n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, top[i].second, "");
+            for (int rep = 0; rep < 3; ++rep)
+                for (size_t i = 0; i < top.size(); ++i) {
+                    float ms = 0;
+                    if (tp[i] && time_plan(tp[i], a, place == GFFTX_IN_PLACE ? a : b, s, 10, &ms, sets, bytes) == GFFTX_SUCCESS)
+                        tms[i] = std::min(tms[i], ms);
+                }
+            const size_t w = std::min_element(tms.begin(), tms.end()) - tms.begin();
+            if (tms[w] < 1e30f) chosen = top[w].second;
+            for (gfftx_plan q : tp) gfftx_plan_destroy(q);
         }
         timings += "]";
         (void)hipStreamSynchronize(s);
