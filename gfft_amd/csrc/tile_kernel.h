@@ -171,7 +171,7 @@ template <class Base, int KIND> struct RealCfg : Base {
 template <class Base> using SplitCfg = RealCfg<Base, REAL_POST>;
 
 // Sequence of lane t in tile `tile` under the split pairing (PAIRED tiles), or -1 for none.
-template <class C> __device__ __forceinline__ long long split_seq(long long S, unsigned tile, int t)
+template <class C> __host__ __device__ __forceinline__ long long split_seq(long long S, unsigned tile, int t)
 {
     constexpr int H = C::NB / 2;
     if (tile == 0) return t == 0 ? 0 : (t == 1 && S % 2 == 0 && S > 1) ? S / 2 : -1;
@@ -179,6 +179,10 @@ template <class C> __device__ __forceinline__ long long split_seq(long long S, u
     if (p > (S - 1) / 2) return -1;
     return t < H ? p : S - p;
 }
+
+// Exponent factor kp of a sequence's pass twiddles W_M^{kp e}.  0 for a lane without a sequence
+// (split_seq's -1): its remainder would be negative, and so would the table index made from it.
+__host__ __device__ __forceinline__ long long pass_phase(bool valid, long long tg, long long ns) { return valid ? tg % ns : 0; }
 
 template <class C> struct Ctx {
     using V = typename C::V;
@@ -321,7 +325,7 @@ template <class C, bool IDLE> __device__ __forceinline__ void load_first(Ctx<C>&
     }
     f.rot = false;
     if (a.ptw_lo != nullptr) {
-        const long long kp = x.tg % a.ns_pass;
+        const long long kp = pass_phase(x.valid, x.tg, a.ns_pass);
         f.rot = kp != 0;
         if (f.rot) {
             const long long mask = (1LL << a.ptw_shift) - 1;
