@@ -370,13 +370,13 @@ __device__ __forceinline__ void mix_first(const MixArgs& x, MixCtx<T>& c)
         // a length that is one butterfly: straight to the output
         const unsigned fo = a.conj_out ? 0x80000000u : 0u;
         const T sc = (T)a.scale;
-        with_nt(a.nt_out != 0, [&](auto ntc) {
+        with_store<MODE != MIX_EE>(a.store, [&](auto kind) {
 #pragma unroll
             for (int b = 0; b < B; ++b) {
                 if (c.jt + b * tpt >= lr) continue;
 #pragma unroll
                 for (int r = 0; r < R; ++r)
-                    put<decltype(ntc)::value>(&c.out[r * c.ons], flip_im(a.scale == 1.0 ? v[b][r] : cscale(v[b][r], sc), fo));
+                    put<decltype(kind)::value>(&c.out[r * c.ons], flip_im(a.scale == 1.0 ? v[b][r] : cscale(v[b][r], sc), fo));
             }
         });
     } else {
@@ -433,7 +433,7 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
             }
         }
         const unsigned cn = x.c.n, ostep = MODE == MIX_EE ? lr : lr * c.ons;
-        with_nt(a.nt_out != 0, [&](auto ntc) {
+        with_store<MODE != MIX_EE>(a.store, [&](auto kind) {
 #pragma unroll
             for (int b = 0; b < B; ++b) {
                 const unsigned j = c.jt + b * tpt;
@@ -446,10 +446,10 @@ __device__ __forceinline__ void mix_stage(const MixArgs& x, MixCtx<T>& c, const 
                         const unsigned k = (REAL == CHIRP_OUT ? (unsigned)c.tg : 0u) + i;
                         if (k < cn) {
                             const V u = cmul(chirp[k], V{v[b][r].x, -v[b][r].y});
-                            put<decltype(ntc)::value>(&c.out[i], flip_im(one ? u : cscale(u, sc), fo));
+                            put<decltype(kind)::value>(&c.out[i], flip_im(one ? u : cscale(u, sc), fo));
                         }
                     } else {
-                        put<decltype(ntc)::value>(&c.out[i], v[b][r]);
+                        put<decltype(kind)::value>(&c.out[i], v[b][r]);
                     }
                 }
             }
@@ -532,12 +532,12 @@ template <typename T> __device__ __forceinline__ void mix_finish_te(const MixArg
     const unsigned fo = a.conj_out ? 0x80000000u : 0u;
     const T sc = (T)a.scale;
     const bool one = a.scale == 1.0;
-    with_nt(a.nt_out != 0, [&](auto ntc) {
+    with_store<true>(a.store, [&](auto kind) {
 #pragma unroll 4
         for (unsigned lin = threadIdx.x; lin < total; lin += x.m.wg) {
             const unsigned t = x.m.dl(lin), q = lin - mul24(t, L);
             const V u = lds[mul24(t, x.m.ts) + mix_pos(x.m, q)];
-            put<decltype(ntc)::value>(&o[lin], flip_im(one ? u : cscale(u, sc), fo));
+            put<decltype(kind)::value>(&o[lin], flip_im(one ? u : cscale(u, sc), fo));
         }
     });
 }

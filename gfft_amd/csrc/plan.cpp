@@ -38,6 +38,29 @@ bool nt_output(size_t bytes)
     return mib >= 0 && bytes > (size_t)mib << 20;
 }
 
+// How pass `ps`, number i of m, stores its `bytes` of output (STORE_*, tile_kernel.h).  Through the L2
+// from 2 MiB (below, the shorter way of a plain store counts more: 59049 FP64, 0.9 MiB, 12.2 us plain,
+// 12.7 through) to 64 MiB (2^23 FP32, 74.0 us plain, 69.4 through; 2^20 x 16 FP32, 128 MiB, 143-147
+// plain, 148 through) where the tile writes whole 128-byte lines.  Parts of lines are written by
+// themselves, so with them the gain ends at 16 MiB (2^20 FP32 in rows of 32 bytes 17.4 -> 15.9 us,
+// but 823543 x 5 FP32, 31 MiB, 49.5 -> 51.9 and 3000000 FP64, 46 MiB, 67.8 -> 74.2), and the R2C
+// split, whose rows are half as long and begin anywhere, gains with long ones alone (3 * 2^20 reals
+// FP32: rows of 256 bytes 32.4 -> 24.9 us, of 16 bytes 27.9 -> 33.1).  GFFTX_THROUGH_STORE=0: never.
+int pass_store(bool nt, size_t i, size_t m, size_t bytes, const Pass& ps, size_t dist, size_t items)
+{
+    if (nt && i + 1 == m) return STORE_NT;
+    if (m < 2 || bytes < (size_t)2 << 20 || env_int("GFFTX_THROUGH_STORE", 1) == 0) return STORE_PLAIN;
+    const TileEntry& k = *ps.k;
+    const size_t eb = elem_bytes(k.prec);
+    auto lines = [&](size_t elems) { return elems * eb % 128 == 0; };
+    size_t mib;
+    if (k.real == REAL_POST) mib = (size_t)k.nb / 2 * eb >= 256 ? 25 : 0;
+    else if (items > 1 && !lines(dist)) mib = 16;
+    else if (k.storeT) mib = lines(k.nb) && lines(ps.ns_pass) ? 64 : 16;
+    else mib = lines(k.real == REAL_PRE ? k.L : k.nb * k.L) ? 64 : 16;
+    return bytes <= mib << 20 ? STORE_THROUGH : STORE_PLAIN;
+}
+
 int dev_alloc(gfftx_plan_s* p, void** out, size_t bytes)
 {
     if (bytes == 0) bytes = 16;
@@ -321,7 +344,7 @@ int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range 
         a.conj_out = (p->inverse && i == m - 1) ? 1 : 0;
         a.scale = (p->inverse && i == m - 1) ? 1.0 / (double)p->n : 1.0;
         a.xcd = ps.xcd;
-        a.nt_out = (r.nt && i == m - 1) ? 1 : 0;
+        a.store = pass_store(r.nt, i, m, (size_t)p->dist * r.nb * elem_bytes(p->prec), ps, p->dist, r.nb);
         const long long nb = ps.k->nb;
         unsigned ntiles = (unsigned)((a.ntrans + nb - 1) / nb);
         if (ps.real) {

@@ -79,6 +79,9 @@ struct Range {
 // Cache (GFFTX_NT_STORE_MIB, default 256; negative: never).
 bool nt_output(size_t bytes);
 
+// How pass `ps`, number i of m, stores its `bytes` of output: `items` batch items, `dist` elements apart.
+int pass_store(bool nt, size_t i, size_t m, size_t bytes, const Pass& ps, size_t dist, size_t items);
+
 inline size_t elem_bytes(int prec) { return prec == PREC_F64 ? 16 : 8; }
 
 // --- mixed_plan.cpp: run-time mixed-radix tiles

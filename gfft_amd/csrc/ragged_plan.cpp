@@ -139,7 +139,7 @@ int ragged_run_long(gfftx_ragged_s* r, const gfftx_ragged_s::LongClass& lc, void
         a.conj_in = (r->inverse && i == 0) ? 1 : 0;
         a.conj_out = (r->inverse && i == m - 1) ? 1 : 0;
         a.scale = (r->inverse && i == m - 1) ? 1.0 / (double)lc.L : 1.0;
-        a.nt_out = (i + 1 == m) ? r->args.nt_out : 0;
+        a.store = i + 1 == m && r->args.nt_out ? STORE_NT : STORE_PLAIN;
         dim3 grid;
         if (ps.items_in_ntrans) {
             a.ntrans = lc.count;

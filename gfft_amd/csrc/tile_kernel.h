@@ -52,7 +52,7 @@ struct TileArgs {
     int sp_shift;
     int split_bins;            // 1: N+1 bins, 0: NR packing
     long long nfull;           // N, the complex length of the transform
-    int nt_out;                // 1: the output is stored non-temporally (see put())
+    int store;                 // how the output is stored (STORE_*, see put())
 };
 
 __device__ __forceinline__ long long batch_offset(const TileArgs& a, unsigned by)
@@ -232,15 +232,32 @@ template <class V> __device__ __forceinline__ V nt_load(const V* p)
     return V{r.x, r.y};
 }
 
-// Store of one complex element of a launch's output: non-temporal when `nt` (the host sets it
-// for the last pass of a call whose output is larger than the 256 MB Infinity Cache and is
-// not read back by the call: caching those lines would only evict what the next loads need).
-template <bool NT, class V> __device__ __forceinline__ void put(V* p, V v)
+// How a launch stores its output (the host chooses):
+//   STORE_NT       non-temporally: the last pass of a call whose output is larger than the 256 MB
+//                  Infinity Cache and is not read back by the call: caching those lines would
+//                  only evict what the next loads need;
+//   STORE_THROUGH  through the L2 (agent scope): a pass of a multi-pass transform.  The eight
+//                  XCDs' L2 caches are written back where a kernel ends, and a pass of a few MB
+//                  ends with nearly all of its output there, so the next pass waited for that.
+//                  Written through, the lines leave while the tiles still run.
+enum { STORE_PLAIN = 0, STORE_NT = 1, STORE_THROUGH = 2 };
+
+// Store of one complex element of a launch's output.
+template <int KIND, class V> __device__ __forceinline__ void put(V* p, V v)
 {
-    if constexpr (NT) {
+    if constexpr (KIND == STORE_NT) {
         using E = decltype(V{}.x);
         typedef E vec __attribute__((ext_vector_type(2)));
         __builtin_nontemporal_store(vec{v.x, v.y}, reinterpret_cast<vec*>(p));
+    } else if constexpr (KIND == STORE_THROUGH && sizeof(V) == 8) {
+        // (no memory clobber: nothing in the kernel reads the output, and the LDS reads of the
+        // next elements may issue ahead of the store)
+        asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(p), "v"(__builtin_bit_cast(unsigned long long, v)));
+    } else if constexpr (KIND == STORE_THROUGH) {
+        typedef unsigned vec __attribute__((ext_vector_type(4)));
+        // (a store of more than 64 bits reads its data late: two wait states before a VALU write to
+        // those registers, which the compiler does not insert behind inline code)
+        asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(__builtin_bit_cast(vec, v)));
     } else {
         *p = v;
     }
@@ -248,7 +265,15 @@ template <bool NT, class V> __device__ __forceinline__ void put(V* p, V v)
 
 // Runs f with the store kind as a compile-time constant, so that each store loop is emitted
 // once per kind and issues its stores back to back (a run-time test per store would put a
-// branch between them).
+// branch between them).  THROUGH: whether the tile can be a pass of a multi-pass transform.
+template <bool THROUGH, class F> __device__ __forceinline__ void with_store(int kind, F&& f)
+{
+    if (kind == STORE_NT) f(std::integral_constant<int, STORE_NT>{});
+    else if (THROUGH && kind == STORE_THROUGH) f(std::integral_constant<int, STORE_THROUGH>{});
+    else f(std::integral_constant<int, STORE_PLAIN>{});
+}
+
+// The same for a flag.
 template <class F> __device__ __forceinline__ void with_nt(bool nt, F&& f)
 {
     if (nt) f(std::true_type{});
@@ -430,16 +455,15 @@ template <class C, bool IDLE, int S> __device__ __forceinline__ void tile_stage(
         if (x.valid && (!IDLE || x.active)) {
             const TileArgs& a = x.a;
             const unsigned mask = a.conj_out ? 0x80000000u : 0u;
-            const bool nt = a.nt_out != 0;
-            with_nt(nt, [&](auto ntc) {
-                constexpr bool NT = decltype(ntc)::value;
+            with_store<C::LOADT>(a.store, [&](auto kind) {
+                constexpr int KIND = decltype(kind)::value;
                 if (a.scale == 1.0) {
 #pragma unroll
                     for (int b = 0; b < B; ++b) {
                         const int j = x.jt + b * C::TPT;
                         if (GUARD && j >= LR) continue;
 #pragma unroll
-                        for (int r = 0; r < R; ++r) put<NT>(&x.out[(unsigned)(j + r * LR) * x.ons], flip_im(v[b][r], mask));
+                        for (int r = 0; r < R; ++r) put<KIND>(&x.out[(unsigned)(j + r * LR) * x.ons], flip_im(v[b][r], mask));
                     }
                 } else {
                     const auto sc = (decltype(v[0][0].x))a.scale;
@@ -449,7 +473,7 @@ template <class C, bool IDLE, int S> __device__ __forceinline__ void tile_stage(
                         if (GUARD && j >= LR) continue;
 #pragma unroll
                         for (int r = 0; r < R; ++r)
-                            put<NT>(&x.out[(unsigned)(j + r * LR) * x.ons], flip_im(cscale(v[b][r], sc), mask));
+                            put<KIND>(&x.out[(unsigned)(j + r * LR) * x.ons], flip_im(cscale(v[b][r], sc), mask));
                     }
                 }
             });
@@ -545,14 +569,13 @@ template <class C, bool IDLE> __device__ __forceinline__ void tile_finish(const 
         const unsigned mask = a.conj_out ? 0x80000000u : 0u;
         const auto sc = (decltype(V{}.x))a.scale;
         const bool scale = a.scale != 1.0;
-        const bool nt = a.nt_out != 0;
         const int tid = threadIdx.x;
         V* out = reinterpret_cast<V*>(a.out) + x.bo;
         if constexpr (C::PAIRED) {
             // paired sequences p and S - p (the C2R pre-pass of a first pass): element lin of
             // the tile is element q = lin % L of lane lin / L's sequence, stored by the rule
             if (!IDLE || x.active) {
-                with_nt(nt, [&](auto ntc) {
+                with_store<C::LOADT>(a.store, [&](auto kind) {
 #pragma unroll
                     for (int i = 0; i < PER; ++i) {
                         const int lin = tid + i * C::WG;
@@ -561,7 +584,7 @@ template <class C, bool IDLE> __device__ __forceinline__ void tile_finish(const 
                         if (tgs >= 0) {
                             V u = x.lds[C::lidx(ts, q)];
                             if (scale) u = cscale(u, sc);
-                            put<decltype(ntc)::value>(&out[out_base<C>(a, tgs) + (unsigned)q * ns], flip_im(u, mask));
+                            put<decltype(kind)::value>(&out[out_base<C>(a, tgs) + (unsigned)q * ns], flip_im(u, mask));
                         }
                     }
                 });
@@ -584,13 +607,13 @@ template <class C, bool IDLE> __device__ __forceinline__ void tile_finish(const 
                     const int lin = tid + i * C::WG;
                     u[i] = x.lds[C::lidx(lin / C::L, lin % C::L)];
                 }
-                with_nt(nt, [&](auto ntc) {
+                with_store<C::LOADT>(a.store, [&](auto kind) {
 #pragma unroll
                     for (int i = 0; i < PER; ++i)
-                        put<decltype(ntc)::value>(&o[tid + i * C::WG], flip_im(scale ? cscale(u[i], sc) : u[i], mask));
+                        put<decltype(kind)::value>(&o[tid + i * C::WG], flip_im(scale ? cscale(u[i], sc) : u[i], mask));
                 });
             } else if (!IDLE || x.active) {
-                with_nt(nt, [&](auto ntc) {
+                with_store<C::LOADT>(a.store, [&](auto kind) {
 #pragma unroll
                     for (int i = 0; i < PER; ++i) {
                         const int lin = tid + i * C::WG;
@@ -598,7 +621,7 @@ template <class C, bool IDLE> __device__ __forceinline__ void tile_finish(const 
                         if (ts < nvalid) {
                             V u = x.lds[C::lidx(ts, q)];
                             if (scale) u = cscale(u, sc);
-                            put<decltype(ntc)::value>(&o[lin], flip_im(u, mask));
+                            put<decltype(kind)::value>(&o[lin], flip_im(u, mask));
                         }
                     }
                 });
@@ -612,20 +635,20 @@ template <class C, bool IDLE> __device__ __forceinline__ void tile_finish(const 
             const long long tgs = (long long)tile * C::NB + ts;
             if ((!IDLE || x.active) && tgs < a.ntrans) {
                 V* o = out + out_base<C>(a, tgs);
-                with_nt(nt, [&](auto ntc) {
+                with_store<C::LOADT>(a.store, [&](auto kind) {
 #pragma unroll
                     for (int i = 0; i < PER; ++i) {
                         const int q = (tid + i * C::WG) / C::NB;
                         V u = x.lds[C::lidx(ts, q)];
                         if (scale) u = cscale(u, sc);
-                        put<decltype(ntc)::value>(&o[(unsigned)q * ns], flip_im(u, mask));
+                        put<decltype(kind)::value>(&o[(unsigned)q * ns], flip_im(u, mask));
                     }
                 });
             }
             return;
         }
         if (!IDLE || x.active) {
-            with_nt(nt, [&](auto ntc) {
+            with_store<C::LOADT>(a.store, [&](auto kind) {
 #pragma unroll
                 for (int i = 0; i < PER; ++i) {
                     const int lin = tid + i * C::WG;
@@ -634,7 +657,7 @@ template <class C, bool IDLE> __device__ __forceinline__ void tile_finish(const 
                     if (tgs < a.ntrans) {
                         V u = x.lds[C::lidx(ts, q)];
                         if (scale) u = cscale(u, sc);
-                        put<decltype(ntc)::value>(&out[out_base<C>(a, tgs) + (unsigned)q * ns], flip_im(u, mask));
+                        put<decltype(kind)::value>(&out[out_base<C>(a, tgs) + (unsigned)q * ns], flip_im(u, mask));
                     }
                 }
             });
@@ -670,31 +693,34 @@ template <class C, bool IDLE> __device__ __forceinline__ void split_finish(const
     const long long k0 = tgs + (long long)q0 * S, kst = (long long)QS * S;
     double2 w = dmul(a.sp_lo[k0 & mask], a.sp_hi[k0 >> a.sp_shift]);
     const double2 step = dmul(a.sp_lo[kst & mask], a.sp_hi[kst >> a.sp_shift]);
+    with_store<true>(a.store, [&](auto kind) {
+        constexpr int KIND = decltype(kind)::value;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int q = q0 + i * QS;
-        const int qp = tgs == 0 ? (q == 0 ? 0 : C::L - q) : C::L - 1 - q;
-        const long long k = tgs + (long long)q * S;
-        const V zk = x.lds[C::lidx(ts, q)], zp = x.lds[C::lidx(pl, qp)];
-        if (k == 0) {
-            const S_ x0 = zk.x + zk.y, xn = zk.x - zk.y;
-            if (a.split_bins) {
-                out[0] = V{x0, 0};
-                out[N] = V{xn, 0};
+        for (int i = 0; i < PER; ++i) {
+            const int q = q0 + i * QS;
+            const int qp = tgs == 0 ? (q == 0 ? 0 : C::L - q) : C::L - 1 - q;
+            const long long k = tgs + (long long)q * S;
+            const V zk = x.lds[C::lidx(ts, q)], zp = x.lds[C::lidx(pl, qp)];
+            if (k == 0) {
+                const S_ x0 = zk.x + zk.y, xn = zk.x - zk.y;
+                if (a.split_bins) {
+                    put<KIND>(&out[0], V{x0, 0});
+                    put<KIND>(&out[N], V{xn, 0});
+                } else {
+                    put<KIND>(&out[0], V{x0, xn});
+                }
             } else {
-                out[0] = V{x0, xn};
+                const bool lo = k <= N - k;
+                const V A = lo ? zk : zp, B = lo ? zp : zk;
+                const V wv = to_v<V>(lo ? w : double2{-w.x, w.y});  // W^k, or W^{N-k} = -conj(W^k)
+                const V h1 = V{half * (A.x + B.x), half * (A.y - B.y)};
+                const V dd = V{half * (A.x - B.x), half * (A.y + B.y)};
+                const V p = cmul(wv, V{dd.y, -dd.x});
+                put<KIND>(&out[k], lo ? V{h1.x + p.x, h1.y + p.y} : V{h1.x - p.x, p.y - h1.y});
             }
-        } else {
-            const bool lo = k <= N - k;
-            const V A = lo ? zk : zp, B = lo ? zp : zk;
-            const V wv = to_v<V>(lo ? w : double2{-w.x, w.y});  // W^k, or W^{N-k} = -conj(W^k)
-            const V h1 = V{half * (A.x + B.x), half * (A.y - B.y)};
-            const V dd = V{half * (A.x - B.x), half * (A.y + B.y)};
-            const V p = cmul(wv, V{dd.y, -dd.x});
-            out[k] = lo ? V{h1.x + p.x, h1.y + p.y} : V{h1.x - p.x, p.y - h1.y};
+            w = dmul(w, step);
         }
-        w = dmul(w, step);
-    }
+    });
 }
 
 // R2C split of an E->E tile (REAL_POST, single pass): the LDS holds each sequence's Z in

@@ -150,7 +150,7 @@ void tune_put(const std::string& key, const std::vector<int>& v)
 
 // Revision of the kernels the cached choices were measured with: part of every key, so that a
 // cache file written by a library with other tiles is measured afresh, not taken over.
-static constexpr int kTuneRevision = 2;
+static constexpr int kTuneRevision = 3;
 
 std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 {
@@ -161,19 +161,28 @@ std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
     return dev + ":r" + std::to_string(kTuneRevision) + "|" + (prec == PREC_F64 ? "f64" : "f32") + "|n=" + std::to_string(n) + "|b=" + std::to_string(batch);
 }
 
-// Time (ms) of one execution of a plan on scratch buffers, as a throughput: three groups of
-// `reps` executions issued back to back between two events, the median of the group means.
+// Time (ms) of one execution of a plan on scratch buffers, as a throughput: three groups of at
+// least `reps` executions issued back to back between two events, the median of the group means.
 // Back-to-back calls are what a batch loop issues; a call timed alone after a synchronisation
 // also carries the start of an idle device.
 // The calls walk over `sets` pairs of arrays, `stride` bytes apart, as a program's successive
 // inputs do: on one pair a transform of a few MB runs from the L2 caches, and the choice between
-// two splits can come out the other way.
-int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float* ms_out, int sets = 1, size_t stride = 0)
+// two splits can come out the other way.  With `alt` (2 (sets - 1) more arrays) the passes'
+// intermediate arrays change with them, as where a program's plans take turns: 3 * 2^20 reals FP32
+// in 1536 * 1024 take 28.6 us on one pair of them and 24.9 on three, in 256 * 96 * 64 26.0 and 25.0.
+int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float* ms_out, int sets = 1, size_t stride = 0,
+              void* alt = nullptr)
 {
     int call = 0;
     auto exec = [&]() {
-        const size_t off = (size_t)(call++ % sets) * stride;
-        return exec_device(p, (char*)a + off, (char*)b + off, s);
+        const size_t set = (size_t)(call++ % sets), off = set * stride;
+        if (alt && set && p->scratch[0]) {
+            p->call_scratch[0] = (char*)alt + 2 * (set - 1) * stride;
+            p->call_scratch[1] = (char*)alt + (2 * (set - 1) + 1) * stride;
+        }
+        const int rc = exec_device(p, (char*)a + off, (char*)b + off, s);
+        p->call_scratch[0] = p->call_scratch[1] = nullptr;
+        return rc;
     };
     for (int i = 0; i < 2; ++i) {
         int rc = exec();
@@ -186,7 +195,8 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
         (void)hipGetLastError();
         return fail(GFFTX_ERR_DEVICE, "cannot create timing events");
     }
-    for (int g = 0; g < 3; ++g) {
+    // a first group that does not count gives the repetitions: at least 0.4 ms in a group
+    for (int g = -1; g < 3; ++g) {
         (void)hipEventRecord(e0, s);
         int rc = GFFTX_SUCCESS;
         for (int i = 0; i < reps && !rc; ++i) rc = exec();
@@ -199,7 +209,11 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
         }
         float ms = 0;
         (void)hipEventElapsedTime(&ms, e0, e1);
-        t.push_back(ms / reps);
+        if (g >= 0) {
+            t.push_back(ms / reps);
+            continue;
+        }
+        reps = std::max(reps, (int)(0.4f / std::max(ms / reps, 0.002f)));
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -251,8 +265,8 @@ static std::vector<std::vector<int>> split_variants(int prec, unsigned long long
     return cands;
 }
 
-// The candidates vary one pass position at a time around the default tiles.  For the winning
-// split, the fastest variant timed at each position combined (ms[i] < 0: candidate i failed);
+// The candidates vary one pass position at a time around the default tiles.  For the split of
+// `chosen`, the fastest variant timed at each position combined (ms[i] < 0: candidate i failed);
 // empty when that is no new candidate.
 static std::vector<int> best_combination(const std::vector<int>& chosen, const std::vector<std::vector<int>>& cands,
                                          const std::vector<float>& ms)
@@ -353,6 +367,11 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             if (a) (void)hipFree(a);
             return GFFTX_SUCCESS;  // no room to tune: keep the cost-model plan
         }
+        void* alt = nullptr;
+        if (sets > 1 && !single_pass && !chirp && hipMalloc(&alt, bytes * 2 * (sets - 1)) != hipSuccess) {
+            (void)hipGetLastError();
+            alt = nullptr;
+        }
         hipStream_t s = nullptr;
         (void)hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
         (void)hipMemsetAsync(a, 0, bytes * sets, s);
@@ -372,7 +391,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
                 GFFTX_SUCCESS)
                 return -1.f;
             float ms = 0;
-            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms, sets, bytes);
+            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms, sets, bytes, alt);
             gfftx_plan_destroy(cp);
             if (trc) return -1.f;
             std::vector<int> sl;
@@ -402,14 +421,27 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             for (size_t i = 0; i < 5; ++i)
                 for (const std::vector<int>& c : chirp_variants(p->prec, n, chosen, i)) try_cand(c);
         } else if (!chosen.empty() && chosen[1] != 1) {
-            const std::vector<int> combo = best_combination(chosen, cands, cms);
-            if (!combo.empty()) try_cand(combo);
+            // the combination of the fastest variants, for each of the three fastest splits
+            std::vector<size_t> order(cands.size());
+            for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+            std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return cms[x] < cms[y]; });
+            std::vector<std::vector<int>> seen;
+            for (size_t i : order) {
+                std::vector<int> l;
+                std::vector<std::pair<int, int>> t;
+                split_choice(cands[i], l, t);
+                if (cms[i] < 0 || (l.size() == 2 && l[1] == 1) || std::find(seen.begin(), seen.end(), l) != seen.end()) continue;
+                seen.push_back(l);
+                const std::vector<int> combo = best_combination(cands[i], cands, cms);
+                if (!combo.empty()) try_cand(combo);
+                if (seen.size() == 3) break;
+            }
         }
         // the fastest few once more, in turn, on plans that stay: a single timing of a short transform
         // moves by more than the candidates differ
         std::vector<std::pair<float, std::vector<int>>> top = timed;
         std::stable_sort(top.begin(), top.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-        top.resize(std::min<size_t>(top.size(), bytes <= (64u << 20) ? 4 : 2));
+        top.resize(std::min<size_t>(top.size(), bytes <= (64u << 20) ? 6 : 2));
         if (top.size() > 1) {
             std::vector<gfftx_plan> tp(top.size(), nullptr);
             std::vector<float> tms(top.size(), 1e30f);
@@ -418,7 +450,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             for (int rep = 0; rep < 3; ++rep)
                 for (size_t i = 0; i < top.size(); ++i) {
                     float ms = 0;
-                    if (tp[i] && time_plan(tp[i], a, place == GFFTX_IN_PLACE ? a : b, s, 10, &ms, sets, bytes) == GFFTX_SUCCESS)
+                    if (tp[i] && time_plan(tp[i], a, place == GFFTX_IN_PLACE ? a : b, s, 10, &ms, sets, bytes, alt) == GFFTX_SUCCESS)
                         tms[i] = std::min(tms[i], ms);
                 }
             const size_t w = std::min_element(tms.begin(), tms.end()) - tms.begin();
@@ -430,6 +462,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         (void)hipStreamDestroy(s);
         (void)hipFree(a);
         (void)hipFree(b);
+        if (alt) (void)hipFree(alt);
         (void)hipGetLastError();
         if (chosen.empty()) return GFFTX_SUCCESS;
         note = timings;
