@@ -113,6 +113,9 @@ def _ptr(x):
     raise TypeError(f"unsupported buffer type {type(x)}")
 
 
+_scalars = {}  # element type of a tensor: bytes of one real scalar, or None
+
+
 def _scalar_bytes(x):
     """Bytes of one real scalar of a float/complex torch tensor or numpy array, else None."""
     if isinstance(x, np.ndarray):
@@ -122,10 +125,15 @@ def _scalar_bytes(x):
             return x.dtype.itemsize // 2
         return None
     dt = getattr(x, "dtype", None)
+    if dt in _scalars:
+        return _scalars[dt]
     if dt is None or not (dt.is_floating_point or dt.is_complex):
-        return None
-    es = x.element_size()
-    return es // 2 if dt.is_complex else es
+        sb = None
+    else:
+        es = x.element_size()
+        sb = es // 2 if dt.is_complex else es
+    _scalars[dt] = sb
+    return sb
 
 
 def _check_buffer(x, need: int, fp64: bool, device: int, what: str):
@@ -140,21 +148,35 @@ def _check_buffer(x, need: int, fp64: bool, device: int, what: str):
     if sb != want:
         raise ValueError(f"{what}: the plan computes in {'FP64' if fp64 else 'FP32'} "
                          f"({want}-byte scalars), the buffer holds {sb}-byte scalars")
-    nbytes = x.nbytes if isinstance(x, np.ndarray) else x.numel() * x.element_size()
+    nbytes = x.nbytes
     if nbytes < need:
         raise ValueError(f"{what}: buffer of {nbytes} bytes, the plan needs {need}")
-    if hasattr(x, "is_cuda") and x.is_cuda and x.device.index != device:
+    if getattr(x, "is_cuda", False) and x.device.index != device:
         raise ValueError(f"{what}: tensor on cuda:{x.device.index}, plan on device {device}")
 
 
 def _stream(x, stream):
     if stream is not None:
         return stream if isinstance(stream, int) else stream.cuda_stream
-    if hasattr(x, "is_cuda") and x.is_cuda:
+    if getattr(x, "is_cuda", False):
+        # the current stream's handle alone: the Stream object that torch.cuda.current_stream()
+        # makes around it took 2.2 us, a quarter of a small transform's call (8.1 us)
+        return _raw_stream()(x.device.index)
+    return None
+
+
+_raw = None
+
+
+def _raw_stream():
+    """Device index -> handle of torch's current stream there."""
+    global _raw
+    if _raw is None:
         import torch
 
-        return torch.cuda.current_stream(x.device).cuda_stream
-    return None
+        _raw = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda index: torch.cuda.current_stream(index).cuda_stream)
+    return _raw
 
 
 def plan_bytes(n: int, vtype: int, ttype: int, flags: int = 0, batch: int = 1):
@@ -193,12 +215,14 @@ class Plan:
         if dst is None:
             _check_buffer(data, self.inplace_bytes, self.fp64, self.device, "fft(data)")
             rc = lib().gfftx_exec_inplace(self._h, _ptr(data), _stream(data, stream))
-            _check(rc, "exec_inplace")
+            if rc:
+                _check(rc, "exec_inplace")
         else:
             _check_buffer(data, self.in_bytes, self.fp64, self.device, "fft(src, dst): src")
             _check_buffer(dst, self.out_bytes, self.fp64, self.device, "fft(src, dst): dst")
             rc = lib().gfftx_exec_oop(self._h, _ptr(data), _ptr(dst), _stream(data, stream))
-            _check(rc, "exec_oop")
+            if rc:
+                _check(rc, "exec_oop")
         return data if dst is None else dst
 
     def describe(self) -> str:

@@ -211,6 +211,11 @@ struct DeviceGuard {
             (void)hipGetLastError();
             prev = -1;
         }
+        if (prev == dev) {  // current already: nothing to set, nothing to set back
+            prev = -1;
+            ok = true;
+            return;
+        }
         ok = hipSetDevice(dev) == hipSuccess;
         if (!ok) (void)hipGetLastError();
     }

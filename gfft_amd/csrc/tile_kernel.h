@@ -268,9 +268,16 @@ template <int KIND, class V> __device__ __forceinline__ void put(V* p, V v)
 // branch between them).  THROUGH: whether the tile can be a pass of a multi-pass transform.
 template <bool THROUGH, class F> __device__ __forceinline__ void with_store(int kind, F&& f)
 {
-    if (kind == STORE_NT) f(std::integral_constant<int, STORE_NT>{});
-    else if (THROUGH && kind == STORE_THROUGH) f(std::integral_constant<int, STORE_THROUGH>{});
-    else f(std::integral_constant<int, STORE_PLAIN>{});
+    if constexpr (!THROUGH) {
+        if (kind != STORE_PLAIN) f(std::integral_constant<int, STORE_NT>{});
+        else f(std::integral_constant<int, STORE_PLAIN>{});
+    } else if (kind == STORE_NT) {
+        f(std::integral_constant<int, STORE_NT>{});
+    } else if (kind == STORE_THROUGH) {
+        f(std::integral_constant<int, STORE_THROUGH>{});
+    } else {
+        f(std::integral_constant<int, STORE_PLAIN>{});
+    }
 }
 
 // The same for a flag.
