@@ -136,7 +136,13 @@ bool fill(MixTile& t, int prec, int L, bool loadT, bool storeT, int real, int nb
     m.dl = divisor(L);
     m.nst = (unsigned)r.size();
     m.ts = L + m.pad * (L / r[0]);
-    if (m.ts % 2 == 0) ++m.ts;      // lanes that walk sequences hit distinct banks
+    // lanes that walk sequences hit distinct banks (TileCfg::lds_distance), where the LDS has room
+    const unsigned banks = prec == PREC_F64 ? 8 : 32, odd = m.ts | 1;
+    if (loadT && nb >= 2 && (unsigned)nb < banks)
+        while (m.ts % banks != banks / nb) ++m.ts;
+    else
+        m.ts = odd;
+    if ((size_t)nb * m.ts * eb > 160 * 1024) m.ts = odd;
     unsigned ns = 1, tw = 0;
     for (size_t s = 0; s < r.size(); ++s) {
         MixStage& st = m.st[s];

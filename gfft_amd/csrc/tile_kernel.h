@@ -117,9 +117,23 @@ struct TileCfg {
     static constexpr bool ahead(int s) { return TW_POW && s > 0 && s < NS && nbf(s) <= 4; }
     static constexpr int ROOTS = TW_POW ? most_roots() : 1;
     static constexpr int TW_ROOT_OFF = (twoff(NS) * (int)sizeof(V2<T_>) + 15) / 16 * 16;  // bytes
-    // LDS: one padded element every 16, odd distance between sequences (bank spread).
-    static constexpr int LP = L + L / 16;
-    static constexpr int TS = (LP % 2 == 0) ? LP + 1 : LP;
+    // LDS layout (bank spread): one pad element every 16, or every 8 where an FP32 pass tile begins
+    // with radix 8, and a distance TS between sequences.  In T mode NB lanes in a row take one
+    // element of NB sequences, the next ones the element after it: TS = 32 / NB modulo 32 FP32 (8 /
+    // NB modulo 8 FP64) spreads the 32 lanes of an 8-byte access (8 of a 16-byte one) over all
+    // banks, both where consecutive elements are read and where the first stage writes them R_0 +
+    // 1 apart.  Otherwise an odd distance.
+    static constexpr int PADSH = LOADT_ && sizeof(T_) == 4 && R[0] == 8 ? 3 : 4;
+    static constexpr int LP = L + (L >> PADSH);
+    static constexpr int lds_distance()
+    {
+        constexpr int banks = sizeof(T_) == 4 ? 32 : 8;
+        if (!LOADT_ || NB_ < 2 || NB_ >= banks || banks % NB_ != 0) return LP % 2 == 0 ? LP + 1 : LP;
+        int ts = LP;
+        while (ts % banks != banks / NB_) ++ts;
+        return ts;
+    }
+    static constexpr int TS = lds_distance();
     static constexpr bool DIRECT = (LOADT == STORET);
     static constexpr bool NEED_LDS = (NS > 1) || !DIRECT;
     static constexpr int LDS_ELEMS = NEED_LDS ? NB * TS : 1;
@@ -129,7 +143,7 @@ struct TileCfg {
     // E->E tiles whose TPT divides the wave size: every sequence is worked on by the lanes of
     // one wave, so the exchanges between stages need no workgroup barrier
     static constexpr bool WAVE_LOCAL = !LOADT && !STORET && (64 % TPT == 0);
-    __device__ static constexpr int lidx(int t, int e) { return t * TS + e + (e >> 4); }
+    __device__ static constexpr int lidx(int t, int e) { return t * TS + e + (e >> PADSH); }
 };
 
 // Orders the LDS accesses of the stages before it against those after it, for the threads
