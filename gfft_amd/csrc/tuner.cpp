@@ -150,7 +150,7 @@ void tune_put(const std::string& key, const std::vector<int>& v)
 
 // Revision of the kernels the cached choices were measured with: part of every key, so that a
 // cache file written by a library with other tiles is measured afresh, not taken over.
-static constexpr int kTuneRevision = 3;
+static constexpr int kTuneRevision = 4;
 
 std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 {
@@ -170,8 +170,10 @@ std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 // two splits can come out the other way.  With `alt` (2 (sets - 1) more arrays) the passes'
 // intermediate arrays change with them, as where a program's plans take turns: 3 * 2^20 reals FP32
 // in 1536 * 1024 take 28.6 us on one pair of them and 24.9 on three, in 256 * 96 * 64 26.0 and 25.0.
+// With `fill`, `a` is set to it before every group: a transform that runs in place would leave the
+// range of its numbers.
 int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float* ms_out, int sets = 1, size_t stride = 0,
-              void* alt = nullptr)
+              void* alt = nullptr, const void* fill = nullptr, size_t fill_bytes = 0)
 {
     int call = 0;
     auto exec = [&]() {
@@ -197,6 +199,7 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
     }
     // a first group that does not count gives the repetitions: at least 0.4 ms in a group
     for (int g = -1; g < 3; ++g) {
+        if (fill) (void)hipMemcpyAsync(a, fill, fill_bytes, hipMemcpyDeviceToDevice, s);
         (void)hipEventRecord(e0, s);
         int rc = GFFTX_SUCCESS;
         for (int i = 0; i < reps && !rc; ++i) rc = exec();
@@ -220,6 +223,26 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
     std::sort(t.begin(), t.end());
     *ms_out = t[t.size() / 2];
     return GFFTX_SUCCESS;
+}
+
+// Numbers between -1 and 1 (a multiplicative generator, repeated every MiB).
+static bool fill_numbers(int prec, void* dst, size_t bytes)
+{
+    const size_t block = std::min<size_t>(bytes, (size_t)1 << 20);
+    std::vector<double> d(prec == PREC_F64 ? block / 8 : 0);
+    std::vector<float> f(prec == PREC_F64 ? 0 : block / 4);
+    uint64_t x = 88172645463325252ull;
+    auto next = [&x]() {
+        x = x * 6364136223846793005ull + 1442695040888963407ull;
+        return (double)(int64_t)x / 9223372036854775808.0;
+    };
+    for (double& v : d) v = next();
+    for (float& v : f) v = (float)next();
+    const void* src = prec == PREC_F64 ? (const void*)d.data() : (const void*)f.data();
+    if (hipMemcpy(dst, src, block, hipMemcpyHostToDevice) != hipSuccess) return false;
+    for (size_t n = block; n < bytes; n *= 2)
+        if (hipMemcpy((char*)dst + n, dst, std::min(n, bytes - n), hipMemcpyDeviceToDevice) != hipSuccess) return false;
+    return true;
 }
 
 // The cost model's best `k` splits, and its best three of compiled tiles alone where they are
@@ -375,6 +398,12 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         hipStream_t s = nullptr;
         (void)hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
         (void)hipMemsetAsync(a, 0, bytes * sets, s);
+        // a large transform is bound by memory and by the power it takes, and on zeros it takes less
+        // power, so it is timed on numbers between -1 and 1 (65536 x 1024 FP64, four sequences a
+        // workgroup against one: 363 and 366 us on zeros, 369 and 364 on numbers)
+        const void* fill = nullptr;
+        if (sets == 1 && fill_numbers(p->prec, b, bytes) && hipMemcpy(a, b, bytes, hipMemcpyDeviceToDevice) == hipSuccess)
+            fill = place == GFFTX_IN_PLACE ? b : nullptr;
         float best = 1e30f;
         std::string timings = ",\"tuned\":[";
         size_t ntimed = 0;
@@ -391,7 +420,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
                 GFFTX_SUCCESS)
                 return -1.f;
             float ms = 0;
-            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms, sets, bytes, alt);
+            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms, sets, bytes, alt, fill, bytes);
             gfftx_plan_destroy(cp);
             if (trc) return -1.f;
             std::vector<int> sl;
@@ -450,7 +479,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             for (int rep = 0; rep < 3; ++rep)
                 for (size_t i = 0; i < top.size(); ++i) {
                     float ms = 0;
-                    if (tp[i] && time_plan(tp[i], a, place == GFFTX_IN_PLACE ? a : b, s, 10, &ms, sets, bytes, alt) == GFFTX_SUCCESS)
+                    if (tp[i] && time_plan(tp[i], a, place == GFFTX_IN_PLACE ? a : b, s, 10, &ms, sets, bytes, alt, fill, bytes) == GFFTX_SUCCESS)
                         tms[i] = std::min(tms[i], ms);
                 }
             const size_t w = std::min_element(tms.begin(), tms.end()) - tms.begin();
