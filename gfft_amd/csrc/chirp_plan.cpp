@@ -62,6 +62,24 @@ void one_tile(int prec, unsigned long long n, unsigned long long batch, int cus,
         }
 }
 
+// Modelled time (us) of one chirp-z pass by tile `k` over `batch` items of m points: 2.5 us of launch,
+// and either the bytes at the bandwidth the tile reaches (less for a run-time tile and for rows below a
+// 128-byte line) or, when there is little to move, the time of one tile, 1.5 us and 0.12 us per KB, for
+// each round of tiles the device holds at once.  (The chirp's and the filter's loads weigh on a
+// tile as its own bytes do, which the fit of pass_cost() to plain passes does not know.)
+double chirp_cost(const TileEntry* k, unsigned long long m, unsigned long long batch, int cus)
+{
+    const int by_lds = k->lds_bytes > 0 ? (160 * 1024) / k->lds_bytes : 8;
+    const int per_cu = std::max(1, std::min(by_lds, 2048 / k->wg));
+    const double tiles = std::ceil((double)(m / (unsigned long long)k->L) / k->nb) * (double)batch;
+    const double rounds = std::ceil(tiles / ((double)cus * per_cu));
+    const double kb = (double)k->nb * k->L * elem_bytes(k->prec) / 1024.0;
+    const double row = (double)k->nb * elem_bytes(k->prec);
+    const double bw = pass_bandwidth(k->prec, k->L) * (k->mix ? 0.9 : 1.0) * (row >= 128 ? 1.0 : row >= 64 ? 0.9 : 0.7);
+    const double move = 2.0 * (double)m * (double)batch * elem_bytes(k->prec) / (bw * 1e6);
+    return 2.5 + std::max(move, rounds * (1.5 + 0.12 * kb));
+}
+
 // Splits of m into two or three passes.
 void splits(int prec, unsigned long long m, unsigned long long batch, int cus, std::vector<Choice>& out)
 {
@@ -77,7 +95,7 @@ void splits(int prec, unsigned long long m, unsigned long long batch, int cus, s
         l.L = (int)d;
         for (int kind = 0; kind < 4; ++kind) {
             for (const TileEntry* k : pass_tiles(prec, l.L, kind == 3 ? 4 : kind, 5)) {
-                const double c = pass_cost(k, m, batch, cus) * (kind == 2 ? 1.5 : 1.0);  // the turn: two transforms
+                const double c = chirp_cost(k, m, batch, cus) * (kind == 2 ? 1.5 : 1.0);  // the turn: two transforms
                 if (l.t[kind] && c >= l.c[kind]) continue;
                 l.t[kind] = k;
                 l.c[kind] = c;

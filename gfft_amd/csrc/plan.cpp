@@ -157,7 +157,7 @@ int build_c2c_passes(gfftx_plan_s* p)
         std::vector<int> lens;
         std::vector<std::pair<int, int>> tiles;
         split_choice(p->forced_lens, lens, tiles);
-        if (lens.empty() && !choose_passes(p->prec, n, lens, p->batch, device_cus(p->device)))
+        if (lens.empty() && !choose_passes(p->prec, n, lens, p->batch, device_cus(p->device), p->real_part()))
             return fail(GFFTX_ERR_UNSUPPORTED, "no multi-pass decomposition for n=%llu", n);
         long long ns = 1;
         for (size_t i = 0; i < lens.size(); ++i) {
@@ -165,7 +165,7 @@ int build_c2c_passes(gfftx_plan_s* p)
             const int want_nb = i < tiles.size() && tiles[i].first ? tiles[i].first : env_int("GFFTX_TNB", 0);
             const int want_wg = i < tiles.size() && tiles[i].first ? tiles[i].second : env_int("GFFTX_TWG", 0);
             const TileEntry* k = want_nb || want_wg ? find_tile(p->prec, L, true, i > 0, want_nb, want_wg)
-                                                    : pass_tile(p->prec, L, i == 0, n, p->batch, device_cus(p->device));
+                                                    : pass_tile(p->prec, L, (unsigned long long)ns, n, p->batch, device_cus(p->device));
             if (!k) return fail(GFFTX_ERR_UNSUPPORTED, "no pass kernel L=%d", L);
             Pass ps;
             ps.k = k;

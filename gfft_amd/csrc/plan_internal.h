@@ -97,15 +97,24 @@ const TileEntry* find_real_tile(const TileEntry* k, int kind);
 int env_int(const char* name, int dflt);
 int device_cus(int device);
 double pass_bandwidth(int prec, int L);
-double pass_cost(const TileEntry* k, unsigned long long n, unsigned long long batch, int cus);
-const TileEntry* pass_tile(int prec, int L, bool first, unsigned long long n, unsigned long long batch, int cus,
+double pass_cost(const TileEntry* k, unsigned long long ns, unsigned long long n, unsigned long long batch, int cus);
+
+// The split of a real transform, as the cost model sees it.
+struct RealPart {
+    int kind = REAL_NONE;  // REAL_POST: forward, in the last pass; REAL_PRE: inverse, in the first one
+    bool copy = false;     // inverse, out of place: unfused, it works on a copy of the input
+};
+
+double split_cost(const RealPart& real, const TileEntry* k, unsigned long long n, unsigned long long batch);
+const TileEntry* pass_tile(int prec, int L, unsigned long long ns, unsigned long long n, unsigned long long batch, int cus,
                            double* cost = nullptr);
 std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch = 1,
-                                               int cus = 256, bool mixed = true);
+                                               int cus = 256, bool mixed = true, RealPart real = RealPart());
 void split_choice(const std::vector<int>& c, std::vector<int>& lens, std::vector<std::pair<int, int>>& tiles);
 int xcd_remap(const TileEntry* k, int prec);
 bool native_length(int prec, unsigned long long n);
-bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch = 1, int cus = 256);
+bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch = 1, int cus = 256,
+                   RealPart real = RealPart());
 int dev_alloc_list(std::vector<void*>& owned, void** out, size_t bytes);
 int upload_stage_table_r(std::vector<void*>& owned, int prec, int nrad, const int* radices, void** out,
                          double scale = 1.0);
@@ -243,6 +252,7 @@ struct gfftx_plan_s {
     bool real = false;
     bool inverse = false;
     unsigned long long dist = 0;   // complex elements between batch items
+    RealPart real_part() const { return RealPart{!real ? REAL_NONE : inverse ? REAL_PRE : REAL_POST, inverse && place == GFFTX_OUT_OF_PLACE}; }
     std::vector<int> forced_lens;  // plan choice made by the autotuner (empty: cost model), see split_choice
     std::string tune_note;         // autotuner record for plan_describe
     std::vector<Pass> passes;

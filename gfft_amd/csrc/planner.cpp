@@ -88,48 +88,73 @@ double pass_bandwidth(int prec, int L)
     return f32 ? 2.6 : 2.5;
 }
 
-// Modelled time (us) of one pass by tile `k` over `batch` items of n points: 2.5 us of launch,
-// and either the bytes at the bandwidth the tile reaches (less for a run-time tile and for rows
-// below a 128-byte line) or, when there is little to move, the time of one tile, 1.5 us and 0.12
-// us per KB, for each round of tiles the device holds at once (LDS and threads limit a CU to
-// 160 KB and 2048 threads).  The tile times are those of short passes issued back to back: 10 KB
-// tiles of 25 points 4.8 us in all, 49 KB ones of 1536 points 12.4 us, 64 KB ones of 1000 points
-// 13 us.
-double pass_cost(const TileEntry* k, unsigned long long n, unsigned long long batch, int cus)
+// Modelled time (us) of one pass by tile `k` after passes of `ns` points in all (1: the first pass),
+// over `batch` items of n points: the launch (a later pass also looks its twiddles up), and the
+// bytes at the bandwidth the tile reaches next to the time of the tiles, one round after the other
+// where the device does not hold them all (LDS and threads limit a CU to 160 KB and 2048 threads).
+// The bandwidth falls with rows below a 128-byte line, with rows that begin anywhere in one, and in a
+// run-time tile.  Fitted to 2193 splits of 69 lengths (16384 to 2^25 points, both precisions, 1 to
+// 300 items, back to back): 8% rms, and the split it ranks first takes 4% more than the fastest
+// of its length.  With one time a KB for every tile, and no stages, the first ranked one took 15%
+// more (262144 FP64 in 512 * 512, rows of 32 bytes, 18.9 us; in 1024 * 256, 13.2).
+double pass_cost(const TileEntry* k, unsigned long long ns, unsigned long long n, unsigned long long batch, int cus)
 {
     const int by_lds = k->lds_bytes > 0 ? (160 * 1024) / k->lds_bytes : 8;
     const int per_cu = std::max(1, std::min(by_lds, 2048 / k->wg));
-    const double tiles = std::ceil((double)(n / (unsigned long long)k->L) / k->nb) * (double)batch;
+    const unsigned long long eb = elem_bytes(k->prec), pitch = n / (unsigned long long)k->L;
+    const double tiles = std::ceil((double)pitch / k->nb) * (double)batch;
     const double rounds = std::ceil(tiles / ((double)cus * per_cu));
-    const double kb = (double)k->nb * k->L * elem_bytes(k->prec) / 1024.0;
-    const double row = (double)k->nb * elem_bytes(k->prec);
-    const double bw = pass_bandwidth(k->prec, k->L) * (k->mix ? 0.9 : 1.0) * (row >= 128 ? 1.0 : row >= 64 ? 0.9 : 0.7);
-    const double move = 2.0 * (double)n * (double)batch * elem_bytes(k->prec) / (bw * 1e6);
-    return 2.5 + std::max(move, rounds * (1.5 + 0.12 * kb));
+    const double kb = (double)k->nb * k->L * (double)eb / 1024.0;
+    const bool f64 = k->prec == PREC_F64;
+    const double tile = k->mix ? -0.4 + 1.7 * k->nrad + (f64 ? 0.061 : 0.056) * kb
+                               : -2.4 + 1.7 * k->nrad + (f64 ? 0.048 : 0.063) * kb;
+    const double bytes = (double)n * (double)batch * (double)eb;
+    const bool cached = bytes <= 64.0 * 1048576;  // the pass's arrays stay in the Infinity Cache
+    const unsigned long long row = (unsigned long long)k->nb * eb;
+    const double bw = 7.0 * (k->mix ? 0.78 : 1.0) *
+                      (row >= 128 ? 1.0 : row >= 64 ? (cached ? 0.85 : 0.65) : (cached ? 0.48 : 0.35)) *
+                      (pitch * eb % 128 ? 0.73 : 1.0) * (ns > 1 && ns * eb % 128 ? 0.88 : 1.0);
+    return (ns > 1 ? 3.0 : 0.4) + std::hypot(2.0 * bytes / (bw * 1e6), rounds * std::max(tile, 1.0));
 }
 
-// The tile a pass of length L takes unless one is named: the default one of a compiled length,
+// Modelled time (us) that a real transform's split adds to the passes when tile `k` is the one it can
+// ride in: the last pass of a forward transform, the first of an inverse one.  Measured against the
+// complex transform in the same passes: as a kernel of its own 2 us and 0.34 us a MB (an out-of-place
+// inverse copies its input as well, the same again); fused 4.5 us and, by the length of the half
+// rows it reads or writes, 0.15 (256 bytes, forward) to 1 us a MB (134 MB FP32 forward: 31 us in half
+// rows of 256 bytes, 49 of 64; 33 MB FP32 inverse: 15 us in half rows of 32 bytes, 42 of 16).
+double split_cost(const RealPart& real, const TileEntry* k, unsigned long long n, unsigned long long batch)
+{
+    if (real.kind == REAL_NONE) return 0;
+    const double mb = (double)n * (double)batch * elem_bytes(k->prec) / 1e6;
+    if (!find_real_tile(k, real.kind)) return (2.0 + 0.34 * mb) * (real.copy ? 2.0 : 1.0);
+    const size_t half = (size_t)k->nb / 2 * elem_bytes(k->prec);
+    const double us = real.kind == REAL_PRE ? (half >= 128 ? 0.2 : half >= 32 ? 0.3 : 0.9)
+                                            : (half >= 256 ? 0.15 : half >= 128 ? 0.28 : half >= 64 ? 0.4 : 1.0);
+    return 4.5 + us * mb;
+}
+
+// The tile a pass of length L takes after passes of `ns` points unless one is named: the default one of a compiled length,
 // the one with the lowest modelled time of a run-time length; null when there is none.  *cost is
-// the lowest modelled time of the length's tiles (the autotuner times them all).
-const TileEntry* pass_tile(int prec, int L, bool first, unsigned long long n, unsigned long long batch, int cus, double* cost)
+// that tile's modelled time: splits are ranked by the tiles they run with.
+const TileEntry* pass_tile(int prec, int L, unsigned long long ns, unsigned long long n, unsigned long long batch, int cus, double* cost)
 {
     const TileEntry* best = nullptr;
     double bc = 0;
-    for (const TileEntry* k : tile_shapes(prec, L, true, !first)) {
-        const double c = pass_cost(k, n, batch, cus);
-        if (!best || (k->mix && c < bc)) best = k;
-        if (best == k || c < bc) bc = c;
+    for (const TileEntry* k : tile_shapes(prec, L, true, ns > 1)) {
+        if (best && !k->mix) break;
+        const double c = pass_cost(k, ns, n, batch, cus);
+        if (best && c >= bc) continue;
+        best = k;
+        bc = c;
     }
     if (cost) *cost = bc;
     return best;
 }
 
-// Pass splits of n into T-mode tile lengths (2..4 passes), best `k` by the cost model
-// (pass_cost()).  The first length of every split has a T->E tile.  The lengths are the compiled
-// ones and, with `mixed`, every other divisor of n with the factors 2, 3, 5 and 7 from 17 up to
-// the run-time tiles' limit.
-std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch,
-                                               int cus, bool mixed)
+// Lengths of the pass tiles that divide n: the compiled ones and, with `mixed`, every other divisor
+// with the factors 2, 3, 5 and 7 from 17 up to the run-time tiles' limit.  Ascending.
+static std::vector<int> pass_lengths(int prec, unsigned long long n, bool mixed)
 {
     std::vector<int> lens;
     for (int i = 0; i < kNumTiles; ++i)
@@ -149,50 +174,73 @@ std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, s
         lens.insert(lens.end(), more.begin(), more.end());
         std::sort(lens.begin(), lens.end());
     }
-    // cost of each length as the first and as a later pass (negative: no such tile)
-    std::vector<double> cost0(lens.size()), cost1(lens.size());
+    return lens;
+}
+
+// Pass splits of n into T-mode tile lengths (2..4 passes), best `k` by the cost model (pass_cost(),
+// and split_cost() of a real transform).  The first length of every split has a T->E tile.
+std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch,
+                                               int cus, bool mixed, RealPart real)
+{
+    const std::vector<int> lens = pass_lengths(prec, n, mixed);
+    // cost of each length as the first pass, after passes of a multiple of 16 points (whole lines in
+    // both precisions) and after others (negative: no such tile), and of the split of a real transform
+    static const unsigned long long kNs[3] = {1, 16, 17};
+    struct Cost {
+        double pass[3] = {-1, -1, -1}, split[3] = {0, 0, 0};
+    };
+    std::vector<Cost> cost(lens.size());
     for (size_t i = 0; i < lens.size(); ++i)
-        for (int later = 0; later < 2; ++later)
-            if (!pass_tile(prec, lens[i], !later, n, batch, cus, &(later ? cost1 : cost0)[i]))
-                (later ? cost1 : cost0)[i] = -1.0;
-    std::vector<std::pair<double, std::vector<int>>> found;
-    std::vector<int> cur;  // indices into lens, largest first
-    std::function<void(unsigned long long, int)> rec = [&](unsigned long long rem, int maxi) {
+        for (int j = 0; j < 3; ++j) {
+            const TileEntry* t = pass_tile(prec, lens[i], kNs[j], n, batch, cus, &cost[i].pass[j]);
+            if (!t) cost[i].pass[j] = -1;
+            else if ((j == 0) == (real.kind == REAL_PRE)) cost[i].split[j] = split_cost(real, t, n, batch);
+        }
+    auto kind = [&](unsigned long long ns) { return ns == 1 ? 0 : ns * elem_bytes(prec) % 128 == 0 ? 1 : 2; };
+    std::vector<std::pair<double, std::vector<int>>> found;  // the best k so far, in the order met where equal
+    std::vector<int> cur;                                    // indices into lens, largest first
+    std::function<void(unsigned long long, int, double)> rec = [&](unsigned long long rem, int maxi, double least) {
+        if (found.size() == k && (k == 0 || least >= found.back().first)) return;  // no better than the best k
         if (rem == 1) {
             if (cur.size() < 2) return;
             std::vector<int> order = cur;
             for (size_t i = 0; i < order.size(); ++i)
-                if (cost0[order[i]] >= 0) {
+                if (cost[order[i]].pass[0] >= 0) {
                     std::swap(order[0], order[i]);
                     break;
                 }
-            if (cost0[order[0]] < 0) return;
-            double cost = 0;
+            double sum = 0;
             std::vector<int> l;
+            unsigned long long ns = 1;
             for (size_t i = 0; i < order.size(); ++i) {
-                const double c = i ? cost1[order[i]] : cost0[order[i]];
-                if (c < 0) return;
-                cost += c;
+                const Cost& c = cost[order[i]];
+                const int j = kind(ns);
+                if (c.pass[j] < 0) return;
+                sum += c.pass[j];
+                if (real.kind == REAL_PRE ? i == 0 : i + 1 == order.size()) sum += c.split[j];
                 l.push_back(lens[order[i]]);
+                ns *= (unsigned long long)lens[order[i]];
             }
-            found.push_back({cost, l});
+            auto at = std::upper_bound(found.begin(), found.end(), sum,
+                                       [](double c, const std::pair<double, std::vector<int>>& f) { return c < f.first; });
+            found.insert(at, {sum, l});
+            if (found.size() > k) found.pop_back();
             return;
         }
         if (cur.size() == 4) return;
         for (int i = maxi; i >= 0; --i) {
             if (rem % (unsigned long long)lens[i]) continue;
+            double c = -1;  // the least this length costs anywhere
+            for (double x : cost[i].pass)
+                if (x >= 0 && (c < 0 || x < c)) c = x;
             cur.push_back(i);
-            rec(rem / lens[i], i);
+            rec(rem / lens[i], i, least + std::max(c, 0.0));
             cur.pop_back();
         }
     };
-    rec(n, (int)lens.size() - 1);
-    std::stable_sort(found.begin(), found.end(),
-                     [](const std::pair<double, std::vector<int>>& x, const std::pair<double, std::vector<int>>& y) {
-                         return x.first < y.first;
-                     });
+    rec(n, (int)lens.size() - 1, 0.0);
     std::vector<std::vector<int>> out;
-    for (size_t i = 0; i < found.size() && out.size() < k; ++i) out.push_back(found[i].second);
+    for (const auto& f : found) out.push_back(f.second);
     return out;
 }
 
@@ -222,13 +270,23 @@ int xcd_remap(const TileEntry* k, int prec)
     return (size_t)k->nb * elem_bytes(prec) % 128 != 0 ? 1 : 0;
 }
 
-// Whether n runs natively: one compiled single-pass tile, or a split into compiled pass
-// tiles (lengths whose factors the tiles carry: 2, 3, 5 and 7).  Any other n runs as a
-// chirp-z convolution.
+// Whether n runs natively: one single-pass tile, or a split into pass tiles (lengths with the
+// factors 2, 3, 5 and 7).  Any other n runs as a chirp-z convolution.  (Every plan asks, so the
+// search ends at the first split: listing them all took 17 ms at 203212800.)
 bool native_length(int prec, unsigned long long n)
 {
     if (n <= (1ull << 30) && find_tile(prec, (int)n, false, false)) return true;
-    return !candidate_passes(prec, n, 1).empty();
+    const std::vector<int> lens = pass_lengths(prec, n, true);
+    std::function<bool(unsigned long long, int, int, bool)> rec = [&](unsigned long long rem, int maxi, int passes, bool first) {
+        if (rem == 1) return passes >= 2 && first;
+        if (passes == 4) return false;
+        for (int i = maxi; i >= 0; --i)
+            if (rem % (unsigned long long)lens[i] == 0 &&
+                rec(rem / lens[i], i, passes + 1, first || find_tile(prec, lens[i], true, false) != nullptr))
+                return true;
+        return false;
+    };
+    return rec(n, (int)lens.size() - 1, 0, false);
 }
 
 // The pass split GFFTX_PASSES="a,b,c" names, when it multiplies to n and every length has a tile.
@@ -265,11 +323,11 @@ const TileEntry* single_tile(int prec, unsigned long long n, int want_nb, int wa
 }
 
 // Split n into pass lengths available as T-mode tiles (largest first), or the override list.
-bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch, int cus)
+bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch, int cus, RealPart real)
 {
     out.clear();
     if (env_passes(prec, n, out)) return true;
-    std::vector<std::vector<int>> c = candidate_passes(prec, n, 1, batch, cus);
+    std::vector<std::vector<int>> c = candidate_passes(prec, n, 1, batch, cus, true, real);
     if (c.empty()) return false;
     out = c[0];
     return true;

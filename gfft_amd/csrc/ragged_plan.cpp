@@ -92,7 +92,7 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
         for (size_t i = 0; i < lens.size(); ++i) {
             const int tnb = i < t_tiles.size() ? t_tiles[i].first : 0, twg = i < t_tiles.size() ? t_tiles[i].second : 0;
             const TileEntry* k = tnb ? find_tile(r->prec, lens[i], true, i > 0, tnb, twg)
-                                     : pass_tile(r->prec, lens[i], i == 0, (unsigned long long)L,
+                                     : pass_tile(r->prec, lens[i], (unsigned long long)ns, (unsigned long long)L,
                                                  (unsigned long long)lc.count, device_cus(r->device));
             if (!k) return fail(GFFTX_ERR_UNSUPPORTED, "ragged batch: no pass kernel L=%d", lens[i]);
             Pass ps;

@@ -247,10 +247,11 @@ static bool fill_numbers(int prec, void* dst, size_t bytes)
 
 // The cost model's best `k` splits, and its best three of compiled tiles alone where they are
 // not among them.
-static std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus)
+static std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus,
+                                                  RealPart real = RealPart())
 {
-    std::vector<std::vector<int>> v = candidate_passes(prec, n, k, batch, cus);
-    for (const std::vector<int>& c : candidate_passes(prec, n, 3, batch, cus, false))
+    std::vector<std::vector<int>> v = candidate_passes(prec, n, k, batch, cus, true, real);
+    for (const std::vector<int>& c : candidate_passes(prec, n, 3, batch, cus, false, real))
         if (std::find(v.begin(), v.end(), c) == v.end()) v.push_back(c);
     return v;
 }
@@ -265,12 +266,15 @@ static std::vector<std::vector<int>> split_variants(int prec, unsigned long long
     for (const std::vector<int>& sp : splits) {
         cands.push_back(sp);
         std::vector<int> seen;
+        unsigned long long ns = 1;
         for (size_t i = 0; i < sp.size(); ++i) {
             const int L = sp[i];
             const bool later = i > 0;
+            const unsigned long long before = ns;
+            ns *= (unsigned long long)L;
             if (later && std::find(seen.begin(), seen.end(), L) != seen.end()) continue;
             if (later) seen.push_back(L);
-            const TileEntry* def = pass_tile(prec, L, !later, n, batch, cus);
+            const TileEntry* def = pass_tile(prec, L, before, n, batch, cus);
             for (const TileEntry* t : tile_shapes(prec, L, true, later)) {
                 if (t == def) continue;
                 const TileEntry& e = *t;
@@ -364,7 +368,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         const uint64_t tiles = single_pass ? (batch + p->passes[0].k->nb - 1) / p->passes[0].k->nb : 0;
         const uint64_t few = single_pass ? (p->passes[0].k->mix ? device_cus(device) : p->real ? 0 : 8) : 0;
         if (!chirp && (!single_pass || (n >= 2048 && tiles <= few)))
-            splits = tuned_splits(p->prec, n, (size_t)env_int("GFFTX_TUNE_CANDIDATES", 5), batch, device_cus(device));
+            splits = tuned_splits(p->prec, n, (size_t)env_int("GFFTX_TUNE_CANDIDATES", 5), batch, device_cus(device), p->real_part());
         // an inverse real transform's first pass carries the C2R pre-split, which halves the runs of
         // its rows: its two-pass splits are timed in the other order too
         if (p->real && p->inverse)

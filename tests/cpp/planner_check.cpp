@@ -1,0 +1,103 @@
+// planner_check.cpp -- the planner's choices, on the CPU.
+//
+//   - the split an untuned plan takes is one of those measured within 15% of the fastest of its
+//     length on an MI355X (back to back, three pairs of arrays), complex and real transforms;
+//   - the search for the best few splits finds what listing them all would;
+//   - a length runs natively exactly where a tile or a split exists.
+#include <cstdio>
+
+#include "../../gfft_amd/csrc/plan_internal.h"
+
+static int fails = 0;
+
+typedef std::vector<std::vector<int>> Splits;
+
+static std::string text(const std::vector<int>& v)
+{
+    std::string s;
+    for (int x : v) s += (s.empty() ? "" : "*") + std::to_string(x);
+    return s;
+}
+
+static const RealPart kComplex{}, kForward{REAL_POST, false}, kInverse{REAL_PRE, true};
+
+static void fast(RealPart real, int prec, unsigned long long n, const Splits& good)
+{
+    std::vector<int> l;
+    if (!choose_passes(prec, n, l, 1, 256, real) || std::find(good.begin(), good.end(), l) == good.end()) {
+        printf("FAIL real %d prec %d n %llu: %s is not among the fast splits\n", real.kind, prec, n, text(l).c_str());
+        ++fails;
+    }
+}
+
+static bool smooth(unsigned long long n)
+{
+    for (int f : {2, 3, 5, 7})
+        while (n % f == 0) n /= f;
+    return n == 1;
+}
+
+int main()
+{
+    unsetenv("GFFTX_PASSES");
+    const int F64 = PREC_F64, F32 = PREC_F32;
+    // (the fastest time, and a slow split for comparison)
+    fast(kComplex, F64, 32768, {{128, 16, 16}, {256, 16, 8}, {256, 128}, {1024, 32}});       // 11.1 us; 32*32*32 16.8
+    fast(kComplex, F32, 32768, {{128, 16, 16}, {256, 16, 8}, {256, 128}});                   // 9.8; 32*32*32 16.6
+    fast(kComplex, F64, 65536, {{256, 16, 16}, {256, 256}, {1024, 64}});                     // 11.4; 2048*32 16.3
+    fast(kComplex, F64, 262144, {{256, 64, 16}, {1024, 16, 16}, {1024, 256}});               // 13.2; 512*512 18.9
+    fast(kComplex, F32, 262144, {{128, 128, 16}, {256, 64, 16}, {256, 256, 4}, {1024, 16, 16}, {1024, 256}});  // 12.4; 512*512 15.2
+    fast(kComplex, F64, 393216, {{192, 128, 16}, {256, 96, 16}, {768, 512}, {1024, 384}, {1536, 256}});  // 16.4; 384*32*32 23.0
+    fast(kForward, F64, 32768, {{128, 16, 16}, {256, 16, 8}, {1024, 32}, {2048, 16}});       // 14.3; 32*32*32 19.3
+    fast(kForward, F32, 32768, {{128, 16, 16}, {256, 16, 8}, {256, 128}, {1024, 32}});       // 13.2; 32*32*32 19.0
+    fast(kForward, F64, 65536, {{256, 16, 16}, {256, 256}, {1024, 64}, {4096, 16}});         // 15.2; 2048*32 19.0
+    fast(kForward, F64, 262144, {{128, 128, 16}, {256, 64, 16}, {1024, 16, 16}, {1024, 256}});  // 17.0; 512*512 22.3
+    fast(kForward, F64, 196608, {{192, 64, 16}, {256, 96, 8}, {768, 256}, {1024, 192}, {1536, 128}});  // 17.5; 512*384 21.7
+    fast(kForward, F32, 1572864, {{192, 128, 64}, {256, 96, 64}, {256, 128, 48}, {384, 256, 16}, {1536, 64, 16}, {1536, 1024}});  // 25.0; 256*128*48 31.0
+    fast(kInverse, F64, 32768, {{128, 16, 16}, {256, 16, 8}, {256, 128}, {512, 64}, {1024, 32}});  // 16.1; 32*32*32 21.5
+    fast(kInverse, F32, 32768, {{128, 16, 16}, {256, 16, 8}, {256, 128}, {512, 64}});        // 14.3; 32*32*32 21.1
+    fast(kInverse, F64, 65536, {{256, 16, 16}, {256, 256}, {512, 128}, {1024, 64}});         // 16.3; 2048*32 23.0
+    fast(kInverse, F32, 65536, {{256, 16, 16}, {256, 256}, {512, 128}, {1024, 64}});         // 14.7; 4096*16 21.0
+    fast(kInverse, F64, 262144, {{256, 64, 16}, {256, 256, 4}, {1024, 16, 16}, {1024, 256}});  // 21.5; 512*512 27.0
+    fast(kInverse, F64, 393216, {{128, 64, 48}, {256, 96, 16}, {256, 192, 8}, {1024, 384}});  // 24.0; 384*32*32 33.5
+    // the split's own pass is part of the price: where the array is large, it rides in a pass
+    for (int prec : {F64, F32})
+        for (unsigned long long n = 1 << 20; n <= 1 << 24; n *= 2)
+            for (const RealPart& real : {kForward, kInverse}) {
+                std::vector<int> l;
+                choose_passes(prec, n, l, 1, 256, real);
+                const bool post = real.kind == REAL_POST;
+                const TileEntry* k = l.empty() ? nullptr : pass_tile(prec, post ? l.back() : l[0], post ? n / l.back() : 1, n, 1, 256);
+                if (!k || !find_real_tile(k, real.kind)) {
+                    printf("FAIL real %d prec %d n %llu: %s leaves the split to a kernel of its own\n", real.kind, prec, n, text(l).c_str());
+                    ++fails;
+                }
+            }
+    // pruned search against the full list
+    for (unsigned long long n : {4096ull, 20000ull, 44100ull, 362880ull, 1ull << 20, 3628800ull, 12700800ull})
+        for (int prec : {F64, F32})
+            for (const RealPart& real : {kComplex, kForward, kInverse}) {
+                Splits all = candidate_passes(prec, n, 1000000, 1, 256, true, real), some = candidate_passes(prec, n, 5, 1, 256, true, real);
+                all.resize(std::min<size_t>(all.size(), 5));
+                if (all != some) {
+                    printf("FAIL prec %d n %llu: the best five differ\n", prec, n);
+                    ++fails;
+                }
+            }
+    for (int prec : {F64, F32}) {
+        for (unsigned long long n = 1; n <= 4000; ++n) {
+            const bool want = find_tile(prec, (int)n, false, false) || !candidate_passes(prec, n, 1).empty();
+            if (native_length(prec, n) != want || (n > 1 && want != smooth(n))) {
+                printf("FAIL prec %d n %llu: native %d\n", prec, n, (int)native_length(prec, n));
+                ++fails;
+            }
+        }
+        for (unsigned long long n : {1ull << 28, 203212800ull, 127008000ull, 1000000ull, 1000003ull, 2097143ull, 282475249ull, 11ull << 20})
+            if (native_length(prec, n) != !candidate_passes(prec, n, 1).empty()) {
+                printf("FAIL prec %d n %llu: native %d\n", prec, n, (int)native_length(prec, n));
+                ++fails;
+            }
+    }
+    printf("%d failures\n", fails);
+    return fails != 0;
+}
