@@ -360,7 +360,7 @@ int run_bluestein(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Ran
             a.scale = last && p->inverse ? 1.0 / (double)p->n : 1.0;
             a.xcd = ps.xcd;
             const size_t odist = last ? p->dist : p->blue_m;
-            a.store = pass_store(r.nt, i, np, odist * nb * eb, ps, odist, nb);
+            a.store = pass_store(p->through, r.nt, i, np, odist * nb * eb, ps, odist, nb);
             if (np == 1) a.seq_off = bo;
             else if (first || last) a.boff = bo;
             ChirpArgs c;

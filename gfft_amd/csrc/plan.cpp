@@ -38,27 +38,45 @@ bool nt_output(size_t bytes)
     return mib >= 0 && bytes > (size_t)mib << 20;
 }
 
-// How pass `ps`, number i of m, stores its `bytes` of output (STORE_*, tile_kernel.h).  Through the L2
-// from 2 MiB (below, the shorter way of a plain store counts more: 59049 FP64, 0.9 MiB, 12.2 us plain,
-// 12.7 through) to 64 MiB (2^23 FP32, 74.0 us plain, 69.4 through; 2^20 x 16 FP32, 128 MiB, 143-147
-// plain, 148 through) where the tile writes whole 128-byte lines.  Parts of lines are written by
-// themselves, so with them the gain ends at 16 MiB (2^20 FP32 in rows of 32 bytes 17.4 -> 15.9 us,
-// but 823543 x 5 FP32, 31 MiB, 49.5 -> 51.9 and 3000000 FP64, 46 MiB, 67.8 -> 74.2), and the R2C
-// split, whose rows are half as long and begin anywhere, gains with long ones alone (3 * 2^20 reals
-// FP32: rows of 256 bytes 32.4 -> 24.9 us, of 16 bytes 27.9 -> 33.1).  GFFTX_THROUGH_STORE=0: never.
-int pass_store(bool nt, size_t i, size_t m, size_t bytes, const Pass& ps, size_t dist, size_t items)
+// How pass `ps`, number i of m, stores its `bytes` of output (STORE_*, tile_kernel.h): non-temporally at
+// the end of a large call, through the L2 where that pays, else plainly.
+//
+// Through the L2 from 2 MiB (below, the shorter way of a plain store counts more: 59049 FP64, 0.9 MiB,
+// 12.2 us plain, 12.7 through) to 64 MiB (2^23 FP32, 74.0 us plain, 69.4 through; 2^20 x 16 FP32, 128 MiB,
+// 143-147 plain, 148 through) where the tile writes whole 128-byte lines.  Parts of lines are written by
+// themselves, so with them the gain ends at 16 MiB (823543 x 5 FP32, 31 MiB, 49.5 -> 51.9 and 3000000
+// FP64, 46 MiB, 67.8 -> 74.2), and with rows below 64 bytes it begins at 8 (524288 FP32 ending in 512,
+// 4 MiB, 16.0 -> 16.5 us; 2^20 FP32, 17.4 -> 15.9).
+//
+// The pass of a real transform's split, plain -> through, us:
+//   forward (rows half as long, beginning anywhere): half rows of 256 bytes 28.4 -> 27.1 (2^21 FP32, 16 MiB),
+//   81.8 -> 80.3 (2^22 FP64, 64 MiB); of 128 bytes 17.9 -> 17.4 (2^18 FP64), 47.5 -> 44.5 (2^21 FP64, 32 MiB),
+//   84.6 -> 83.7 (2^23 FP32, 64 MiB); of 64 bytes 16.2 -> 15.8 (2^18 FP32, 2 MiB), 161.5 -> 167.9 (2^24 FP32,
+//   128 MiB); of 32 bytes 25.6 -> 26.3 (2^20 FP32), 32.7 -> 34.6 (FP64);
+//   inverse (whole sequences, a pair's elements side by side): FP32 17.7 -> 21.5 (2^18, 2 MiB), 26.5 -> 27.3
+//   (2^20, 8 MiB), 34.6 -> 32.3 (3 * 2^19, 12 MiB), 38.2 -> 34.7 (2^21), 53.9 -> 53.8 (2^22, 32 MiB), 85.5 ->
+//   89.8 (2^23); FP64 17.5 -> 20.4 (2^17, 2 MiB), 27.7 -> 29.3 (2^19, 8 MiB), 36.3 -> 36.1 (2^20, 16 MiB), with the
+//   passes behind it through as well 55.6 -> 51.8 (2^21, 32 MiB), 83.7 -> 88.5 (2^22).
+// Non-temporally, the forward split's pass wants half rows of 256 bytes: 2^25 FP64 811 -> 778 us, 2^26 FP32 897
+// -> 855, but 2^24 FP64 (128 bytes) 336 -> 389 and 2^25 FP32 (128 bytes) 424 -> 433.
+// GFFTX_THROUGH_STORE=0 (when the plan is made): never through.
+int pass_store(bool through, bool nt, size_t i, size_t m, size_t bytes, const Pass& ps, size_t dist, size_t items)
 {
-    if (nt && i + 1 == m) return STORE_NT;
-    if (m < 2 || bytes < (size_t)2 << 20 || env_int("GFFTX_THROUGH_STORE", 1) == 0) return STORE_PLAIN;
     const TileEntry& k = *ps.k;
-    const size_t eb = elem_bytes(k.prec);
+    const size_t eb = elem_bytes(k.prec), half = (size_t)k.nb / 2 * eb;
+    const bool post = k.real == REAL_POST && k.loadT;
+    if (nt && i + 1 == m) return post && half < 256 ? STORE_PLAIN : STORE_NT;
+    if (m < 2 || !through) return STORE_PLAIN;
     auto lines = [&](size_t elems) { return elems * eb % 128 == 0; };
-    size_t mib;
-    if (k.real == REAL_POST) mib = (size_t)k.nb / 2 * eb >= 256 ? 25 : 0;
-    else if (items > 1 && !lines(dist)) mib = 16;
-    else if (k.storeT) mib = lines(k.nb) && lines(ps.ns_pass) ? 64 : 16;
-    else mib = lines(k.real == REAL_PRE ? k.L : k.nb * k.L) ? 64 : 16;
-    return bytes <= mib << 20 ? STORE_THROUGH : STORE_PLAIN;
+    size_t least = 2, most;  // MiB
+    if (post) most = half >= 128 ? 64 : half >= 64 ? 16 : 0;
+    else if (items > 1 && !lines(dist)) most = 16;
+    else if (k.storeT) most = lines(k.nb) && lines(ps.ns_pass) ? 64 : 16;
+    else if (k.real == REAL_PRE) most = lines(k.L) ? 32 : 16;
+    else most = lines((size_t)k.nb * k.L) ? 64 : 16;
+    if (k.real == REAL_PRE) least = k.prec == PREC_F64 ? 16 : 12;
+    else if (k.storeT && !post && (size_t)k.nb * eb < 64) least = 8;
+    return bytes >= least << 20 && bytes <= most << 20 ? STORE_THROUGH : STORE_PLAIN;
 }
 
 int dev_alloc(gfftx_plan_s* p, void** out, size_t bytes)
@@ -344,7 +362,7 @@ int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range 
         a.conj_out = (p->inverse && i == m - 1) ? 1 : 0;
         a.scale = (p->inverse && i == m - 1) ? 1.0 / (double)p->n : 1.0;
         a.xcd = ps.xcd;
-        a.store = pass_store(r.nt, i, m, (size_t)p->dist * r.nb * elem_bytes(p->prec), ps, p->dist, r.nb);
+        a.store = pass_store(p->through, r.nt, i, m, (size_t)p->dist * r.nb * elem_bytes(p->prec), ps, p->dist, r.nb);
         const long long nb = ps.k->nb;
         unsigned ntiles = (unsigned)((a.ntrans + nb - 1) / nb);
         if (ps.real) {
@@ -543,6 +561,7 @@ int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int
     p->inverse = ttype == GFFTX_IDFT || ttype == GFFTX_IRDFT;
     p->dist = n + ((real && (flags & GFFTX_FLAG_R2C_BINS)) ? 1 : 0);
     p->forced_lens = forced;
+    p->through = env_int("GFFTX_THROUGH_STORE", 1) != 0;
     p->tune_note = note;
     int rc = native_length(p->prec, n) ? build_c2c_passes(p) : build_bluestein(p);
     // an unfused split runs as a kernel of its own with a table; that of an out-of-place

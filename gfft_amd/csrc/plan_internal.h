@@ -80,7 +80,8 @@ struct Range {
 bool nt_output(size_t bytes);
 
 // How pass `ps`, number i of m, stores its `bytes` of output: `items` batch items, `dist` elements apart.
-int pass_store(bool nt, size_t i, size_t m, size_t bytes, const Pass& ps, size_t dist, size_t items);
+// `through`: stores through the L2 are allowed; nt: the last pass's output is stored non-temporally.
+int pass_store(bool through, bool nt, size_t i, size_t m, size_t bytes, const Pass& ps, size_t dist, size_t items);
 
 inline size_t elem_bytes(int prec) { return prec == PREC_F64 ? 16 : 8; }
 
@@ -253,6 +254,7 @@ struct gfftx_plan_s {
     bool inverse = false;
     unsigned long long dist = 0;   // complex elements between batch items
     RealPart real_part() const { return RealPart{!real ? REAL_NONE : inverse ? REAL_PRE : REAL_POST, inverse && place == GFFTX_OUT_OF_PLACE}; }
+    bool through = true;           // passes may store through the L2 (GFFTX_THROUGH_STORE when the plan was made)
     std::vector<int> forced_lens;  // plan choice made by the autotuner (empty: cost model), see split_choice
     std::string tune_note;         // autotuner record for plan_describe
     std::vector<Pass> passes;

@@ -3,6 +3,7 @@
 //   - the split an untuned plan takes is one of those measured within 15% of the fastest of its
 //     length on an MI355X (back to back, three pairs of arrays), complex and real transforms;
 //   - the search for the best few splits finds what listing them all would;
+//   - passes store the way that was measured fastest for their kind, rows and size;
 //   - a length runs natively exactly where a tile or a split exists.
 #include <cstdio>
 
@@ -26,6 +27,22 @@ static void fast(RealPart real, int prec, unsigned long long n, const Splits& go
     std::vector<int> l;
     if (!choose_passes(prec, n, l, 1, 256, real) || std::find(good.begin(), good.end(), l) == good.end()) {
         printf("FAIL real %d prec %d n %llu: %s is not among the fast splits\n", real.kind, prec, n, text(l).c_str());
+        ++fails;
+    }
+}
+
+// Store kind of pass i of the split `lens` for n points, one item.
+static void store(int want, RealPart real, int prec, unsigned long long n, const std::vector<int>& lens, size_t i, bool nt = false)
+{
+    unsigned long long ns = 1;
+    for (size_t j = 0; j < i; ++j) ns *= (unsigned long long)lens[j];
+    Pass ps;
+    ps.k = pass_tile(prec, lens[i], ns, n, 1, 256);
+    if (real.kind == REAL_POST ? i + 1 == lens.size() : real.kind == REAL_PRE && i == 0) ps.k = find_real_tile(ps.k, real.kind);
+    ps.ns_pass = (long long)ns;
+    const int got = !ps.k ? -1 : pass_store(true, nt, i, lens.size(), (size_t)n * elem_bytes(prec), ps, (size_t)n, 1);
+    if (got != want || (ps.k && pass_store(false, false, i, lens.size(), (size_t)n * elem_bytes(prec), ps, (size_t)n, 1) != STORE_PLAIN)) {
+        printf("FAIL real %d prec %d n %llu %s pass %zu: store %d, not %d\n", real.kind, prec, n, text(lens).c_str(), i, got, want);
         ++fails;
     }
 }
@@ -73,6 +90,37 @@ int main()
                     ++fails;
                 }
             }
+    // forward splits: half rows of 128 bytes and more through the L2 to 64 MiB, of 64 to 16, shorter ones never
+    store(STORE_THROUGH, kForward, F32, 3 << 19, {256, 96, 64}, 2);
+    store(STORE_THROUGH, kForward, F32, 1 << 22, {256, 256, 64}, 2);
+    store(STORE_THROUGH, kForward, F64, 1 << 21, {128, 128, 128}, 2);
+    store(STORE_THROUGH, kForward, F32, 1 << 18, {1024, 256}, 1);
+    store(STORE_PLAIN, kForward, F32, 1 << 17, {1024, 128}, 1);
+    store(STORE_PLAIN, kForward, F32, 1 << 24, {256, 256, 256}, 2);
+    store(STORE_PLAIN, kForward, F64, 1 << 20, {1024, 1024}, 1);
+    // at the end of a call above the Infinity Cache: non-temporally with half rows of 256 bytes
+    store(STORE_PLAIN, kForward, F64, 1 << 24, {256, 256, 256}, 2, true);
+    store(STORE_PLAIN, kForward, F32, 1 << 26, {1024, 512, 128}, 2, true);
+    store(STORE_NT, kForward, F64, 1 << 25, {1024, 256, 128}, 2, true);
+    store(STORE_NT, kForward, F32, 1 << 26, {1024, 1024, 64}, 2, true);
+    store(STORE_NT, kComplex, F32, 1 << 26, {1024, 512, 128}, 2, true);
+    // inverse splits: from 12 (FP64 16) to 32 MiB
+    store(STORE_PLAIN, kInverse, F32, 1 << 18, {1024, 256}, 0);
+    store(STORE_PLAIN, kInverse, F64, 1 << 17, {1024, 128}, 0);
+    store(STORE_PLAIN, kInverse, F32, 1 << 20, {256, 64, 64}, 0);
+    store(STORE_THROUGH, kInverse, F32, 3 << 19, {256, 96, 64}, 0);
+    store(STORE_THROUGH, kInverse, F32, 1 << 22, {256, 256, 64}, 0);
+    store(STORE_PLAIN, kInverse, F32, 1 << 23, {256, 256, 128}, 0);
+    store(STORE_PLAIN, kInverse, F64, 1 << 19, {256, 128, 16}, 0);
+    store(STORE_THROUGH, kInverse, F64, 1 << 21, {256, 128, 64}, 0);
+    store(STORE_PLAIN, kInverse, F64, 1 << 22, {256, 256, 64}, 0);
+    store(STORE_THROUGH, kInverse, F64, 1 << 21, {256, 128, 64}, 1);
+    // complex passes: from 2 MiB, rows below 64 bytes from 8, whole lines to 64 MiB
+    store(STORE_THROUGH, kComplex, F64, 1 << 17, {1024, 128}, 0);
+    store(STORE_PLAIN, kComplex, F32, 1 << 17, {1024, 128}, 0);
+    store(STORE_THROUGH, kComplex, F32, 1 << 23, {256, 256, 128}, 2);
+    store(STORE_PLAIN, kComplex, F64, 1 << 23, {256, 256, 128}, 2);
+    store(STORE_PLAIN, kComplex, F32, 3 << 20, {256, 192, 64}, 1);
     // pruned search against the full list
     for (unsigned long long n : {4096ull, 20000ull, 44100ull, 362880ull, 1ull << 20, 3628800ull, 12700800ull})
         for (int prec : {F64, F32})
