@@ -161,6 +161,15 @@ std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
     return dev + ":r" + std::to_string(kTuneRevision) + "|" + (prec == PREC_F64 ? "f64" : "f32") + "|n=" + std::to_string(n) + "|b=" + std::to_string(batch);
 }
 
+// Transforms of n points that may run in place one after the other from numbers around 1: each
+// forward one multiplies their rms by sqrt(n) (a real one of 2n points by sqrt(2n)), each inverse one
+// divides it.  Up to 2^100 FP32 and 2^900 FP64 either way: a chirp-z transform's convolution goes up to 2^14
+// higher, and single numbers 2^3.  At least one.
+int fill_reps(int prec, unsigned long long n)
+{
+    return std::max(1, (int)((prec == PREC_F64 ? 1800.0 : 200.0) / std::log2(2.0 * (double)n)));
+}
+
 // Time (ms) of one execution of a plan on scratch buffers, as a throughput: three groups of at
 // least `reps` executions issued back to back between two events, the median of the group means.
 // Back-to-back calls are what a batch loop issues; a call timed alone after a synchronisation
@@ -170,11 +179,13 @@ std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 // two splits can come out the other way.  With `alt` (2 (sets - 1) more arrays) the passes'
 // intermediate arrays change with them, as where a program's plans take turns: 3 * 2^20 reals FP32
 // in 1536 * 1024 take 28.6 us on one pair of them and 24.9 on three, in 256 * 96 * 64 26.0 and 25.0.
-// With `fill`, `a` is set to it before every group: a transform that runs in place would leave the
-// range of its numbers.
+// With `fill`, `a` is set to it before every group, which then has at most fill_reps() executions: a
+// transform that runs in place would leave the range of its numbers.
 int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float* ms_out, int sets = 1, size_t stride = 0,
               void* alt = nullptr, const void* fill = nullptr, size_t fill_bytes = 0)
 {
+    const int most = fill ? fill_reps(p->prec, p->n) : 1 << 30;
+    reps = std::min(reps, most);
     int call = 0;
     auto exec = [&]() {
         const size_t set = (size_t)(call++ % sets), off = set * stride;
@@ -216,7 +227,7 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
             t.push_back(ms / reps);
             continue;
         }
-        reps = std::max(reps, (int)(0.4f / std::max(ms / reps, 0.002f)));
+        reps = std::min(most, std::max(reps, (int)(0.4f / std::max(ms / reps, 0.002f))));
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -225,8 +236,8 @@ int time_plan(gfftx_plan_s* p, void* a, void* b, hipStream_t s, int reps, float*
     return GFFTX_SUCCESS;
 }
 
-// Numbers between -1 and 1 (a multiplicative generator, repeated every MiB).
-static bool fill_numbers(int prec, void* dst, size_t bytes)
+// Numbers between -1 and 1 (a multiplicative generator, repeated every MiB), written on stream s.
+static bool fill_numbers(int prec, void* dst, size_t bytes, hipStream_t s)
 {
     const size_t block = std::min<size_t>(bytes, (size_t)1 << 20);
     std::vector<double> d(prec == PREC_F64 ? block / 8 : 0);
@@ -239,10 +250,10 @@ static bool fill_numbers(int prec, void* dst, size_t bytes)
     for (double& v : d) v = next();
     for (float& v : f) v = (float)next();
     const void* src = prec == PREC_F64 ? (const void*)d.data() : (const void*)f.data();
-    if (hipMemcpy(dst, src, block, hipMemcpyHostToDevice) != hipSuccess) return false;
-    for (size_t n = block; n < bytes; n *= 2)
-        if (hipMemcpy((char*)dst + n, dst, std::min(n, bytes - n), hipMemcpyDeviceToDevice) != hipSuccess) return false;
-    return true;
+    bool ok = hipMemcpyAsync(dst, src, block, hipMemcpyHostToDevice, s) == hipSuccess;
+    for (size_t n = block; ok && n < bytes; n *= 2)
+        ok = hipMemcpyAsync((char*)dst + n, dst, std::min(n, bytes - n), hipMemcpyDeviceToDevice, s) == hipSuccess;
+    return hipStreamSynchronize(s) == hipSuccess && ok;  // before the host arrays go
 }
 
 // The cost model's best `k` splits, and its best three of compiled tiles alone where they are
@@ -406,7 +417,9 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         // power, so it is timed on numbers between -1 and 1 (65536 x 1024 FP64, four sequences a
         // workgroup against one: 363 and 366 us on zeros, 369 and 364 on numbers)
         const void* fill = nullptr;
-        if (sets == 1 && fill_numbers(p->prec, b, bytes) && hipMemcpy(a, b, bytes, hipMemcpyDeviceToDevice) == hipSuccess)
+        // (all of it on `s`: that stream does not wait for the null stream)
+        if (sets == 1 && fill_numbers(p->prec, b, bytes, s) &&
+            hipMemcpyAsync(a, b, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess)
             fill = place == GFFTX_IN_PLACE ? b : nullptr;
         float best = 1e30f;
         std::string timings = ",\"tuned\":[";

@@ -4,6 +4,7 @@
 //     length on an MI355X (back to back, three pairs of arrays), complex and real transforms;
 //   - the search for the best few splits finds what listing them all would;
 //   - passes store the way that was measured fastest for their kind, rows and size;
+//   - the autotuner's repeated in-place transforms stay in the range of their numbers;
 //   - a length runs natively exactly where a tile or a split exists.
 #include <cstdio>
 
@@ -121,6 +122,15 @@ int main()
     store(STORE_THROUGH, kComplex, F32, 1 << 23, {256, 256, 128}, 2);
     store(STORE_PLAIN, kComplex, F64, 1 << 23, {256, 256, 128}, 2);
     store(STORE_PLAIN, kComplex, F32, 3 << 20, {256, 192, 64}, 1);
+    // in-place timing stays in the range of its numbers (27 bits of FP32's, 123 of FP64's kept clear)
+    for (unsigned long long n = 2; n <= 1ull << 28; n = n * 5 / 3 + 1)
+        for (int prec : {F64, F32}) {
+            const int r = fill_reps(prec, n);
+            if (r < 1 || r * std::log2(2.0 * (double)n) / 2 > (prec == F64 ? 900 : 100)) {
+                printf("FAIL prec %d n %llu: %d transforms in place\n", prec, n, r);
+                ++fails;
+            }
+        }
     // pruned search against the full list
     for (unsigned long long n : {4096ull, 20000ull, 44100ull, 362880ull, 1ull << 20, 3628800ull, 12700800ull})
         for (int prec : {F64, F32})
