@@ -432,7 +432,7 @@ int exec_device(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range
         // back, so a large one is stored non-temporally (the host path's staged chunks are
         // copied out right after, and stay cached)
         r.nb = p->batch;
-        r.nt = nt_output((size_t)p->dist * p->batch * elem_bytes(p->prec));
+        r.nt = p->nt < 0 ? nt_output((size_t)p->dist * p->batch * elem_bytes(p->prec)) : p->nt != 0;
     }
     if (!p->real || p->split_fused) return run_c2c(p, in, out, s, r);
     if (!p->inverse) {

@@ -255,6 +255,7 @@ struct gfftx_plan_s {
     unsigned long long dist = 0;   // complex elements between batch items
     RealPart real_part() const { return RealPart{!real ? REAL_NONE : inverse ? REAL_PRE : REAL_POST, inverse && place == GFFTX_OUT_OF_PLACE}; }
     bool through = true;           // passes may store through the L2 (GFFTX_THROUGH_STORE when the plan was made)
+    int nt = -1;                   // the last pass stores non-temporally: by the call's size (-1), or fixed
     std::vector<int> forced_lens;  // plan choice made by the autotuner (empty: cost model), see split_choice
     std::string tune_note;         // autotuner record for plan_describe
     std::vector<Pass> passes;
@@ -372,7 +373,7 @@ int exec_host(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, bool di
 // --- tuner.cpp: plan creation with the measured autotuner
 int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
                 uint32_t flags);
-bool tune_length_class(int device, int prec, long long L, long long count, bool inverse, bool* single,
+bool tune_length_class(int device, int prec, long long L, long long count, bool inverse, bool nt, bool* single,
                        std::vector<int>* lens, std::vector<std::pair<int, int>>* tiles);
 int fill_reps(int prec, unsigned long long n);
 // cache entries of other choices (the ragged batch's persistent-kernel limit)

@@ -64,7 +64,7 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
     std::vector<int> t_lens;
     std::vector<std::pair<int, int>> t_tiles;  // (nb, wg) per pass, (0, 0) = the default tile
     if (!(r->flags & GFFTX_FLAG_NO_AUTOTUNE) && !getenv("GFFTX_RAGGED_MIN_SINGLE") && !getenv("GFFTX_PASSES") &&
-        tune_length_class(r->device, r->prec, L, lc.count, r->inverse, &t_single, &t_lens, &t_tiles)) {
+        tune_length_class(r->device, r->prec, L, lc.count, r->inverse, r->args.nt_out != 0, &t_single, &t_lens, &t_tiles)) {
         if (t_single && k1) {
             use_single = true;
             k1 = find_tile(r->prec, (int)L, false, false, t_tiles.empty() ? 0 : t_tiles[0].first,

@@ -150,7 +150,7 @@ void tune_put(const std::string& key, const std::vector<int>& v)
 
 // Revision of the kernels the cached choices were measured with: part of every key, so that a
 // cache file written by a library with other tiles is measured afresh, not taken over.
-static constexpr int kTuneRevision = 4;
+static constexpr int kTuneRevision = 5;
 
 std::string tune_key(int device, int prec, uint64_t n, uint64_t batch)
 {
@@ -255,6 +255,100 @@ static bool fill_numbers(int prec, void* dst, size_t bytes, hipStream_t s)
         ok = hipMemcpyAsync((char*)dst + n, dst, std::min(n, bytes - n), hipMemcpyDeviceToDevice, s) == hipSuccess;
     return hipStreamSynchronize(s) == hipSuccess && ok;  // before the host arrays go
 }
+
+// Arrays and stream the candidates of one choice run on: up to 64 MiB three pairs of arrays that the
+// calls walk over (time_plan) and, with `passes`, three sets of intermediate ones; above, one pair of
+// numbers.  A large transform is bound by memory and by the power it takes, and on zeros it takes
+// less power (65536 x 1024 FP64, four sequences a workgroup against one: 363 and 366 us on zeros, 369
+// and 364 on numbers).
+struct TuneArrays {
+    void *a = nullptr, *b = nullptr, *alt = nullptr;
+    hipStream_t s = nullptr;
+    size_t bytes = 0;
+    int sets = 1;
+    const void* fill = nullptr;
+
+    // false: no room for the arrays a call needs
+    bool make(int prec, size_t want, bool inplace, bool passes)
+    {
+        bytes = (want + 255) / 256 * 256;
+        sets = bytes <= (64u << 20) ? 3 : 1;
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess || hipMalloc(&a, bytes * sets) != hipSuccess ||
+            (!inplace && hipMalloc(&b, bytes * sets) != hipSuccess)) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (sets > 1 && passes && hipMalloc(&alt, bytes * 2 * (sets - 1)) != hipSuccess) alt = nullptr;
+        if (sets == 1 && inplace && hipMalloc(&b, bytes) != hipSuccess) b = nullptr;  // (then on zeros)
+        // all of it on `s`: that stream does not wait for the null stream
+        (void)hipMemsetAsync(a, 0, bytes * sets, s);
+        if (sets == 1 && b && fill_numbers(prec, b, bytes, s) &&
+            hipMemcpyAsync(a, b, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess)
+            fill = inplace ? b : nullptr;
+        (void)hipGetLastError();
+        return true;
+    }
+    int time(gfftx_plan_s* p, int reps, float* ms) const
+    {
+        return time_plan(p, a, p->place == GFFTX_IN_PLACE ? a : b, s, reps, ms, sets, bytes, alt, fill, bytes);
+    }
+    ~TuneArrays()
+    {
+        if (s) {
+            (void)hipStreamSynchronize(s);
+            (void)hipStreamDestroy(s);
+        }
+        for (void* p : {a, b, alt})
+            if (p) (void)hipFree(p);
+        (void)hipGetLastError();
+    }
+};
+
+// The candidates of one choice, timed on `arrays`; `make` builds one (null: it cannot be built).
+struct TuneRun {
+    const TuneArrays& arrays;
+    std::function<gfftx_plan(const std::vector<int>&)> make;
+    std::vector<std::pair<float, std::vector<int>>> timed;
+    std::vector<int> chosen;  // the fastest so far
+    float best = 1e30f;
+
+    // ms of one execution, or -1
+    float time(const std::vector<int>& c)
+    {
+        gfftx_plan p = make(c);
+        if (!p) return -1.f;
+        float ms = 0;
+        const int rc = arrays.time(p, 5, &ms);
+        gfftx_plan_destroy(p);
+        if (rc) return -1.f;
+        timed.push_back({ms, c});
+        if (ms < best) {
+            best = ms;
+            chosen = c;
+        }
+        return ms;
+    }
+    // the fastest few once more, in turn, on plans that stay: a single timing of a short transform
+    // moves by more than the candidates differ
+    void again(size_t few)
+    {
+        std::vector<std::pair<float, std::vector<int>>> top = timed;
+        std::stable_sort(top.begin(), top.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+        top.resize(std::min<size_t>(top.size(), arrays.bytes <= (64u << 20) ? few : 2));
+        if (top.size() < 2) return;
+        std::vector<gfftx_plan> tp;
+        std::vector<float> tms(top.size(), 1e30f);
+        for (const auto& t : top) tp.push_back(make(t.second));
+        for (int rep = 0; rep < 3; ++rep)
+            for (size_t i = 0; i < top.size(); ++i) {
+                float ms = 0;
+                if (tp[i] && arrays.time(tp[i], 10, &ms) == GFFTX_SUCCESS) tms[i] = std::min(tms[i], ms);
+            }
+        const size_t w = std::min_element(tms.begin(), tms.end()) - tms.begin();
+        if (tms[w] < 1e30f) chosen = top[w].second;
+        for (gfftx_plan q : tp) gfftx_plan_destroy(q);
+    }
+};
 
 // The cost model's best `k` splits, and its best three of compiled tiles alone where they are
 // not among them.
@@ -397,49 +491,24 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         // the 256 MB Infinity Cache, so the timings see HBM as the plan will
         const size_t item_bytes = (size_t)p->dist * elem_bytes(p->prec);
         const uint64_t tbatch = std::min<uint64_t>(batch, std::max<uint64_t>(1, (1ull << 30) / item_bytes));
-        const size_t bytes = (item_bytes * tbatch + 255) / 256 * 256;
-        const int sets = bytes <= (64u << 20) ? 3 : 1;
-        void *a = nullptr, *b = nullptr;
-        if (hipMalloc(&a, bytes * sets) != hipSuccess || hipMalloc(&b, bytes * sets) != hipSuccess) {
-            (void)hipGetLastError();
-            if (a) (void)hipFree(a);
-            return GFFTX_SUCCESS;  // no room to tune: keep the cost-model plan
-        }
-        void* alt = nullptr;
-        if (sets > 1 && !single_pass && !chirp && hipMalloc(&alt, bytes * 2 * (sets - 1)) != hipSuccess) {
-            (void)hipGetLastError();
-            alt = nullptr;
-        }
-        hipStream_t s = nullptr;
-        (void)hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-        (void)hipMemsetAsync(a, 0, bytes * sets, s);
-        // a large transform is bound by memory and by the power it takes, and on zeros it takes less
-        // power, so it is timed on numbers between -1 and 1 (65536 x 1024 FP64, four sequences a
-        // workgroup against one: 363 and 366 us on zeros, 369 and 364 on numbers)
-        const void* fill = nullptr;
-        // (all of it on `s`: that stream does not wait for the null stream)
-        if (sets == 1 && fill_numbers(p->prec, b, bytes, s) &&
-            hipMemcpyAsync(a, b, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess)
-            fill = place == GFFTX_IN_PLACE ? b : nullptr;
-        float best = 1e30f;
+        TuneArrays arrays;
+        // no room to tune: keep the cost-model plan
+        if (!arrays.make(p->prec, item_bytes * tbatch, place == GFFTX_IN_PLACE, !single_pass && !chirp)) return GFFTX_SUCCESS;
+        // the candidates are the plan's own transform (a real forward plan times its last pass with the
+        // R2C split fused in) with its own placement: an in-place plan runs on one buffer, which the caches
+        // treat differently from two; the arrays cover the bins layout
+        TuneRun run{arrays, [&](const std::vector<int>& c) {
+            gfftx_plan cp = nullptr;
+            (void)create_plan_impl(&cp, n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, c, "");
+            return cp;
+        }};
         std::string timings = ",\"tuned\":[";
         size_t ntimed = 0;
         std::vector<float> cms(cands.size(), -1.f);  // time of each candidate (-1: failed)
-        std::vector<std::pair<float, std::vector<int>>> timed;
-        // time one candidate, record it in `timings`, keep it if it is the fastest so far
+        // time one candidate and record it in `timings`
         auto try_cand = [&](const std::vector<int>& c) -> float {
-            gfftx_plan cp = nullptr;
-            // the candidates are the plan's own transform (a real forward plan times its last
-            // pass with the R2C split fused in) with its own placement: an in-place plan runs
-            // on one buffer, which the caches treat differently from two; `bytes` covers the
-            // bins layout
-            if (create_plan_impl(&cp, n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, c, "") !=
-                GFFTX_SUCCESS)
-                return -1.f;
-            float ms = 0;
-            const int trc = time_plan(cp, a, place == GFFTX_IN_PLACE ? a : b, s, 5, &ms, sets, bytes, alt, fill, bytes);
-            gfftx_plan_destroy(cp);
-            if (trc) return -1.f;
+            const float ms = run.time(c);
+            if (ms < 0) return ms;
             std::vector<int> sl;
             std::vector<std::pair<int, int>> tl;
             split_choice(c, sl, tl);
@@ -455,18 +524,13 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             char buf[160];
             snprintf(buf, sizeof(buf), "%s{\"split\":\"%s\",\"ms\":%.4f}", ntimed++ ? "," : "", lens.c_str(), ms);
             timings += buf;
-            if (ms < best) {
-                best = ms;
-                chosen = c;
-            }
-            timed.push_back({ms, c});
             return ms;
         };
         for (size_t i = 0; i < cands.size(); ++i) cms[i] = try_cand(cands[i]);
-        if (chirp && !chosen.empty()) {
+        if (chirp && !run.chosen.empty()) {
             for (size_t i = 0; i < 5; ++i)
-                for (const std::vector<int>& c : chirp_variants(p->prec, n, chosen, i)) try_cand(c);
-        } else if (!chosen.empty() && chosen[1] != 1) {
+                for (const std::vector<int>& c : chirp_variants(p->prec, n, run.chosen, i)) try_cand(c);
+        } else if (!run.chosen.empty() && run.chosen[1] != 1) {
             // the combination of the fastest variants, for each of the three fastest splits
             std::vector<size_t> order(cands.size());
             for (size_t i = 0; i < order.size(); ++i) order[i] = i;
@@ -483,33 +547,9 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
                 if (seen.size() == 3) break;
             }
         }
-        // the fastest few once more, in turn, on plans that stay: a single timing of a short transform
-        // moves by more than the candidates differ
-        std::vector<std::pair<float, std::vector<int>>> top = timed;
-        std::stable_sort(top.begin(), top.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-        top.resize(std::min<size_t>(top.size(), bytes <= (64u << 20) ? 6 : 2));
-        if (top.size() > 1) {
-            std::vector<gfftx_plan> tp(top.size(), nullptr);
-            std::vector<float> tms(top.size(), 1e30f);
-            for (size_t i = 0; i < top.size(); ++i)
-                (void)create_plan_impl(&tp[i], n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, top[i].second, "");
-            for (int rep = 0; rep < 3; ++rep)
-                for (size_t i = 0; i < top.size(); ++i) {
-                    float ms = 0;
-                    if (tp[i] && time_plan(tp[i], a, place == GFFTX_IN_PLACE ? a : b, s, 10, &ms, sets, bytes, alt, fill, bytes) == GFFTX_SUCCESS)
-                        tms[i] = std::min(tms[i], ms);
-                }
-            const size_t w = std::min_element(tms.begin(), tms.end()) - tms.begin();
-            if (tms[w] < 1e30f) chosen = top[w].second;
-            for (gfftx_plan q : tp) gfftx_plan_destroy(q);
-        }
+        run.again(6);
         timings += "]";
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
-        (void)hipFree(a);
-        (void)hipFree(b);
-        if (alt) (void)hipFree(alt);
-        (void)hipGetLastError();
+        chosen = run.chosen;
         if (chosen.empty()) return GFFTX_SUCCESS;
         note = timings;
         std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -526,11 +566,12 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
 
 // Plan choice for one length class of a ragged batch (count transforms of length L): every
 // compiled single-pass tile of the length against the cost model's best three pass splits,
-// each timed on a contiguous batch of the class's size.  Returns false when nothing was
+// each timed on a contiguous batch of the class's size, stored the way the class stores: plainly, and
+// non-temporally at the end where the whole batch is (`nt`).  Returns false when nothing was
 // measured (autotuning off, or no buffers), and the caller keeps its built-in rule.  Cached
 // like plans, under the class's own key; a single-pass choice is stored as [L, 1, 0, nb, wg]
 // and returned with *single set and the tile's shape in *nb, *wg.
-bool tune_length_class(int device, int prec, long long L, long long count, bool inverse, bool* single,
+bool tune_length_class(int device, int prec, long long L, long long count, bool inverse, bool nt, bool* single,
                        std::vector<int>* lens, std::vector<std::pair<int, int>>* tiles)
 {
     if (env_int("GFFTX_AUTOTUNE", 1) == 0) return false;
@@ -538,7 +579,7 @@ bool tune_length_class(int device, int prec, long long L, long long count, bool 
     const std::vector<std::vector<int>> splits = tuned_splits(prec, (unsigned long long)L, 3, (unsigned long long)count,
                                                               device_cus(device));
     if ((has_single ? 1 : 0) + splits.size() < 2) return false;
-    const std::string key = tune_key(device, prec, (uint64_t)L, (uint64_t)count) + "|class";
+    const std::string key = tune_key(device, prec, (uint64_t)L, (uint64_t)count) + (nt ? "|class|nt" : "|class");
     std::vector<int> chosen;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -557,46 +598,28 @@ bool tune_length_class(int device, int prec, long long L, long long count, bool 
         // at most 1 GiB of data, like plan tuning
         const uint64_t tcount = std::min<uint64_t>((uint64_t)count,
                                                    std::max<uint64_t>(1, (1ull << 30) / ((size_t)L * elem_bytes(prec))));
-        const size_t bytes = (size_t)L * tcount * elem_bytes(prec);
-        void* a = nullptr;
-        if (hipMalloc(&a, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        hipStream_t s = nullptr;
-        (void)hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-        (void)hipMemsetAsync(a, 0, bytes, s);
+        TuneArrays arrays;
+        // (in place, as the classes of a ragged batch run)
+        if (!arrays.make(prec, (size_t)L * tcount * elem_bytes(prec), true, true)) return false;
         const int cvt = prec == PREC_F64 ? GFFTX_COMPLEX_DOUBLE : GFFTX_COMPLEX_FLOAT;
-        float best = 1e30f;
-        bool found = false;
-        auto try_cand = [&](const std::vector<int>& c) -> float {
+        TuneRun run{arrays, [&](const std::vector<int>& c) {
             gfftx_plan cp = nullptr;
-            // in place, as the classes of a ragged batch run
-            if (create_plan_impl(&cp, (uint64_t)L, tcount, cvt, inverse ? GFFTX_IDFT : GFFTX_DFT, GFFTX_IN_PLACE,
-                                 device, GFFTX_FLAG_NO_AUTOTUNE, c, "") != GFFTX_SUCCESS)
-                return -1.f;
-            float ms = 0;
-            const int trc = time_plan(cp, a, a, s, 5, &ms);
-            gfftx_plan_destroy(cp);
-            if (trc) return -1.f;
-            if (ms < best) {
-                best = ms;
-                chosen = c;
-                found = true;
+            if (create_plan_impl(&cp, (uint64_t)L, tcount, cvt, inverse ? GFFTX_IDFT : GFFTX_DFT, GFFTX_IN_PLACE, device,
+                                 GFFTX_FLAG_NO_AUTOTUNE, c, "") == GFFTX_SUCCESS) {
+                cp->through = false;
+                cp->nt = nt ? 1 : 0;
             }
-            return ms;
-        };
+            return cp;
+        }};
         std::vector<float> cms(cands.size(), -1.f);
-        for (size_t i = 0; i < cands.size(); ++i) cms[i] = try_cand(cands[i]);
-        if (found && !(chosen.size() >= 2 && chosen[1] == 1 && chosen[0] == (int)L)) {
-            const std::vector<int> combo = best_combination(chosen, cands, cms);
-            if (!combo.empty()) try_cand(combo);
+        for (size_t i = 0; i < cands.size(); ++i) cms[i] = run.time(cands[i]);
+        if (run.chosen.empty()) return false;
+        if (!(run.chosen[1] == 1 && run.chosen[0] == (int)L)) {
+            const std::vector<int> combo = best_combination(run.chosen, cands, cms);
+            if (!combo.empty()) run.time(combo);
         }
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
-        (void)hipFree(a);
-        (void)hipGetLastError();
-        if (!found) return false;
+        run.again(3);  // (a batch may have dozens of classes)
+        chosen = run.chosen;
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tune[key] = chosen;
         tune_store();
