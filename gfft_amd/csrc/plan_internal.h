@@ -376,6 +376,7 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
 bool tune_length_class(int device, int prec, long long L, long long count, bool inverse, bool nt, bool* single,
                        std::vector<int>* lens, std::vector<std::pair<int, int>>* tiles);
 int fill_reps(int prec, unsigned long long n);
+std::string choice_label(const std::vector<int>& c, bool chirp);
 // cache entries of other choices (the ragged batch's persistent-kernel limit)
 std::string ragged_tune_key(int device, int prec, const uint64_t* lengths, uint64_t count);
 bool tune_get(const std::string& key, std::vector<int>* v);

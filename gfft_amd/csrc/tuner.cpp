@@ -431,6 +431,45 @@ static std::vector<int> best_combination(const std::vector<int>& chosen, const s
     return combo;
 }
 
+// A choice as describe() names it: the pass lengths, each with /nb-wg where the choice names the tile,
+// or single/nb-wg; for a chirp-z plan the convolution length m first, then all of its passes (a split of
+// m into k lengths runs in 2k - 1).
+std::string choice_label(const std::vector<int>& c, bool chirp)
+{
+    std::vector<int> l;
+    std::vector<std::pair<int, int>> t;
+    split_choice(c, l, t);
+    std::string s;
+    if (chirp && l.size() > 1) {
+        s = std::to_string(l[0]) + ": ";
+        l.erase(l.begin());
+        if (l.size() > 1)
+            for (size_t i = l.size() - 1; i-- > 0;) l.push_back(l[i]);
+    } else if (l.size() == 2 && l[1] == 1) {
+        l.erase(l.begin());
+    }
+    for (size_t j = 0; j < l.size(); ++j) {
+        s += (j ? "x" : "") + (l.size() == 1 && l[0] == 1 ? std::string("single") : std::to_string(l[j]));
+        if (j < t.size() && t[j].first) s += "/" + std::to_string(t[j].first) + "-" + std::to_string(t[j].second);
+    }
+    return s;
+}
+
+// The candidates timed, for describe(): the fastest 32, fastest first (a length with many divisors
+// has over a hundred, more than describe()'s callers have room for).
+static std::string tune_note(std::vector<std::pair<float, std::vector<int>>> timed, bool chirp)
+{
+    std::stable_sort(timed.begin(), timed.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+    timed.resize(std::min<size_t>(timed.size(), 32));
+    std::string s = ",\"tuned\":[";
+    for (size_t i = 0; i < timed.size(); ++i) {
+        char ms[32];
+        snprintf(ms, sizeof(ms), "%.4f", timed[i].first);
+        s += std::string(i ? "," : "") + "{\"split\":\"" + choice_label(timed[i].second, chirp) + "\",\"ms\":" + ms + "}";
+    }
+    return s + "]";
+}
+
 int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
                 uint32_t flags)
 {
@@ -502,34 +541,11 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
             (void)create_plan_impl(&cp, n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, c, "");
             return cp;
         }};
-        std::string timings = ",\"tuned\":[";
-        size_t ntimed = 0;
         std::vector<float> cms(cands.size(), -1.f);  // time of each candidate (-1: failed)
-        // time one candidate and record it in `timings`
-        auto try_cand = [&](const std::vector<int>& c) -> float {
-            const float ms = run.time(c);
-            if (ms < 0) return ms;
-            std::vector<int> sl;
-            std::vector<std::pair<int, int>> tl;
-            split_choice(c, sl, tl);
-            std::string lens;
-            if (sl.size() == 2 && sl[1] == 1) {
-                lens = "single/" + std::to_string(tl[0].first) + "-" + std::to_string(tl[0].second);
-            } else {
-                for (size_t j = 0; j < sl.size(); ++j) {
-                    lens += (j ? "x" : "") + std::to_string(sl[j]);
-                    if (j < tl.size() && tl[j].first) lens += "/" + std::to_string(tl[j].first) + "-" + std::to_string(tl[j].second);
-                }
-            }
-            char buf[160];
-            snprintf(buf, sizeof(buf), "%s{\"split\":\"%s\",\"ms\":%.4f}", ntimed++ ? "," : "", lens.c_str(), ms);
-            timings += buf;
-            return ms;
-        };
-        for (size_t i = 0; i < cands.size(); ++i) cms[i] = try_cand(cands[i]);
+        for (size_t i = 0; i < cands.size(); ++i) cms[i] = run.time(cands[i]);
         if (chirp && !run.chosen.empty()) {
             for (size_t i = 0; i < 5; ++i)
-                for (const std::vector<int>& c : chirp_variants(p->prec, n, run.chosen, i)) try_cand(c);
+                for (const std::vector<int>& c : chirp_variants(p->prec, n, run.chosen, i)) run.time(c);
         } else if (!run.chosen.empty() && run.chosen[1] != 1) {
             // the combination of the fastest variants, for each of the three fastest splits
             std::vector<size_t> order(cands.size());
@@ -543,15 +559,14 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
                 if (cms[i] < 0 || (l.size() == 2 && l[1] == 1) || std::find(seen.begin(), seen.end(), l) != seen.end()) continue;
                 seen.push_back(l);
                 const std::vector<int> combo = best_combination(cands[i], cands, cms);
-                if (!combo.empty()) try_cand(combo);
+                if (!combo.empty()) run.time(combo);
                 if (seen.size() == 3) break;
             }
         }
+        note = tune_note(run.timed, chirp);
         run.again(6);
-        timings += "]";
         chosen = run.chosen;
         if (chosen.empty()) return GFFTX_SUCCESS;
-        note = timings;
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tune[key] = chosen;
         tune_store();

@@ -5,6 +5,7 @@
 //   - the search for the best few splits finds what listing them all would;
 //   - passes store the way that was measured fastest for their kind, rows and size;
 //   - the autotuner's repeated in-place transforms stay in the range of their numbers;
+//   - describe() names a tuned choice in full;
 //   - a length runs natively exactly where a tile or a split exists.
 #include <cstdio>
 
@@ -130,6 +131,23 @@ int main()
                 printf("FAIL prec %d n %llu: %d transforms in place\n", prec, n, r);
                 ++fails;
             }
+        }
+    // a choice's name shows every pass with its own tile
+    const struct {
+        std::vector<int> c;
+        bool chirp;
+        const char* want;
+    } names[] = {{{1000, 1, 0, 2, 256}, false, "single/2-256"},
+                 {{512, 256}, false, "512x256"},
+                 {{512, 256, 0, 4, 128, 0, 0}, false, "512/4-128x256"},
+                 {{2048, 1, 0, 1, 128}, true, "2048: single/1-128"},
+                 {{131220, 324, 405, 0, 2, 128, 4, 64, 2, 192}, true, "131220: 324/2-128x405/4-64x324/2-192"},
+                 {{8388608, 128, 256, 256, 0, 16, 128, 16, 256, 8, 129, 16, 512, 32, 64}, true,
+                  "8388608: 128/16-128x256/16-256x256/8-129x256/16-512x128/32-64"}};
+    for (const auto& x : names)
+        if (choice_label(x.c, x.chirp) != x.want) {
+            printf("FAIL label %s, not %s\n", choice_label(x.c, x.chirp).c_str(), x.want);
+            ++fails;
         }
     // pruned search against the full list
     for (unsigned long long n : {4096ull, 20000ull, 44100ull, 362880ull, 1ull << 20, 3628800ull, 12700800ull})

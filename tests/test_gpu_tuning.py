@@ -31,3 +31,18 @@ def test_ragged_classes_tuned_with_the_stores_they_run_with(torch_cuda, tmp_path
         off += n
     keys = [k for k in json.loads(cache.read_text())["entries"] if "|class" in k]
     assert len(keys) == 3 and all(k.endswith(suffix) for k in keys), keys
+
+
+@pytest.mark.parametrize("n,ttype", [(3628800, api.DFT), (3628800, api.IRDFT), (65537, api.DFT)])
+def test_describe_lists_the_fastest_candidates(torch_cuda, tmp_path, monkeypatch, n, ttype):
+    """Dozens of candidates: describe() has room for its list, and no two of them read alike."""
+    monkeypatch.setenv("GFFTX_TUNE_CACHE", str(tmp_path / "tune.json"))
+    monkeypatch.setenv("GFFTX_TUNE_CANDIDATES", "20")
+    with api.Plan(n, api.COMPLEX_FLOAT, ttype, api.OUT_OF_PLACE) as p:
+        d = json.loads(p.describe())
+    splits, ms = [t["split"] for t in d["tuned"]], [t["ms"] for t in d["tuned"]]
+    assert 2 <= len(splits) <= 32 and ms == sorted(ms)
+    assert len(set(splits)) == len(splits)
+    if n == 65537:
+        m = [int(s.split(":")[0]) for s in splits]
+        assert all(v >= 2 * n - 1 for v in m) and all(s.count("x") == 2 and s.count("/") == 3 for s in splits)
