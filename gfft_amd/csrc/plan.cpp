@@ -10,6 +10,8 @@
 // (src/gfftalg.h:249-261); tables avoid the recurrence's error growth.
 #include "plan_internal.h"
 
+#include <system_error>
+
 namespace gfftx {
 namespace detail {
 
@@ -224,34 +226,54 @@ int build_c2c_passes(gfftx_plan_s* p)
     return GFFTX_SUCCESS;
 }
 
-int upload_split_table(gfftx_plan_s* p)
+// W_{2n}^k, k = 0..n/2 (n even), in the working precision.  Entries above n/4 mirror those below
+// (root_ld folds an angle to the first octant, so the bits are those of an evaluation), and the
+// others are shared out to up to 8 threads: 2^24 + 1 entries took one thread 3.8 s.
+template <typename T> std::vector<T> split_roots(long long n)
 {
-    const long long n = (long long)p->n;
-    const long long cnt = n / 2 + 1;
-    if (p->prec == PREC_F64) {
-        std::vector<double> t(2 * cnt);
-        for (long long k = 0; k < cnt; ++k) {
+    std::vector<T> t(2 * (n / 2 + 1));
+    const long long direct = n / 4 + 1;  // k <= n/4
+    auto part = [&](long long lo, long long hi) {
+        for (long long k = lo; k < hi; ++k) {
             long double c, s;
             root_ld(k, 2 * n, &c, &s);
-            t[2 * k] = (double)c;
-            t[2 * k + 1] = (double)s;
+            t[2 * k] = (T)c;
+            t[2 * k + 1] = (T)s;
         }
-        int rc = dev_alloc(p, &p->split_tw, t.size() * sizeof(double));
-        if (rc) return rc;
-        HIP_TRY(hipMemcpy(p->split_tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-    } else {
-        std::vector<float> t(2 * cnt);
-        for (long long k = 0; k < cnt; ++k) {
-            long double c, s;
-            root_ld(k, 2 * n, &c, &s);
-            t[2 * k] = (float)c;
-            t[2 * k + 1] = (float)s;
+    };
+    const long long want = std::min<long long>({8, std::max(1u, std::thread::hardware_concurrency()), direct >> 15});
+    std::vector<std::thread> th;
+    long long done = 0;
+    for (long long i = 1; i < want; ++i) {
+        const long long hi = direct * i / want;
+        try {
+            th.emplace_back(part, done, hi);
+        } catch (const std::system_error&) {
+            break;  // no more threads: the rest below
         }
-        int rc = dev_alloc(p, &p->split_tw, t.size() * sizeof(float));
-        if (rc) return rc;
-        HIP_TRY(hipMemcpy(p->split_tw, t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice));
+        done = hi;
     }
-    return GFFTX_SUCCESS;
+    part(done, direct);
+    for (auto& x : th) x.join();
+    for (long long k = direct; k <= n / 2; ++k) {
+        t[2 * k] = -t[2 * (n / 2 - k) + 1];
+        t[2 * k + 1] = -t[2 * (n / 2 - k)];
+    }
+    return t;
+}
+template std::vector<float> split_roots<float>(long long n);
+template std::vector<double> split_roots<double>(long long n);
+
+int upload_split_table(std::vector<void*>& owned, int prec, long long n, void** out)
+{
+    auto up = [&](const auto& t) -> int {
+        const size_t bytes = t.size() * sizeof(t[0]);
+        const int rc = dev_alloc_list(owned, out, bytes);
+        if (rc) return rc;
+        HIP_TRY(hipMemcpy(*out, t.data(), bytes, hipMemcpyHostToDevice));
+        return GFFTX_SUCCESS;
+    };
+    return prec == PREC_F64 ? up(split_roots<double>(n)) : up(split_roots<float>(n));
 }
 
 bool is_device_ptr(const void* ptr)
@@ -518,7 +540,7 @@ int exec_any(gfftx_plan_s* p, const void* in, void* out, hipStream_t s)
 }
 
 int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
-                     uint32_t flags, const std::vector<int>& forced, const std::string& note)
+                     uint32_t flags, const std::vector<int>& forced, const std::string& note, SplitTable* lent)
 {
     if (!out) return fail(GFFTX_ERR_INVALID_ARG, "plan pointer is NULL");
     *out = nullptr;
@@ -566,7 +588,14 @@ int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int
     int rc = native_length(p->prec, n) ? build_c2c_passes(p) : build_bluestein(p);
     // an unfused split runs as a kernel of its own with a table; that of an out-of-place
     // IRDFT works on a copy of the input
-    if (rc == GFFTX_SUCCESS && real && !p->split_fused) rc = upload_split_table(p);
+    if (rc == GFFTX_SUCCESS && real && !p->split_fused) {
+        if (!lent) {
+            rc = upload_split_table(p->allocs, p->prec, (long long)n, &p->split_tw);
+        } else {
+            if (!lent->tw) rc = upload_split_table(lent->owned, p->prec, (long long)n, &lent->tw);
+            p->split_tw = lent->tw;
+        }
+    }
     if (rc == GFFTX_SUCCESS && real && p->inverse && !p->split_fused)
         rc = dev_alloc(p, &p->real_work, (size_t)p->dist * batch * elem_bytes(p->prec));
     if (rc == GFFTX_SUCCESS && p->passes.size() > 1) {

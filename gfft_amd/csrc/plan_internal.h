@@ -351,8 +351,19 @@ namespace detail {
 
 // --- plan.cpp: plan construction and execution
 int dev_alloc(gfftx_plan_s* p, void** out, size_t bytes);
+// The table of an unfused real split, lent to the candidates of one tuning run: made by the first
+// that needs it, freed with this (after them).
+struct SplitTable {
+    void* tw = nullptr;
+    std::vector<void*> owned;
+    ~SplitTable()
+    {
+        for (void* p : owned) (void)hipFree(p);
+    }
+};
+template <typename T> std::vector<T> split_roots(long long n);
 int create_plan_impl(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttype, int place, int device,
-                     uint32_t flags, const std::vector<int>& forced, const std::string& note);
+                     uint32_t flags, const std::vector<int>& forced, const std::string& note, SplitTable* lent = nullptr);
 int exec_device(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r = Range());
 int run_passes(gfftx_plan_s* p, const void* in, void* out, hipStream_t s, Range r);
 bool prof_begin(gfftx_plan_s* p, size_t slot, const char* name, hipStream_t s, std::pair<hipEvent_t, hipEvent_t>* ev,

@@ -536,9 +536,11 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         // the candidates are the plan's own transform (a real forward plan times its last pass with the
         // R2C split fused in) with its own placement: an in-place plan runs on one buffer, which the caches
         // treat differently from two; the arrays cover the bins layout
+        SplitTable split;
+        split.tw = p->split_tw;
         TuneRun run{arrays, [&](const std::vector<int>& c) {
             gfftx_plan cp = nullptr;
-            (void)create_plan_impl(&cp, n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, c, "");
+            (void)create_plan_impl(&cp, n, tbatch, vtype, ttype, place, device, flags & GFFTX_FLAG_R2C_BINS, c, "", &split);
             return cp;
         }};
         std::vector<float> cms(cands.size(), -1.f);  // time of each candidate (-1: failed)

@@ -6,6 +6,7 @@
 //   - passes store the way that was measured fastest for their kind, rows and size;
 //   - the autotuner's repeated in-place transforms stay in the range of their numbers;
 //   - describe() names a tuned choice in full;
+//   - the table of an unfused real split holds the roots, bit for bit;
 //   - a length runs natively exactly where a tile or a split exists.
 #include <cstdio>
 
@@ -149,6 +150,21 @@ int main()
             printf("FAIL label %s, not %s\n", choice_label(x.c, x.chirp).c_str(), x.want);
             ++fails;
         }
+    // the split table's mirrored and shared-out entries are the roots themselves
+    for (long long n : {2ll, 4ll, 6ll, 10ll, 12ll, 98ll, 1000ll, 4096ll, 200000ll, 524290ll}) {
+        const std::vector<float> f = split_roots<float>(n);
+        const std::vector<double> d = split_roots<double>(n);
+        bool ok = f.size() == (size_t)n + 2 && d.size() == (size_t)n + 2;
+        for (long long k = 0; ok && k <= n / 2; ++k) {
+            long double c, s;
+            root_ld(k, 2 * n, &c, &s);
+            ok = f[2 * k] == (float)c && f[2 * k + 1] == (float)s && d[2 * k] == (double)c && d[2 * k + 1] == (double)s;
+        }
+        if (!ok) {
+            printf("FAIL split table of %lld\n", n);
+            ++fails;
+        }
+    }
     // pruned search against the full list
     for (unsigned long long n : {4096ull, 20000ull, 44100ull, 362880ull, 1ull << 20, 3628800ull, 12700800ull})
         for (int prec : {F64, F32})
