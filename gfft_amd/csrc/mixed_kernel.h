@@ -54,7 +54,7 @@ struct MixShape {
     unsigned ts;              // LDS distance between sequences
     unsigned pad;             // LDS pad elements after every R_0 elements: 0 or 1
     unsigned nst;
-    int nt_in;                // 1: rows are whole 128-byte lines, the input is loaded non-temporally
+    int nt_in;                // 1: rows of L (T modes: nb) elements are whole 128-byte lines, the input is loaded non-temporally
     MixStage st[MIX_STAGES];
 };
 

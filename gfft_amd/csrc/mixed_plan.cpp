@@ -157,6 +157,10 @@ bool fill(MixTile& t, int prec, int L, bool loadT, bool storeT, int real, int nb
         if (s) tw += prec == PREC_F64 ? ns * (r[s] - 1) : ns;
         ns *= r[s];
     }
+    // (a CHIRP_ALL tile's L is the convolution length, its input rows are shorter.  Whole lines are not what
+    // decides there: non-temporal against plain loads, 8192 x 1009 FP32 on rotating arrays above the
+    // Infinity Cache 63.2 and 65.4 us, 32768 x 1009 230 and 238, the same for 1012 and its half lines;
+    // with the input in that cache 8192 x 1104, whole lines, 76.6 and 72.9, 8192 x 1009 FP64 129 and 121)
     const size_t row = (loadT ? (size_t)nb : (size_t)nb * L) * eb;
     m.nt_in = row % 128 == 0 ? 1 : 0;
     const size_t lds = r.size() > 1 ? (size_t)nb * m.ts * eb : 0;

@@ -28,10 +28,10 @@ struct TileEntry {
     TileLaunch launch;
     const char* name;
     int real;  // REAL_NONE, or the real-transform split fused in (REAL_POST, REAL_PRE: RealCfg)
-    const MixShape* mix = nullptr;  // run-time mixed-radix tile (mixed.hip; `launch` is null)
+    const MixShape* mix = nullptr;  // run-time mixed-radix tile (mixed.cpp; `launch` is null)
 };
 
-// Run-time mixed-radix tiles (mixed.hip).  mixed_prepare lifts the kernel's limit on dynamic
+// Run-time mixed-radix tiles (mixed.cpp).  mixed_prepare lifts the kernel's limit on dynamic
 // LDS; it is called once per shape, when a plan is made.
 hipError_t mixed_prepare(const TileEntry& k);
 hipError_t launch_mixed(const TileEntry& k, const TileArgs& a, dim3 grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1,
