@@ -108,9 +108,9 @@ struct RealPart {
 
 double split_cost(const RealPart& real, const TileEntry* k, unsigned long long n, unsigned long long batch);
 const TileEntry* pass_tile(int prec, int L, unsigned long long ns, unsigned long long n, unsigned long long batch, int cus,
-                           double* cost = nullptr);
+                           double* cost = nullptr, bool any = false);
 std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch = 1,
-                                               int cus = 256, bool mixed = true, RealPart real = RealPart());
+                                               int cus = 256, bool mixed = true, RealPart real = RealPart(), bool any = false);
 void split_choice(const std::vector<int>& c, std::vector<int>& lens, std::vector<std::pair<int, int>>& tiles);
 int xcd_remap(const TileEntry* k, int prec);
 bool native_length(int prec, unsigned long long n);
@@ -387,6 +387,8 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
 bool tune_length_class(int device, int prec, long long L, long long count, bool inverse, bool nt, bool* single,
                        std::vector<int>* lens, std::vector<std::pair<int, int>>* tiles);
 int fill_reps(int prec, unsigned long long n);
+std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus,
+                                           RealPart real = RealPart());
 std::string choice_label(const std::vector<int>& c, bool chirp);
 // cache entries of other choices (the ragged batch's persistent-kernel limit)
 std::string ragged_tune_key(int device, int prec, const uint64_t* lengths, uint64_t count);

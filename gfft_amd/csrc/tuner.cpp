@@ -350,14 +350,26 @@ struct TuneRun {
     }
 };
 
-// The cost model's best `k` splits, and its best three of compiled tiles alone where they are
-// not among them.
-static std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus,
-                                                  RealPart real = RealPart())
+// The splits to time: the cost model's best `k` and its best three of compiled tiles alone, each length
+// counted with its cheapest tile; the best two of the fewest passes, which the model's price of a
+// stage can put behind (480000 FP32: 960 * 500 15.5 us, 768 * 25 * 25 16.4); of a real transform also the best three of its passes alone (the
+// price of a fused split is the model's least certain part: 393216 FP32 forward, 1536 * 256 fused
+// 17.1 us, the best with its split priced 19.0); and the one an untuned plan takes.
+std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus, RealPart real)
 {
-    std::vector<std::vector<int>> v = candidate_passes(prec, n, k, batch, cus, true, real);
-    for (const std::vector<int>& c : candidate_passes(prec, n, 3, batch, cus, false, real))
-        if (std::find(v.begin(), v.end(), c) == v.end()) v.push_back(c);
+    std::vector<std::vector<int>> v = candidate_passes(prec, n, k, batch, cus, true, real, true);
+    auto add = [&v](const std::vector<std::vector<int>>& more) {
+        for (const std::vector<int>& c : more)
+            if (std::find(v.begin(), v.end(), c) == v.end()) v.push_back(c);
+    };
+    add(candidate_passes(prec, n, 3, batch, cus, false, real, true));
+    std::vector<std::vector<int>> few = candidate_passes(prec, n, 40, batch, cus, true, real, true);
+    std::stable_sort(few.begin(), few.end(), [](const auto& x, const auto& y) { return x.size() < y.size(); });
+    if (few.size() > 1 && few[1].size() > few[0].size()) few.resize(1);
+    few.resize(std::min<size_t>(few.size(), 2));
+    add(few);
+    if (real.kind != REAL_NONE) add(candidate_passes(prec, n, 3, batch, cus, false, RealPart(), true));
+    add(candidate_passes(prec, n, 1, batch, cus, true, real));
     return v;
 }
 

@@ -3,6 +3,7 @@
 //   - the split an untuned plan takes is one of those measured within 15% of the fastest of its
 //     length on an MI355X (back to back, three pairs of arrays), complex and real transforms;
 //   - the search for the best few splits finds what listing them all would;
+//   - the splits a tuned plan times include those;
 //   - passes store the way that was measured fastest for their kind, rows and size;
 //   - the autotuner's repeated in-place transforms stay in the range of their numbers;
 //   - describe() names a tuned choice in full;
@@ -93,6 +94,21 @@ int main()
                     ++fails;
                 }
             }
+    // the autotuner gets to time the splits that are fast with tiles other than the default ones, the ones
+    // of few passes and, of a real transform, those of its passes alone
+    const struct {
+        RealPart real;
+        unsigned long long n;
+        std::vector<int> split;
+    } timed[] = {{kComplex, 32768, {4096, 8}}, {kComplex, 12288, {4096, 3}}, {kComplex, 393216, {1536, 256}}, {kComplex, 480000, {1280, 375}},
+                 {kForward, 131072, {1024, 128}}, {kForward, 262144, {1024, 256}}, {kForward, 393216, {1536, 256}}, {kInverse, 393216, {1536, 256}}};
+    for (const auto& x : timed) {
+        const Splits v = tuned_splits(F32, x.n, 5, 1, 256, x.real);
+        if (std::find(v.begin(), v.end(), x.split) == v.end()) {
+            printf("FAIL real %d n %llu: %s is not timed\n", x.real.kind, x.n, text(x.split).c_str());
+            ++fails;
+        }
+    }
     // forward splits: half rows of 128 bytes and more through the L2 to 64 MiB, of 64 to 16, shorter ones never
     store(STORE_THROUGH, kForward, F32, 3 << 19, {256, 96, 64}, 2);
     store(STORE_THROUGH, kForward, F32, 1 << 22, {256, 256, 64}, 2);
