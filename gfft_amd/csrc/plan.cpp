@@ -179,6 +179,7 @@ int build_c2c_passes(gfftx_plan_s* p)
         split_choice(p->forced_lens, lens, tiles);
         if (lens.empty() && !choose_passes(p->prec, n, lens, p->batch, device_cus(p->device), p->real_part()))
             return fail(GFFTX_ERR_UNSUPPORTED, "no multi-pass decomposition for n=%llu", n);
+        if (!passes_fit(lens, n)) return fail(GFFTX_ERR_UNSUPPORTED, "passes that do not multiply to n=%llu", n);
         long long ns = 1;
         for (size_t i = 0; i < lens.size(); ++i) {
             const int L = lens[i];

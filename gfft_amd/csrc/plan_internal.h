@@ -112,6 +112,7 @@ const TileEntry* pass_tile(int prec, int L, unsigned long long ns, unsigned long
 std::vector<std::vector<int>> candidate_passes(int prec, unsigned long long n, size_t k, unsigned long long batch = 1,
                                                int cus = 256, bool mixed = true, RealPart real = RealPart(), bool any = false);
 void split_choice(const std::vector<int>& c, std::vector<int>& lens, std::vector<std::pair<int, int>>& tiles);
+bool passes_fit(const std::vector<int>& lens, unsigned long long n);
 int xcd_remap(const TileEntry* k, int prec);
 bool native_length(int prec, unsigned long long n);
 bool choose_passes(int prec, unsigned long long n, std::vector<int>& out, unsigned long long batch = 1, int cus = 256,

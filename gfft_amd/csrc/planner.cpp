@@ -262,6 +262,17 @@ void split_choice(const std::vector<int>& c, std::vector<int>& lens, std::vector
     }
 }
 
+// Whether the pass lengths of a choice, which may come from a cache file, multiply to n.
+bool passes_fit(const std::vector<int>& lens, unsigned long long n)
+{
+    unsigned long long prod = 1;
+    for (int L : lens) {
+        if (L < 2 || prod > n / (unsigned long long)L) return false;
+        prod *= (unsigned long long)L;
+    }
+    return lens.size() >= 2 && prod == n;
+}
+
 // XCD-aware tile order for a pass tile (GFFTX_XCD overrides): on when the tile's rows are not
 // whole 128-byte lines, so that the neighbouring tiles that share the lines at their ends run
 // on one XCD and meet in its L2.  Tiles with whole-line rows share no lines; they load their

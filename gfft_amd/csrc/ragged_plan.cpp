@@ -69,7 +69,7 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
             use_single = true;
             k1 = find_tile(r->prec, (int)L, false, false, t_tiles.empty() ? 0 : t_tiles[0].first,
                            t_tiles.empty() ? 0 : t_tiles[0].second);
-        } else if (!t_single && t_lens.size() >= 2) {
+        } else if (!t_single && passes_fit(t_lens, (unsigned long long)L)) {
             use_single = false;
             multi = true;
             lens = t_lens;

@@ -149,6 +149,12 @@ int main()
                 ++fails;
             }
         }
+    // choices of a cache file that are no split of n
+    if (!passes_fit({512, 256}, 1 << 17) || passes_fit({512, 256}, 1 << 18) || passes_fit({1 << 17, 1}, 1 << 17) || passes_fit({1 << 17}, 1 << 17) ||
+        passes_fit({}, 1) || passes_fit({65536, 65536, 65536, 65536, 65536}, 1 << 16)) {
+        printf("FAIL passes_fit\n");
+        ++fails;
+    }
     // a choice's name shows every pass with its own tile
     const struct {
         std::vector<int> c;

@@ -46,3 +46,33 @@ def test_describe_lists_the_fastest_candidates(torch_cuda, tmp_path, monkeypatch
     if n == 65537:
         m = [int(s.split(":")[0]) for s in splits]
         assert all(v >= 2 * n - 1 for v in m) and all(s.count("x") == 2 and s.count("/") == 3 for s in splits)
+
+
+def test_cache_entries_that_are_no_split(torch_cuda, tmp_path, monkeypatch):
+    """A cache file may hold anything: lengths that do not multiply to n are not run."""
+    cache = tmp_path / "tune.json"
+    monkeypatch.setenv("GFFTX_TUNE_CACHE", str(cache))
+    n, lens = 1 << 17, [20000, 49152]
+
+    def run():
+        x = inputs.complex_normal(n, 6)
+        with api.Plan(n, api.COMPLEX_DOUBLE, api.DFT, api.IN_PLACE) as p:
+            d = torch_cuda.from_numpy(x.copy()).cuda()
+            p.fft(d)
+            assert rel_l2(d.cpu().numpy(), np.fft.fft(x)) <= 1e-13
+        x = inputs.complex_normal(sum(lens), 7)
+        p = api.RaggedPlan(lens, api.COMPLEX_DOUBLE, api.DFT)
+        d = torch_cuda.from_numpy(x.copy()).cuda()
+        p.fft(d)
+        y = d.cpu().numpy()
+        p.close()
+        assert rel_l2(y[:lens[0]], np.fft.fft(x[:lens[0]])) <= 1e-13
+        assert rel_l2(y[lens[0]:], np.fft.fft(x[lens[0]:])) <= 1e-13
+
+    run()  # measured, for the keys
+    keys = list(json.loads(cache.read_text())["entries"])
+    assert len(keys) == 3
+    forged = tmp_path / "forged.json"
+    forged.write_text('{"version": 2, "entries": {\n' + ",\n".join(f'"{k}": [256, 128]' for k in keys) + "\n}}\n")
+    monkeypatch.setenv("GFFTX_TUNE_CACHE", str(forged))
+    run()
