@@ -390,6 +390,7 @@ bool tune_length_class(int device, int prec, long long L, long long count, bool 
 int fill_reps(int prec, unsigned long long n);
 std::vector<std::vector<int>> tuned_splits(int prec, unsigned long long n, size_t k, unsigned long long batch, int cus,
                                            RealPart real = RealPart());
+std::vector<int> with_tiles(int prec, unsigned long long n, unsigned long long batch, int cus, const std::vector<int>& c);
 std::string choice_label(const std::vector<int>& c, bool chirp);
 // cache entries of other choices (the ragged batch's persistent-kernel limit)
 std::string ragged_tune_key(int device, int prec, const uint64_t* lengths, uint64_t count);

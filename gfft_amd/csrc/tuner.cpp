@@ -443,6 +443,29 @@ static std::vector<int> best_combination(const std::vector<int>& chosen, const s
     return combo;
 }
 
+// A choice with the run-time tiles its lengths ran with: which one is the default depends on the number of
+// items, and the candidates of a batch above 1 GiB run on fewer than the plan has.
+std::vector<int> with_tiles(int prec, unsigned long long n, unsigned long long batch, int cus, const std::vector<int>& c)
+{
+    std::vector<int> l;
+    std::vector<std::pair<int, int>> t;
+    split_choice(c, l, t);
+    if (!passes_fit(l, n) || getenv("GFFTX_TNB") || getenv("GFFTX_TWG")) return c;
+    t.resize(l.size(), {0, 0});
+    unsigned long long ns = 1;
+    for (size_t i = 0; i < l.size(); ++i) {
+        const TileEntry* k = t[i].first ? nullptr : pass_tile(prec, l[i], ns, n, batch, cus);
+        if (k && k->mix) t[i] = {k->nb, k->wg};
+        ns *= (unsigned long long)l[i];
+    }
+    l.push_back(0);
+    for (const auto& x : t) {
+        l.push_back(x.first);
+        l.push_back(x.second);
+    }
+    return l;
+}
+
 // A choice as describe() names it: the pass lengths, each with /nb-wg where the choice names the tile,
 // or single/nb-wg; for a chirp-z plan the convolution length m first, then all of its passes (a split of
 // m into k lengths runs in 2k - 1).
@@ -579,8 +602,8 @@ int create_plan(gfftx_plan* out, uint64_t n, uint64_t batch, int vtype, int ttyp
         }
         note = tune_note(run.timed, chirp);
         run.again(6);
-        chosen = run.chosen;
-        if (chosen.empty()) return GFFTX_SUCCESS;
+        if (run.chosen.empty()) return GFFTX_SUCCESS;
+        chosen = chirp ? run.chosen : with_tiles(p->prec, n, tbatch, device_cus(device), run.chosen);
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tune[key] = chosen;
         tune_store();
@@ -648,7 +671,7 @@ bool tune_length_class(int device, int prec, long long L, long long count, bool 
             if (!combo.empty()) run.time(combo);
         }
         run.again(3);  // (a batch may have dozens of classes)
-        chosen = run.chosen;
+        chosen = with_tiles(prec, (unsigned long long)L, tcount, device_cus(device), run.chosen);
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tune[key] = chosen;
         tune_store();

@@ -149,6 +149,18 @@ int main()
                 ++fails;
             }
         }
+    // a choice keeps the run-time tiles it was timed with: the default one changes with the items
+    {
+        const std::vector<int> one = with_tiles(F32, 40000, 1, 256, {200, 200}), many = with_tiles(F32, 40000, 256, 256, {200, 200});
+        const TileEntry *a = pass_tile(F32, 200, 1, 40000, 1, 256), *b = pass_tile(F32, 200, 1, 40000, 256, 256);
+        if (one.size() != 7 || one[2] != 0 || one[3] != a->nb || one[4] != a->wg || many[3] != b->nb || many[4] != b->wg || a == b ||
+            with_tiles(F32, 1 << 18, 1, 256, {1024, 256}) != std::vector<int>({1024, 256, 0, 0, 0, 0, 0}) ||
+            with_tiles(F32, 1000, 1, 256, {1000, 1, 0, 2, 256}) != std::vector<int>({1000, 1, 0, 2, 256}) ||
+            with_tiles(F32, 1000000, 1, 256, {1000, 1000, 0, 8, 832, 4, 448}) != std::vector<int>({1000, 1000, 0, 8, 832, 4, 448})) {
+            printf("FAIL with_tiles\n");
+            ++fails;
+        }
+    }
     // choices of a cache file that are no split of n
     if (!passes_fit({512, 256}, 1 << 17) || passes_fit({512, 256}, 1 << 18) || passes_fit({1 << 17, 1}, 1 << 17) || passes_fit({1 << 17}, 1 << 17) ||
         passes_fit({}, 1) || passes_fit({65536, 65536, 65536, 65536, 65536}, 1 << 16)) {
