@@ -328,7 +328,7 @@ struct gfftx_ragged_s {
         long long count = 0;
         const long long* offs = nullptr;  // element offsets of the class's transforms
         std::vector<Pass> passes;         // one pass: single-pass tile over all of them
-        gfftx_plan_s* blue = nullptr;     // length with a prime factor above 5: chirp-z plan
+        gfftx_plan_s* blue = nullptr;     // length with a prime factor above 7: chirp-z plan
     };
     std::vector<LongClass> longs;
     void* lscratch[2][kRaggedSides] = {};  // per side stream, the size of the whole batch: same offsets

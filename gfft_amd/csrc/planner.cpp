@@ -76,7 +76,8 @@ int device_cus(int device)
 }
 
 // Bandwidth (TB/s) a multi-pass tile of length L reaches on MI355X with XCD remapping,
-// measured over N = 2^24 passes; lengths not listed are interpolated by size class.
+// measured over N = 2^24 passes; lengths not listed are interpolated by size class.  (The price of a
+// chirp-z pass, chirp_plan.cpp.)
 double pass_bandwidth(int prec, int L)
 {
     const bool f32 = prec == PREC_F32;

@@ -43,8 +43,8 @@ int ragged_long_class(gfftx_ragged_s* r, long long L, const std::vector<long lon
     HIP_TRY(hipMemcpy(d, offs.data(), offs.size() * sizeof(long long), hipMemcpyHostToDevice));
     lc.offs = (const long long*)d;
     if (!native_length(r->prec, (unsigned long long)L)) {
-        // chirp-z plan for the whole class; its element-wise kernels address the transforms
-        // through the offset table
+        // chirp-z plan for the whole class; its first and last pass address the transforms through the
+        // offset table
         gfftx_plan bp = nullptr;
         const int cvt = r->prec == PREC_F64 ? GFFTX_COMPLEX_DOUBLE : GFFTX_COMPLEX_FLOAT;
         e = create_plan(&bp, (uint64_t)L, (uint64_t)lc.count, cvt, r->inverse ? GFFTX_IDFT : GFFTX_DFT,

@@ -24,7 +24,7 @@
  *
  * Lengths: any n >= 2 (GFFT's out-of-place path takes any N, src/gfftalg.h:459-507).
  * Products of 2, 3, 5 and 7 run as Stockham passes (FP32 up to 2^28, FP64 up to 2^26); any
- * other n runs as a chirp-z convolution of a 2/3/5-smooth length m >= 2n-1 with the same
+ * other n runs as a chirp-z convolution of such a length m >= 2n-1 with the same
  * limits on m.  RDFT/IRDFT need an even n (GFFT's Separate assumes it,
  * src/gfftswap.h:255,279).
  *
@@ -78,8 +78,8 @@ typedef enum gfftx_status {
 #define GFFTX_FLAG_NO_AUTOTUNE 0x4u  /* use the built-in schedule, ignore the tuning cache */
 #define GFFTX_FLAG_GRAPH 0x8u        /* replay execution through a captured hipGraph      */
 #define GFFTX_FLAG_PROFILE 0x10u     /* time every kernel launch with a HIP event pair
-                                        (FFT tile and MFMA kernels: events attached to the
-                                        dispatch; element-wise kernels: recorded around it) */
+                                        (FFT tile, chirp-z and MFMA kernels: events attached to
+                                        the dispatch; a real split's own kernel: recorded around it) */
 
 typedef struct gfftx_plan_s* gfftx_plan;
 typedef struct gfftx_ragged_s* gfftx_ragged;
@@ -157,7 +157,7 @@ int gfftx_plan_profile(gfftx_plan plan, double* total_ms, uint64_t* count, const
  * (transform i starts at complex offset sum_{j<i} lengths[j]).  Any length n >= 2 within
  * the plan limits, FP32 or FP64.  In FP32, lengths 2^k, 3*2^k, 5*2^k from 16 to 4096 run
  * in one persistent launch; every other length class (all of them in FP64) runs as batched
- * launches on side streams that overlap it (a class with a prime factor above 5 as a
+ * launches on side streams that overlap it (a class with a prime factor above 7 as a
  * chirp-z plan over its transforms); one call (or one hipGraph with GFFTX_FLAG_GRAPH)
  * covers all.  With autotuning on, plan creation also times the batch with every length as
  * a class launch and keeps that form where it is faster (the choice is cached per set of
