@@ -287,12 +287,11 @@ int upload_mix_table(std::vector<void*>& owned, const TileEntry& k, void** out)
     long long ns = k.radices[0];
     for (int s = 1; s < k.nrad; ++s) {
         const long long R = k.radices[s];
+        const auto w = all_roots(ns * R);
         for (long long r = 1; r < (k.prec == PREC_F64 ? R : 2); ++r)
             for (long long kk = 0; kk < ns; ++kk) {
-                long double c, si;
-                root_ld(kk * r, ns * R, &c, &si);
-                t.push_back((double)c);
-                t.push_back((double)si);
+                t.push_back((double)w[kk * r].first);
+                t.push_back((double)w[kk * r].second);
             }
         ns *= R;
     }

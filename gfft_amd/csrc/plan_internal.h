@@ -43,6 +43,7 @@ int fail(int code, const char* fmt, ...);
 
 // --- planner.cpp: roots, tile lookup, cost model, pass splits, tables
 void root_ld(long long m, long long N, long double* c, long double* s);
+std::vector<std::pair<long double, long double>> all_roots(long long N);
 
 struct DevBuf {
     void* p = nullptr;

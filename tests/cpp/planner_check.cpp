@@ -7,7 +7,7 @@
 //   - passes store the way that was measured fastest for their kind, rows and size;
 //   - the autotuner's repeated in-place transforms stay in the range of their numbers;
 //   - describe() names a tuned choice in full;
-//   - the table of an unfused real split holds the roots, bit for bit;
+//   - twiddle tables and the table of an unfused real split hold the roots, bit for bit;
 //   - a length runs natively exactly where a tile or a split exists.
 #include <cstdio>
 
@@ -184,6 +184,21 @@ int main()
             printf("FAIL label %s, not %s\n", choice_label(x.c, x.chirp).c_str(), x.want);
             ++fails;
         }
+    // the roots of a table, folded out of the first octant or not, are the evaluated ones
+    for (long long N : {1ll, 2ll, 6ll, 8ll, 15ll, 16ll, 24ll, 40ll, 100ll, 256ll, 1000ll, 1536ll, 4096ll, 10000ll, 16384ll}) {
+        const auto w = all_roots(N);
+        bool ok = w.size() == (size_t)N;
+        for (long long m = 0; ok && m < N; ++m) {
+            long double c, s, c2, s2;
+            root_ld(m, N, &c, &s);
+            root_ld(m * 64, N * 64, &c2, &s2);  // (and a power of two scales out)
+            ok = w[m].first == c && w[m].second == s && c2 == c && s2 == s;
+        }
+        if (!ok) {
+            printf("FAIL roots of order %lld\n", N);
+            ++fails;
+        }
+    }
     // the split table's mirrored and shared-out entries are the roots themselves
     for (long long n : {2ll, 4ll, 6ll, 10ll, 12ll, 98ll, 1000ll, 4096ll, 200000ll, 524290ll}) {
         const std::vector<float> f = split_roots<float>(n);
