@@ -118,16 +118,19 @@ struct TileCfg {
     static constexpr int ROOTS = TW_POW ? most_roots() : 1;
     static constexpr int TW_ROOT_OFF = (twoff(NS) * (int)sizeof(V2<T_>) + 15) / 16 * 16;  // bytes
     // LDS layout (bank spread): one pad element every 16, or every 8 where an FP32 pass tile begins
-    // with radix 8, and a distance TS between sequences.  In T mode NB lanes in a row take one
-    // element of NB sequences, the next ones the element after it: TS = 32 / NB modulo 32 FP32 (8 /
-    // NB modulo 8 FP64) spreads the 32 lanes of an 8-byte access (8 of a 16-byte one) over all
-    // banks, both where consecutive elements are read and where the first stage writes them R_0 +
-    // 1 apart.  Otherwise an odd distance.
+    // with radix 8, and a distance TS between sequences.  The LDS moves 128 bytes a cycle: 16 lanes of
+    // an 8-byte access, 8 of a 16-byte one.  In T mode NB lanes in a row take one element of NB
+    // sequences, the next ones the element after it: TS = 16 / NB modulo 16 FP32 (8 / NB modulo 8
+    // FP64) spreads a cycle's lanes over all banks, both where consecutive elements are read and
+    // where the first stage writes them R_0 + 1 apart.  Otherwise an odd distance.  LDS cycles an
+    // instruction (counted; 16 / NB, then 32 / NB modulo 32, then odd): 1536 points, NB 4, 4.6, 6.0,
+    // 12.0 (2^21 points 17.9, 18.2, 20.1 us); 4096, NB 4, 4.4, 5.8, 12.4 (22.3, 22.7, 24.9); 1024, NB 8,
+    // 4.6, 5.7, 9.1 (10.1, 10.1, 10.6); 256, NB 16, 5.3, 6.7, 5.3.
     static constexpr int PADSH = LOADT_ && sizeof(T_) == 4 && R[0] == 8 ? 3 : 4;
     static constexpr int LP = L + (L >> PADSH);
     static constexpr int lds_distance()
     {
-        constexpr int banks = sizeof(T_) == 4 ? 32 : 8;
+        constexpr int banks = sizeof(T_) == 4 ? 16 : 8;
         if (!LOADT_ || NB_ < 2 || NB_ >= banks || banks % NB_ != 0) return LP % 2 == 0 ? LP + 1 : LP;
         int ts = LP;
         while (ts % banks != banks / NB_) ++ts;

@@ -6,10 +6,12 @@
 //   - the splits a tuned plan times include those;
 //   - passes store the way that was measured fastest for their kind, rows and size;
 //   - the autotuner's repeated in-place transforms stay in the range of their numbers;
+//   - the lanes of one LDS cycle meet distinct banks in the pass tiles;
 //   - describe() names a tuned choice in full;
 //   - twiddle tables and the table of an unfused real split hold the roots, bit for bit;
 //   - a length runs natively exactly where a tile or a split exists.
 #include <cstdio>
+#include <functional>
 
 #include "../../gfft_amd/csrc/plan_internal.h"
 
@@ -47,6 +49,31 @@ static void store(int want, RealPart real, int prec, unsigned long long n, const
     const int got = !ps.k ? -1 : pass_store(true, nt, i, lens.size(), (size_t)n * elem_bytes(prec), ps, (size_t)n, 1);
     if (got != want || (ps.k && pass_store(false, false, i, lens.size(), (size_t)n * elem_bytes(prec), ps, (size_t)n, 1) != STORE_PLAIN)) {
         printf("FAIL real %d prec %d n %llu %s pass %zu: store %d, not %d\n", real.kind, prec, n, text(lens).c_str(), i, got, want);
+        ++fails;
+    }
+}
+
+// LDS cycles of a T-mode pass tile: `lanes` lanes in a row (one cycle's: 128 bytes), NB of them on one element of
+// NB sequences, the next ones on the element `step` further; their places modulo the banks differ.
+static bool spread(int prec, int nb, unsigned ts, const std::function<unsigned(unsigned)>& place, unsigned step)
+{
+    const unsigned lanes = prec == PREC_F64 ? 8 : 16;
+    for (unsigned j0 = 0; j0 < 4; ++j0) {
+        std::vector<char> hit(lanes, 0);
+        for (unsigned l = 0; l < lanes; ++l) {
+            const unsigned lane = j0 * lanes + l, p = lane % nb * ts + place(lane / nb * step);
+            if (hit[p % lanes]++) return false;
+        }
+    }
+    return true;
+}
+
+template <class C> static void spread_tile()
+{
+    auto place = [](unsigned e) { return e + (e >> C::PADSH); };
+    if (!spread(sizeof(typename C::T) == 8 ? PREC_F64 : PREC_F32, C::NB, C::TS, place, 1) ||
+        !spread(sizeof(typename C::T) == 8 ? PREC_F64 : PREC_F32, C::NB, C::TS, place, C::R[0])) {
+        printf("FAIL banks of L %d nb %d ts %d\n", C::L, C::NB, C::TS);
         ++fails;
     }
 }
@@ -167,6 +194,27 @@ int main()
         printf("FAIL passes_fit\n");
         ++fails;
     }
+    // a cycle's lanes of a pass tile meet distinct banks
+    spread_tile<TileCfg<float, 256, 16, 256, true, true, 16, 16>>();
+    spread_tile<TileCfg<float, 256, 8, 128, true, true, 16, 16>>();
+    spread_tile<TileCfg<float, 192, 16, 192, true, true, 16, 4, 3>>();
+    spread_tile<TileCfg<float, 128, 32, 256, true, true, 16, 8>>();
+    spread_tile<TileCfg<float, 1024, 8, 512, true, true, 16, 16, 4>>();
+    spread_tile<TileCfg<float, 1024, 8, 1024, true, true, 8, 8, 8, 2>>();
+    spread_tile<TileCfg<float, 1024, 4, 256, true, false, 16, 16, 4>>();
+    spread_tile<TileCfg<float, 1536, 4, 768, true, false, 8, 8, 8, 3>>();
+    spread_tile<TileCfg<float, 4096, 2, 512, true, false, 16, 16, 16>>();
+    spread_tile<TileCfg<float, 4096, 4, 1024, true, false, 16, 16, 16>>();
+    spread_tile<TileCfg<double, 1024, 4, 256, true, true, 16, 16, 4>>();
+    spread_tile<TileCfg<double, 256, 16, 256, true, true, 16, 16>>();
+    spread_tile<TileCfg<double, 4096, 2, 512, true, false, 16, 16, 16>>();
+    for (int L : {96, 250, 384, 500, 512, 1000, 1250})
+        for (const TileEntry* k : mix_tiles(F64, L, true, true))
+            if ((size_t)k->nb * k->mix->ts * elem_bytes(F64) <= 150 * 1024 &&
+                !spread(F64, k->nb, k->mix->ts, [](unsigned e) { return e; }, 1)) {
+                printf("FAIL banks of %s ts %u\n", k->name, k->mix->ts);
+                ++fails;
+            }
     // a choice's name shows every pass with its own tile
     const struct {
         std::vector<int> c;
